@@ -285,7 +285,7 @@ def timer_read(name):
 
 def set_flag(name, value):
     """Selects an implementation variant (am_set_flag), e.g.
-    set_flag("table_prepartition", 0)."""
+    set_flag("table_atomic", 0)."""
     check(load().am_set_flag(name.encode(), int(value)), "am_set_flag")
 
 

@@ -879,44 +879,17 @@ __device__ __forceinline__ void geo_eval_bwd_an(const GeoArgs& a, const float* s
 }
 
 // ---- pair emission with merging ----
-// A tile's pairs go to [keys, keys + limit): limit is the count the count
-// pass found for the tile; the emit pass makes the same decisions, and never
-// writes past limit.
+// The pairs of a tile at one level go to [keys, keys + limit): limit is the
+// count the count pass found for them; the emit pass makes the same
+// decisions, and never writes past limit.  Each lane group (16 lanes, one
+// level) has its own.
 template <class VT>
 struct EmitTile {
-    uint32_t* keys;   // tile's first pair (keys); partitioned: the arrays' start
-    VT* vals;         // tile's first pair (values); partitioned: the arrays' start
-    int cursor;       // wave-uniform write position
-    int limit;        // pairs reserved for the tile
-    // Partitioned form (part != nullptr): the pairs of the tile with radix
-    // digit d = (row >> 9) & 255 go to base[d] + [0, lim[d]); part[d] counts
-    // them as they are written (in the count pass: the counts themselves).
-    // Wave-private LDS arrays of kPartDigits entries.
-    int32_t* part;
-    const int32_t* lim;
-    const int64_t* base;
+    uint32_t* keys;   // the tile's first pair at the level (keys)
+    VT* vals;         // the same (values); atomic form: the table gradient
+    int cursor;       // group-uniform write position
+    int limit;        // pairs reserved
 };
-
-// Partitioned pair emission (flag "table_prepartition", off by default): the
-// first 8-bit digit of the table-gradient radix sort (key bits [9, 17)) is
-// applied as pairs are written, and the sort makes one pass over [17, 25)
-// instead of two.  Measured on the Neuralangelo step it loses: the sort
-// drops from 4.6 to 2.4 ms, but the emission's stores scatter over 256
-// partitions and write partial lines (emit 3.0 -> 7.7 ms, count 0.4 ->
-// 0.9 ms); 32 partitions with one 11-bit pass measured no better (emit 5.5,
-// sort 4.7 ms).
-constexpr int kPartShift = 9;
-constexpr int kPartBits = 8;
-constexpr int kPartDigits = 1 << kPartBits;
-
-__device__ __forceinline__ uint32_t pair_digit(uint32_t row) {
-    return (row >> kPartShift) & (uint32_t)(kPartDigits - 1);
-}
-
-__device__ __forceinline__ uint64_t lanemask_lt() {
-    const int l = lane_id();
-    return l == 0 ? 0ull : (~0ull >> (64 - l));
-}
 
 // Atomic form (flag "table_atomic"): the "pair array" is the table gradient
 // itself, [n_entries] rows of 2 floats, and each pair is added into its row
@@ -944,10 +917,9 @@ __device__ __forceinline__ void set_pair(AtomicRow& v, float a, float b) {   // 
     v.v[1] = b;
 }
 
-// The group's K * n pairs (n lanes on) fill [cursor, cursor + K n) corner-
-// major: pair c of the lane of rank r goes to cursor + c n + r, so each store
-// instruction writes consecutive addresses across the lanes.  The order is a
-// fixed function of the data (the reduction's summation order follows it).
+// The lane group's K * n pairs (n lanes on) fill [cursor, cursor + K n)
+// corner-major: pair c of the lane of rank r goes to cursor + c n + r, so each
+// store instruction writes consecutive addresses across the group's lanes.
 template <int K, bool COUNT, class VT>
 __device__ __forceinline__ void emit_pairs(EmitTile<VT>& et, bool on, const uint32_t rows[K],
                                            const float vals[2 * K]) {
@@ -963,45 +935,13 @@ __device__ __forceinline__ void emit_pairs(EmitTile<VT>& et, bool on, const uint
         }
         return;
     }
+    const int l = lane_id(), k = l >> 4;
     const uint64_t mask = __ballot(on);
-    const int n_on = __popcll(mask);
-    if (et.part) {   // partitioned form (rows are computed in both passes)
-        if (mask == 0) return;
-        const uint64_t lt = lanemask_lt();
-#pragma unroll
-        for (int c = 0; c < K; ++c) {
-            const uint32_t d = on ? pair_digit(rows[c]) : 0u;
-            if constexpr (COUNT) {
-                if (on) atomicAdd(&et.part[d], 1);   // counts: order-free
-            } else {
-                // lanes with the same digit (one ballot a bit), ranked by lane: the
-                // order inside a partition is corner-major, then lane, as in
-                // the compact form, so every sum keeps its order
-                uint64_t peers = mask;
-#pragma unroll
-                for (int b = 0; b < kPartBits; ++b) {
-                    const uint64_t ones = __ballot(on && ((d >> b) & 1u));
-                    peers &= ((d >> b) & 1u) ? ones : ~ones;
-                }
-                const int before = __popcll(peers & lt);
-                // one wave's LDS operations complete in issue order: every
-                // lane reads part[d] before its group's first lane updates it
-                const int have = on ? et.part[d] : 0;
-                if (on && before == 0) et.part[d] = have + __popcll(peers);
-                if (on && have + before < et.lim[d]) {
-                    const int64_t at = et.base[d] + have + before;
-                    et.keys[at] = rows[c];
-                    VT v;
-                    set_pair(v, vals[2 * c], vals[2 * c + 1]);
-                    et.vals[at] = v;
-                }
-            }
-        }
-        et.cursor += K * n_on;
-        return;
-    }
+    const uint32_t half = (k & 2) ? (uint32_t)(mask >> 32) : (uint32_t)mask;
+    const uint32_t group = ((k & 1) ? half >> 16 : half) & 0xffffu;
+    const int n_on = __popc(group);
     if (!COUNT && on && et.cursor + K * n_on <= et.limit) {
-        const int off = et.cursor + __popcll(mask & lanemask_lt());
+        const int off = et.cursor + __popc(group & ((1u << (l & 15)) - 1u));
 #pragma unroll
         for (int c = 0; c < K; ++c) {
             et.keys[off + c * n_on] = rows[c];
@@ -1080,8 +1020,8 @@ __device__ __forceinline__ void merge_step(int p, float acc[16], bool& end) {
     }
 }
 
-// Reduces the stored encode gradients of one cluster of evaluations into
-// (row, value) pairs with a star-stencil merge.  Per level, B = the cell of
+// Reduces the stored encode gradients of one cluster of evaluations at level
+// slot j into (row, value) pairs with a star-stencil merge.  B = the cell of
 // the cluster centre; an evaluation whose cell C
 //   * is B adds its 8 corner values into B's accumulators,
 //   * is B +- e_axis (a face neighbour, the usual case of an offset of about
@@ -1093,18 +1033,13 @@ __device__ __forceinline__ void merge_step(int p, float acc[16], bool& end) {
 // tree, and the segment head emits them.  Every sum has a fixed order.
 // genc_base: LDS [eval][LJ][2][64] of this wave; the cluster's q-th
 // evaluation is genc slot slot0 + q.  COUNT: positions only (no gradients);
-// the cursor ends at the tile's pair count.
+// the cursor advances by the lane group's pairs.
 template <int LJ, int CL, bool COUNT, class VT>
-__device__ __forceinline__ void flush_cluster(const GeoArgs& a, const LevelParams* lv,
-                                              const GeoSample& s, bool valid, const float* genc_base,
+__device__ __forceinline__ void flush_cluster(const GeoArgs& a, const LevelParams& lp, bool on,
+                                              const GeoSample& s, const float* genc_base, int j,
                                               int n_q, int slot0, EmitTile<VT>& et) {
-    const int l = lane_id(), p = l & 15, k = l >> 4;
-#pragma unroll 1
-    for (int j = 0; j < LJ; ++j) {
-        const int level = k + 4 * j;
-        const bool on = valid && level < a.active;
-        LevelParams lp{};
-        if (level < a.g.L) lp = lv[level];
+    const int l = lane_id(), p = l & 15;
+    {
         uint32_t B[3];
         {
             float xc[3];
@@ -1162,7 +1097,7 @@ __device__ __forceinline__ void flush_cluster(const GeoArgs& a, const LevelParam
                 const bool em = on && !same && !adj;
                 uint32_t rows[8];
                 float v[16];
-                if ((!COUNT || et.part) && em) corner_rows(lp, pp.c, rows);
+                if (!COUNT && em) corner_rows(lp, pp.c, rows);
                 if (!COUNT && em) {
 #pragma unroll
                     for (int c = 0; c < 8; ++c) {
@@ -1178,7 +1113,7 @@ __device__ __forceinline__ void flush_cluster(const GeoArgs& a, const LevelParam
                 const bool em = on && adj;
                 uint32_t rows[4];
                 float v[8];
-                if ((!COUNT || et.part) && em) {
+                if (!COUNT && em) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int c = face_corner(i, axm, far_bit);
@@ -1250,7 +1185,7 @@ __device__ __forceinline__ void flush_cluster(const GeoArgs& a, const LevelParam
         const uint32_t u0 = row_up1(key0), u1 = row_up1(key1), u2 = row_up1(key2);
         const bool head = live && (p == 0 || !(u0 == key0 && u1 == key1 && u2 == key2));
         uint32_t rows[8];
-        if ((!COUNT || et.part) && head) corner_rows(lp, B, rows);
+        if (!COUNT && head) corner_rows(lp, B, rows);
         emit_pairs<8, COUNT, VT>(et, head, rows, acc);
     }
 }
@@ -1302,29 +1237,22 @@ __host__ __device__ inline int64_t geo_genc_floats(int64_t tiles, int n_evals, i
 }
 
 // Pair pass.  COUNT: the number of (row, value) pairs each tile of 16
-// samples emits, from positions alone.  Otherwise: the same decisions with
-// the encode gradients, each tile's pairs written from offsets[tile] (never
-// past counts[tile]; a different count sets status[1]).
-// PART: the pairs are partitioned by their digit d = (row >> 9) & 255 as
-// they are written: counts and offsets then hold kPartDigits entries per
-// tile, digit-major ([d * n_tiles + tile]), and a tile's pairs of digit d go
-// to [offsets[d n_tiles + tile], + counts[...]) in emission order.
-template <int LJ, bool COUNT, class VT, bool PART>
+// samples emits at each level, from positions alone (counts[level * tiles +
+// tile]).  Otherwise: the same decisions with the encode gradients, the pairs
+// written from offsets[level * tiles + tile] on (one stream per level, never
+// past the tile's count; a different count sets status[1]).
+template <int LJ, bool COUNT, class VT>
 __global__ void __launch_bounds__(256) k_geo_pairs(
     GeoArgs a, const float* __restrict__ pts, const float* __restrict__ randn, int64_t N,
     const float* __restrict__ fdv, const float* __restrict__ genc, uint32_t* __restrict__ keys,
     VT* __restrict__ vals, const int64_t* __restrict__ offsets, int64_t* __restrict__ counts,
     int64_t* __restrict__ status, int64_t capacity) {
     __shared__ LevelParams lv[AM_MAX_LEVELS];
-    // per wave: running count, limit and first position of each digit
-    __shared__ int32_t part_s[PART ? 4 : 1][PART ? kPartDigits : 1];
-    __shared__ int32_t lim_s[PART && !COUNT ? 4 : 1][PART && !COUNT ? kPartDigits : 1];
-    __shared__ int64_t base_s[PART && !COUNT ? 4 : 1][PART && !COUNT ? kPartDigits : 1];
 #pragma unroll
     for (int q = 0; q < AM_MAX_LEVELS; ++q)
         if ((int)threadIdx.x == q && q < a.g.L) lv[q] = a.g.lv[q];
     __syncthreads();
-    const int l = lane_id(), p = l & 15;
+    const int l = lane_id(), p = l & 15, k = l >> 4;
     const int nw = blockDim.x >> 6, wave = threadIdx.x >> 6;
     const int64_t n_tiles = (N + 15) / 16;
     for (int64_t tile = (int64_t)blockIdx.x * nw + wave; tile < n_tiles;
@@ -1333,63 +1261,39 @@ __global__ void __launch_bounds__(256) k_geo_pairs(
         const bool valid = n < N;
         GeoSample s;
         geo_rebuild(a, pts, randn, fdv, n, caller_row(a, n, valid), valid, s);
-        EmitTile<VT> et{nullptr, nullptr, 0, 0, nullptr, nullptr, nullptr};
-        const float* gt = nullptr;
-        if constexpr (PART) {
-            int32_t* part = part_s[wave];
-            for (int d = l; d < kPartDigits; d += 64) {
-                part[d] = 0;
-                if constexpr (!COUNT) {
-                    // a run past the arrays' capacity is cut there (and the
-                    // consistency flag set): never a write out of range
-                    const int64_t at = (int64_t)d * n_tiles + tile;
-                    const int64_t b0 = offsets[at];
-                    const int64_t room = capacity - b0;
-                    const int64_t want = counts[at];
-                    base_s[wave][d] = b0;
-                    lim_s[wave][d] = (int32_t)(want <= room ? want : (room > 0 ? room : 0));
-                    if (want > room) status[1] = 1;
+        const float* gt = COUNT ? nullptr : genc + tile * a.genc_slots * LJ * 128;
+#pragma unroll 1
+        for (int j = 0; j < LJ; ++j) {
+            const int level = k + 4 * j;
+            const bool there = level < a.g.L;
+            const bool on = valid && level < a.active;
+            const int64_t entry = level * n_tiles + tile;
+            LevelParams lp{};
+            if (there) lp = lv[level];
+            EmitTile<VT> et{nullptr, nullptr, 0, 0};
+            if constexpr (kAtomicPairs<VT>) {
+                et.vals = vals;
+            } else if constexpr (!COUNT) {
+                if (there) {
+                    const int64_t off = offsets[entry];
+                    const int64_t room = capacity - off;
+                    int64_t lim = counts[entry];
+                    if (lim > room) {   // cut at the arrays' capacity, flagged
+                        lim = room > 0 ? room : 0;
+                        if (p == 0) status[1] = 1;
+                    }
+                    et = EmitTile<VT>{keys + off, vals + off, 0, (int)lim};
                 }
             }
-            mlp::wave_sync();
+            if (a.with_laplace)
+                flush_cluster<LJ, 1, COUNT>(a, lp, on, s, gt, j, 6, a.curv0, et);
+            flush_cluster<LJ, 0, COUNT>(a, lp, on, s, gt, j, a.with_grad && !a.analytic ? 7 : 1, 0,
+                                        et);
             if constexpr (COUNT) {
-                et.part = part;
-            } else {
-                et = EmitTile<VT>{keys, vals, 0, 0, part, lim_s[wave], base_s[wave]};
-                gt = genc + tile * a.genc_slots * LJ * 128;
+                if (there && p == 0) counts[entry] = et.cursor;
+            } else if constexpr (!kAtomicPairs<VT>) {
+                if (there && p == 0 && et.cursor != et.limit) status[1] = 1;
             }
-        } else if constexpr (kAtomicPairs<VT>) {
-            et = EmitTile<VT>{nullptr, vals, 0, 0, nullptr, nullptr, nullptr};
-            gt = genc + tile * a.genc_slots * LJ * 128;
-        } else if constexpr (!COUNT) {
-            const int64_t off = offsets[tile];
-            const int64_t room = capacity - off;
-            int64_t lim = counts[tile];
-            if (lim > room) {   // cut at the arrays' capacity, flagged
-                lim = room > 0 ? room : 0;
-                if (l == 0) status[1] = 1;
-            }
-            et = EmitTile<VT>{keys + off, vals + off, 0, (int)lim, nullptr, nullptr, nullptr};
-            gt = genc + tile * a.genc_slots * LJ * 128;
-        }
-        if (a.with_laplace) flush_cluster<LJ, 1, COUNT>(a, lv, s, valid, gt, 6, a.curv0, et);
-        flush_cluster<LJ, 0, COUNT>(a, lv, s, valid, gt, a.with_grad && !a.analytic ? 7 : 1, 0,
-                                    et);
-        if constexpr (PART) {
-            mlp::wave_sync();
-            bool bad = false;
-            for (int d = l; d < kPartDigits; d += 64) {
-                const int32_t got = et.part[d];
-                if constexpr (COUNT) counts[(int64_t)d * n_tiles + tile] = got;
-                else bad = bad || got != et.lim[d];
-            }
-            if constexpr (!COUNT)
-                if (__ballot(bad) != 0 && l == 0) status[1] = 1;
-            mlp::wave_sync();
-        } else if constexpr (COUNT) {
-            if (l == 0) counts[tile] = et.cursor;
-        } else if constexpr (!kAtomicPairs<VT>) {
-            if (l == 0 && et.cursor != et.limit) status[1] = 1;
         }
     }
 }
@@ -1642,7 +1546,7 @@ k_geo_bwd_o2(AM_GEO_BWD_PARAMS) {
 }
 
 // Sentinel keys and zero values in [status[0], bound): the unused tail of
-// pair arrays carved for the worst-case bound.
+// pair arrays carved for the worst-case bound (sorted form).
 template <class VT>
 __global__ void k_pair_tail(uint32_t* __restrict__ keys, VT* __restrict__ vals,
                             const int64_t* __restrict__ status, int64_t bound, uint32_t sentinel) {
@@ -1657,13 +1561,18 @@ __global__ void k_pair_tail(uint32_t* __restrict__ keys, VT* __restrict__ vals,
     }
 }
 
-// status[0] = number of pairs (offset + count of the last entry: the last
-// tile, or the last digit of the last tile); status[1] = 0, set by the
-// backward on a count mismatch.
-__global__ void k_pair_total(const int64_t* __restrict__ offsets, const int64_t* __restrict__ counts,
-                             int64_t tiles, int64_t* __restrict__ status) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        status[0] = offsets[tiles - 1] + counts[tiles - 1];
+// status[0] = number of pairs; status[1] = 0, set by the emit pass on a
+// count mismatch; level_start = the level streams' bounds.
+__global__ void k_pair_streams(const int64_t* __restrict__ offsets,
+                               const int64_t* __restrict__ counts, int64_t tiles, int L,
+                               int64_t* __restrict__ status, int64_t* __restrict__ level_start) {
+    const int l = threadIdx.x;
+    if (l < L) level_start[l] = offsets[l * tiles];
+    if (l == L) {
+        const int64_t last = L * tiles - 1;
+        const int64_t n = offsets[last] + counts[last];
+        level_start[L] = n;
+        status[0] = n;
         status[1] = 0;
     }
 }
@@ -1782,26 +1691,13 @@ static int geo_fwd_launch(const GeoArgs& a, const float* pts, const float* randn
 
 template <int LJ>
 static int geo_count_launch(const GeoArgs& a, const float* pts, const float* randn, int64_t n,
-                            const float* fdv, int64_t* counts, bool part, hipStream_t s) {
+                            const float* fdv, int64_t* counts, hipStream_t s) {
     KernelTimer kt_("pair_count", s);
-    if (part)
-        hipLaunchKernelGGL((k_geo_pairs<LJ, true, Vals<2>, true>), dim3(count_blocks(n)), dim3(256),
-                           0, s, a, pts, randn, n, fdv, nullptr, nullptr, nullptr, nullptr, counts,
-                           nullptr, (int64_t)0);
-    else
-        hipLaunchKernelGGL((k_geo_pairs<LJ, true, Vals<2>, false>), dim3(count_blocks(n)),
-                           dim3(256), 0, s, a, pts, randn, n, fdv, nullptr, nullptr, nullptr,
-                           nullptr, counts, nullptr, (int64_t)0);
+    hipLaunchKernelGGL((k_geo_pairs<LJ, true, Vals<2>>), dim3(count_blocks(n)), dim3(256), 0, s, a,
+                       pts, randn, n, fdv, nullptr, nullptr, nullptr, nullptr, counts, nullptr,
+                       (int64_t)0);
     AM_LAUNCH_CHECK();
     return AM_OK;
-}
-
-// Partitioned pair emission applies when the table reduce sorts key bits
-// [9, end) (9 < end <= 25) and the "table_prepartition" flag is on (off by
-// default: it measured slower, see kPartDigits).
-static bool geo_prepartition(const am_grid_desc* g) {
-    return table_bucket_bits(table_key_bits(g->n_entries)) == kPartShift &&
-           flag_value("table_prepartition", 0) != 0;
 }
 
 // The backward's workspace before the pair arrays: the pair count is only
@@ -1815,17 +1711,18 @@ struct GeoBwdWs {
     float* ctmp;
     int64_t* counts;
     int64_t* offsets;
-    int64_t entries;   // count / offset entries (tiles, or tiles x digits)
+    int64_t entries;   // count / offset entries: levels x tiles
     int64_t* status;
+    int64_t* level_start;
     void* scan_tmp;
     size_t scan_bytes;
 };
 
 static void carve_geo_bwd_head(WsCarver& c, const GeoArgs& a, int LJ, int64_t n, bool need_fdv,
-                               bool part, GeoBwdWs* w) {
+                               GeoBwdWs* w) {
     const int waves = bwd_blocks(n) * 4;
     const int64_t tiles = (n + 15) / 16;
-    const int64_t entries = tiles * (part ? kPartDigits : 1);   // count / offset entries
+    const int64_t entries = tiles * a.g.L;
     w->fdv = need_fdv ? c.take<float>((size_t)n * 12 + 1) : nullptr;
     w->sdf_tmp = need_fdv ? c.take<float>((size_t)n + 1) : nullptr;
     w->genc = c.take<float>((size_t)geo_genc_floats(tiles, a.genc_slots, LJ) + 1);
@@ -1835,6 +1732,7 @@ static void carve_geo_bwd_head(WsCarver& c, const GeoArgs& a, int LJ, int64_t n,
     w->offsets = c.take<int64_t>((size_t)entries + 1);
     w->entries = entries;
     w->status = c.take<int64_t>(2);
+    w->level_start = c.take<int64_t>(AM_MAX_LEVELS + 1);
     size_t sb = 0;
     rocprim::exclusive_scan(nullptr, sb, (const int64_t*)nullptr, (int64_t*)nullptr, (int64_t)0,
                             (size_t)(entries > 0 ? entries : 1), rocprim::plus<int64_t>(), 0,
@@ -1932,8 +1830,7 @@ static int geo_bwd_launch_t(const GeoArgs& a, const am_grid_desc* g, const float
     AM_CHECK_ARG(!store || !need_fdv, "a stored encoding needs the stored FD values too");
     WsCarver c(ws, ws_bytes);
     GeoBwdWs w;
-    const bool part = geo_prepartition(g);
-    carve_geo_bwd_head(c, a, LJ, n, need_fdv, part, &w);
+    carve_geo_bwd_head(c, a, LJ, n, need_fdv, &w);
     if (!c.ok()) return workspace_short(c.used, ws_bytes);
     const float* fdv = fdv_in;
     if (need_fdv) {  // recompute the stored SDF values with a forward pass
@@ -1974,7 +1871,7 @@ static int geo_bwd_launch_t(const GeoArgs& a, const am_grid_desc* g, const float
         if (int rc = launch_bwd()) return rc;
         {
             KernelTimer kt_("pair_atomic", s);
-            hipLaunchKernelGGL((k_geo_pairs<LJ, false, AtomicRow, false>), dim3(pair_blocks(n)),
+            hipLaunchKernelGGL((k_geo_pairs<LJ, false, AtomicRow>), dim3(pair_blocks(n)),
                                dim3(256), 0, s, a, pts, randn, n, fdv, w.genc, nullptr,
                                reinterpret_cast<AtomicRow*>(dtable), nullptr, nullptr, nullptr,
                                (int64_t)0);
@@ -1982,8 +1879,8 @@ static int geo_bwd_launch_t(const GeoArgs& a, const am_grid_desc* g, const float
         AM_LAUNCH_CHECK();
         return colsum_f32(w.partial, waves, a.n_params, dparams, w.ctmp, s);
     }
-    // 1. pairs per tile, 2. exclusive prefix sum -> each tile's first pair
-    if (int rc = geo_count_launch<LJ>(a, pts, randn, n, fdv, w.counts, part, s)) return rc;
+    // 1. pairs per level and tile, 2. exclusive prefix sum -> each one's first pair
+    if (int rc = geo_count_launch<LJ>(a, pts, randn, n, fdv, w.counts, s)) return rc;
     size_t sb = w.scan_bytes;
     hipError_t e = rocprim::exclusive_scan(w.scan_tmp, sb, w.counts, w.offsets, (int64_t)0,
                                            (size_t)w.entries, rocprim::plus<int64_t>(), s, false);
@@ -1991,15 +1888,14 @@ static int geo_bwd_launch_t(const GeoArgs& a, const am_grid_desc* g, const float
         set_error("tile-count scan failed: %s", hipGetErrorString(e));
         return AM_ERR_HIP;
     }
-    hipLaunchKernelGGL(k_pair_total, dim3(1), dim3(64), 0, s, w.offsets, w.counts, w.entries,
-                       w.status);
+    hipLaunchKernelGGL(k_pair_streams, dim3(1), dim3(64), 0, s, w.offsets, w.counts, tiles, a.g.L,
+                       w.status, w.level_start);
     AM_LAUNCH_CHECK();
     // 3. the pair arrays.  Sync-free form (flag "sdf_bwd_sync_free"): arrays
-    // of the worst-case pair bound, no host read; the tail past the
-    // device-side count is filled with sentinel keys (they sort last and are
-    // skipped) and the sort covers the bound.  Otherwise one host read of the
-    // pair count carves the arrays for exactly that many pairs.  A workspace
-    // too small is rejected here, before any output is written, with
+    // of the worst-case pair bound, no host read (the reduction reads the
+    // streams' bounds on the device).  Otherwise one host read of the pair
+    // count carves the arrays for exactly that many pairs.  A workspace too
+    // small is rejected here, before any output is written, with
     // am_last_workspace_need() = what this call needs.
     const int64_t max_pairs = geo_max_pairs(a, LJ, n);
     const bool bounded = flag_value("sdf_bwd_sync_free", 0) != 0;
@@ -2011,12 +1907,11 @@ static int geo_bwd_launch_t(const GeoArgs& a, const am_grid_desc* g, const float
     }
     if (int rc = collect_flags(false)) return rc;
     TableReduceWs tw;
-    if (int rc = table_reduce_carve(c, 2, bounded ? max_pairs : st[0], g->n_entries, &tw,
-                                    PR == mlp::kBF16, part))
-        return rc;
+    const int64_t capacity = bounded ? max_pairs : st[0];
+    if (int rc = table_reduce_carve(c, g, capacity, &tw, PR == mlp::kBF16)) return rc;
     if (!c.ok()) return workspace_short(c.used, ws_bytes);
-    tw.m = bounded ? max_pairs : st[0];   // the arrays' capacity (and the sort's size)
-    if (bounded && max_pairs > 0) {
+    if (tw.paged) tw.level_start = w.level_start;
+    if (bounded && !tw.paged && max_pairs > 0) {   // the sorted form's unused tail
         const int64_t want = ceil_div(max_pairs, 256);
         hipLaunchKernelGGL((k_pair_tail<PairV<PR>>), dim3((unsigned)(want < 16384 ? want : 16384)),
                            dim3(256), 0, s, tw.keys[0], reinterpret_cast<PairV<PR>*>(tw.vals[0]),
@@ -2026,21 +1921,15 @@ static int geo_bwd_launch_t(const GeoArgs& a, const am_grid_desc* g, const float
     if (int rc = launch_bwd()) return rc;
     {
         KernelTimer kt_("pair_emit", s);
-        if (part)
-            hipLaunchKernelGGL((k_geo_pairs<LJ, false, PairV<PR>, true>), dim3(pair_blocks(n)), dim3(256),
-                               0, s, a, pts, randn, n, fdv, w.genc, tw.keys[0],
-                               reinterpret_cast<PairV<PR>*>(tw.vals[0]), w.offsets, w.counts,
-                               w.status, tw.m);
-        else
-            hipLaunchKernelGGL((k_geo_pairs<LJ, false, PairV<PR>, false>), dim3(pair_blocks(n)),
-                               dim3(256), 0, s, a, pts, randn, n, fdv, w.genc, tw.keys[0],
-                               reinterpret_cast<PairV<PR>*>(tw.vals[0]), w.offsets, w.counts,
-                               w.status, tw.m);
+        hipLaunchKernelGGL((k_geo_pairs<LJ, false, PairV<PR>>), dim3(pair_blocks(n)), dim3(256), 0,
+                           s, a, pts, randn, n, fdv, w.genc, tw.keys[0],
+                           reinterpret_cast<PairV<PR>*>(tw.vals[0]), w.offsets, w.counts, w.status,
+                           capacity);
     }
     AM_LAUNCH_CHECK();
     if (int rc = colsum_f32(w.partial, waves, a.n_params, dparams, w.ctmp, s)) return rc;
-    if (!bounded) timer_units("table_pairs", tw.m);
-    if (int rc = table_reduce_run(tw, 2, g->n_entries, dtable, s)) return rc;
+    if (!bounded) timer_units("table_pairs", capacity);
+    if (int rc = table_reduce_run(tw, g, dtable, s)) return rc;
     return arm_flag(w.status + 1, s);
 }
 
@@ -2127,11 +2016,9 @@ extern "C" size_t am_sdf_bwd_workspace_size(const am_grid_desc* g, const am_mlp_
     if (make_geo_args(g, m, sd, &a, &LJ) || n < 0) return 0;
     WsCarver c(nullptr, 0);
     GeoBwdWs w;
-    const bool part = geo_prepartition(g);
-    carve_geo_bwd_head(c, a, LJ, n, true, part, &w);
+    carve_geo_bwd_head(c, a, LJ, n, true, &w);
     TableReduceWs tw;
-    if (table_reduce_carve(c, 2, geo_max_pairs(a, LJ, n), g->n_entries, &tw, false, part))
-        return 0;
+    if (table_reduce_carve(c, g, geo_max_pairs(a, LJ, n), &tw)) return 0;
     return c.used + 256;
 }
 

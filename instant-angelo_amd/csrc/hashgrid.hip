@@ -173,8 +173,14 @@ static int hg_fwd(const GridArgs& ga, const float* x, int64_t n, const float* ta
     return AM_OK;
 }
 
+// First pair of each level's stream of k_hg_emit.
+__global__ void k_hg_streams(int L, int active, int64_t per_level, int64_t* __restrict__ start) {
+    const int l = threadIdx.x;
+    if (l <= L) start[l] = per_level * (l < active ? l : active);
+}
+
 template <int F>
-static int hg_bwd(const GridArgs& ga, uint32_t n_entries, const float* x, int64_t n,
+static int hg_bwd(const GridArgs& ga, const am_grid_desc* g, const float* x, int64_t n,
                   const float* table, const float* dy, int active, float* dtable, float* dx,
                   void* ws, size_t ws_bytes, const int32_t* order, hipStream_t s) {
     if (dx) {
@@ -184,10 +190,10 @@ static int hg_bwd(const GridArgs& ga, uint32_t n_entries, const float* x, int64_
     }
     if (dtable) {
         const int64_t m = n * active * 8;
-        if (m == 0) return fill_f32(dtable, (int64_t)n_entries * F, 0.0f, s);
+        if (m == 0) return fill_f32(dtable, (int64_t)g->n_entries * F, 0.0f, s);
         WsCarver c(ws, ws_bytes);
         TableReduceWs w;
-        int rc = table_reduce_carve(c, F, m, n_entries, &w);
+        int rc = table_reduce_carve(c, g, m, &w);
         if (rc) return rc;
         if (!c.ok()) return workspace_short(c.used, ws_bytes);
         {
@@ -198,7 +204,12 @@ static int hg_bwd(const GridArgs& ga, uint32_t n_entries, const float* x, int64_
         }
         AM_LAUNCH_CHECK();
         timer_units("encode_table_pairs", w.m);
-        return table_reduce_run(w, F, n_entries, dtable, s);
+        if (w.paged) {
+            hipLaunchKernelGGL(k_hg_streams, dim3(1), dim3(64), 0, s, ga.L, active, n * 8,
+                               w.level_start);
+            AM_LAUNCH_CHECK();
+        }
+        return table_reduce_run(w, g, dtable, s);
     }
     return AM_OK;
 }
@@ -294,7 +305,7 @@ extern "C" size_t am_hashgrid_bwd_workspace_size(const am_grid_desc* g, int64_t 
     if (check_grid(g) || n < 0 || active_levels < 0 || active_levels > g->n_levels) return 0;
     WsCarver c(nullptr, 0);
     TableReduceWs w;
-    if (table_reduce_carve(c, g->n_features, n * active_levels * 8, g->n_entries, &w)) return 0;
+    if (table_reduce_carve(c, g, n * active_levels * 8, &w)) return 0;
     return c.used + 256;
 }
 
@@ -313,10 +324,10 @@ static int hashgrid_bwd(const am_grid_desc* g, const float* x, int64_t n, const 
     const GridArgs ga = make_grid_args(g);
     hipStream_t s = to_stream(stream);
     switch (g->n_features) {
-        case 1: return hg_bwd<1>(ga, g->n_entries, x, n, table, dy, active_levels, dtable, dx, workspace, workspace_bytes, order, s);
-        case 2: return hg_bwd<2>(ga, g->n_entries, x, n, table, dy, active_levels, dtable, dx, workspace, workspace_bytes, order, s);
-        case 4: return hg_bwd<4>(ga, g->n_entries, x, n, table, dy, active_levels, dtable, dx, workspace, workspace_bytes, order, s);
-        default: return hg_bwd<8>(ga, g->n_entries, x, n, table, dy, active_levels, dtable, dx, workspace, workspace_bytes, order, s);
+        case 1: return hg_bwd<1>(ga, g, x, n, table, dy, active_levels, dtable, dx, workspace, workspace_bytes, order, s);
+        case 2: return hg_bwd<2>(ga, g, x, n, table, dy, active_levels, dtable, dx, workspace, workspace_bytes, order, s);
+        case 4: return hg_bwd<4>(ga, g, x, n, table, dy, active_levels, dtable, dx, workspace, workspace_bytes, order, s);
+        default: return hg_bwd<8>(ga, g, x, n, table, dy, active_levels, dtable, dx, workspace, workspace_bytes, order, s);
     }
 }
 

@@ -1,5 +1,5 @@
-// Deterministic table-gradient reduction: stable radix sort of (row, value)
-// pairs, then a fixed-order segmented reduce (see table_grad.h).
+// Deterministic table-gradient reduction: the paged form, and the stable
+// radix sort with a fixed-order segmented reduce (see table_grad.h).
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 #include "table_grad.h"
@@ -11,6 +11,50 @@ constexpr int64_t kUnitItems = 16384;   // sorted items per work unit (256 chunk
 // Partial-sum slots the units of multi-unit buckets can need: each such
 // bucket holds more than kUnitItems items and fewer than 2n / kUnitItems units.
 static int64_t bucket_slots(int64_t m) { return 2 * (m / kUnitItems) + 1; }
+
+// ---- paged form ----
+constexpr int kPage = 6144;          // pairs a page (two blocks' LDS a CU)
+constexpr int kRowBits = 13;         // rows a bucket: its sums fill the LDS
+constexpr int kRows = 1 << kRowBits;
+constexpr int kMaxDigits = 256;      // buckets a level: 2^21 rows
+constexpr int kRunStride = kMaxDigits + 2;
+// Pairs of a work unit: a level's buckets are cut into slices of about this
+// many pairs where they hold more (coarse levels), fewer when the whole
+// gradient makes less than about 1024 units of the most.
+constexpr int64_t kUnitMost = 1 << 19;
+constexpr int64_t kUnitLeast = 16384;
+
+static bool table_paged(const am_grid_desc* g) {
+    if (g->n_features != 2) return false;
+    for (int l = 0; l < g->n_levels; ++l)
+        if (g->size[l] > (uint32_t)kMaxDigits * kRows) return false;
+    return true;
+}
+
+TableLevels table_levels(const am_grid_desc* g) {
+    TableLevels t{};
+    t.L = g->n_levels;
+    for (int l = 0; l < g->n_levels; ++l) {
+        t.offset[l] = g->offset[l];
+        t.offset[l + 1] = g->offset[l] + g->size[l];
+    }
+    return t;
+}
+
+static int64_t page_bound(int64_t m, int L) { return m / kPage + L; }
+
+// Units of sliced levels: a level of n pairs and D buckets has
+// S = ceil(n / (D U)) slices, D S <= 2 n / U where S > 1.
+static int64_t slot_bound(int64_t m) {
+    const int64_t a = 2 * (m / kUnitLeast), b = 2 * (m / kUnitMost);
+    return (a < 2048 ? a : (b > 2048 ? b : 2048)) + 2;
+}
+
+static int64_t table_digits(const am_grid_desc* g) {
+    int64_t d = 0;
+    for (int l = 0; l < g->n_levels; ++l) d += ceil_div(g->size[l], kRows);
+    return d;
+}
 
 int table_key_bits(uint32_t n_entries) {
     int b = 1;
@@ -52,15 +96,7 @@ static hipError_t sort_pairs(void* tmp, size_t& bytes, TableReduceWs& w, uint32_
     rocprim::double_buffer<uint32_t> kb(w.keys[0], w.keys[1]);
     rocprim::double_buffer<VT> vb(reinterpret_cast<VT*>(w.vals[0]), reinterpret_cast<VT*>(w.vals[1]));
     hipError_t e;
-    if (w.prepart) {   // one 8-bit pass over [17, end_bit), or none
-        e = hipSuccess;
-        if (w.end_bit > kPrepartBits)
-            e = rocprim::radix_sort_pairs<Sort8Config>(tmp, bytes, kb, vb, (size_t)w.m,
-                                                       (unsigned)kPrepartBits,
-                                                       (unsigned)w.end_bit, s, false);
-        else if (tmp == nullptr)
-            bytes = 0;
-    } else if (w.n_buckets > 0 && digit_bits(w) == 8)
+    if (w.n_buckets > 0 && digit_bits(w) == 8)
         e = rocprim::radix_sort_pairs<Sort8Config>(tmp, bytes, kb, vb, (size_t)w.m,
                                                    (unsigned)w.begin_bit, (unsigned)w.end_bit, s,
                                                    false);
@@ -76,18 +112,26 @@ static hipError_t sort_pairs(void* tmp, size_t& bytes, TableReduceWs& w, uint32_
     return e;
 }
 
-int table_reduce_carve(WsCarver& c, int F, int64_t m, uint32_t n_entries, TableReduceWs* out,
-                       bool half_vals, bool prepart) {
+int table_reduce_carve(WsCarver& c, const am_grid_desc* g, int64_t m, TableReduceWs* out,
+                       bool half_vals) {
+    const int F = g->n_features;
+    const uint32_t n_entries = g->n_entries;
     TableReduceWs w{};
     w.m = m;
     w.end_bit = table_key_bits(n_entries);
     w.half_vals = half_vals;
-    if (prepart && (F != 2 || table_bucket_bits(w.end_bit) != 9 || w.end_bit > 25)) {
-        set_error("prepartitioned pairs need two features and 9 < key bits <= 25 (got %d, %d)",
-                  F, w.end_bit);
-        return AM_ERR_INTERNAL;
+    w.paged = table_paged(g);
+    if (w.paged) {
+        const size_t vb = half_vals ? 4 : 8;
+        w.keys[0] = c.take<uint32_t>((size_t)m + 1);
+        w.vals[0] = c.take<char>((size_t)(m + 1) * vb);
+        w.run_start = c.take<uint16_t>((size_t)page_bound(m, g->n_levels) * kRunStride);
+        w.partial2 = c.take<double2>((size_t)slot_bound(m) << kRowBits);
+        w.plan = c.take<PagePlan>(1);
+        w.level_start = c.take<int64_t>(AM_MAX_LEVELS + 1);
+        *out = w;
+        return AM_OK;
     }
-    w.prepart = prepart;
     const size_t vbytes = (size_t)F * (half_vals ? sizeof(__half) : sizeof(float));
     w.keys[0] = c.take<uint32_t>((size_t)m);
     w.keys[1] = c.take<uint32_t>((size_t)m);
@@ -489,6 +533,427 @@ __global__ void __launch_bounds__(256) k_bucket_combine(const uint64_t* __restri
     }
 }
 
+// ---- paged form: kernels ----
+__device__ __forceinline__ int level_digits(const TableLevels& t, int l) {
+    return (int)((t.offset[l + 1] - t.offset[l] + (uint32_t)kRows - 1u) >> kRowBits);
+}
+
+// Inclusive sum over the wave's lanes.
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = __shfl_up(v, d, 64);
+        if ((int)(threadIdx.x & 63) >= d) v += o;
+    }
+    return v;
+}
+
+// One wave, lane = level: pages, slices and work units of the streams.
+__global__ void k_page_plan(TableLevels t, const int64_t* __restrict__ level_start,
+                            PagePlan* __restrict__ plan) {
+    const int l = threadIdx.x;
+    const bool on = l < t.L;
+    const int64_t s = on ? level_start[l] : 0, e = on ? level_start[l + 1] : 0;
+    const int64_t total = level_start[t.L] - level_start[0];
+    int64_t unit = total / 1024;
+    unit = unit < kUnitLeast ? kUnitLeast : (unit > kUnitMost ? kUnitMost : unit);
+    const int64_t n = e - s;
+    const int D = on ? level_digits(t, l) : 0;
+    const uint32_t pages = (uint32_t)((n + kPage - 1) / kPage);
+    int64_t S = on ? (n + D * unit - 1) / (D * unit) : 0;
+    if (on && S < 1) S = 1;
+    const uint32_t units = (uint32_t)(D * S);
+    const uint32_t slots = S > 1 ? units : 0u;
+    const uint32_t rows = S > 1 ? t.offset[l + 1] - t.offset[l] : 0u;   // combined afterwards
+    const uint32_t ps = wave_scan(pages), us = wave_scan(units), ss = wave_scan(slots),
+                   rs = wave_scan(rows);
+    const uint32_t all = __shfl(us, 63, 64);
+    if (on) {
+        plan->level_start[l] = s;
+        plan->page_base[l] = (int32_t)(ps - pages);
+        // finest level first: its buckets hold the most pairs
+        plan->unit_base[l] = (int32_t)(all - us);
+        plan->slices[l] = (int32_t)S;
+        plan->slot_base[l] = (int32_t)(ss - slots);
+        plan->row_base[l] = (int32_t)(rs - rows);
+        if (l == t.L - 1) {
+            plan->level_start[l + 1] = e;
+            plan->page_base[l + 1] = (int32_t)ps;
+            plan->row_base[l + 1] = (int32_t)rs;
+        }
+        if (l == 0) plan->unit_base[t.L] = (int32_t)all;
+    }
+}
+
+__device__ __forceinline__ float2 pair_value(uint2 v) {
+    return make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
+}
+__device__ __forceinline__ float2 pair_value(uint32_t v) {
+    return __half22float2(__builtin_bit_cast(__half2, v));
+}
+
+__device__ __forceinline__ uint32_t pair_word(uint2 v, int w) { return w ? v.y : v.x; }
+__device__ __forceinline__ uint32_t pair_word(uint32_t v, int) { return v; }
+
+// Partitions one page in place by its pairs' bucket (row >> 13 within the
+// level): a bucket's run holds its pairs in any order (the reduce's sums do
+// not depend on it), so each pair's place comes from one LDS counter; in runs
+// of 64 pairs or more, pairs that arrive together (neighbouring samples,
+// often of one row) are set a load apart, so that the reduce's LDS additions
+// seldom meet in one row (runs of 16 equal rows: reduce 0.80 -> 0.34 ms for
+// 60 M pairs).  The key words then hold the row within the bucket (bits 0-12)
+// and the two values' exponents (13-20, 21-28).  Bound by memory: 12 bytes in
+// and 12 out a pair, 0.29 ms for 60 M pairs (5.0 TB/s).  Two blocks of 1024
+// threads share a CU, one loading while the other scatters; pages twice as
+// long give the reduce longer runs (0.34 -> 0.29 ms) but take 0.40 ms here.
+template <class VT>
+__global__ void __launch_bounds__(1024) k_page_partition(TableLevels t,
+                                                         const PagePlan* __restrict__ plan,
+                                                         uint32_t* __restrict__ keys,
+                                                         VT* __restrict__ vals,
+                                                         uint16_t* __restrict__ run_start) {
+    __shared__ VT sv[kPage];
+    __shared__ __attribute__((aligned(16))) uint16_t sk[kPage];
+    __shared__ uint32_t hist[kMaxDigits + 1];
+    __shared__ uint32_t wsum[kMaxDigits / 64];
+    constexpr int kItems = kPage / 1024;
+    const int page = (int)blockIdx.x, tid = (int)threadIdx.x;
+    if (page >= plan->page_base[t.L]) return;
+    int l = 0;
+    while (page >= plan->page_base[l + 1]) ++l;
+    const int64_t first = plan->level_start[l] + (int64_t)(page - plan->page_base[l]) * kPage;
+    const int64_t left = plan->level_start[l + 1] - first;
+    const int n = left < kPage ? (int)left : kPage;
+    const uint32_t off = t.offset[l];
+    uint32_t key[kItems], rank[kItems];
+    VT val[kItems];
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {
+        const int i = tid + 1024 * k;
+        if (i < n) {
+            key[k] = keys[first + i] - off;
+            val[k] = vals[first + i];
+        }
+    }
+    if (tid < kMaxDigits) hist[tid] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kItems; ++k)
+        if (tid + 1024 * k < n)
+            rank[k] = atomicAdd(&hist[(key[k] >> kRowBits) & (uint32_t)(kMaxDigits - 1)], 1u);
+    __syncthreads();
+    uint32_t c = 0, inc = 0;
+    if (tid < kMaxDigits) {
+        c = hist[tid];
+        inc = wave_scan(c);
+        if ((tid & 63) == 63) wsum[tid >> 6] = inc;
+    }
+    __syncthreads();
+    if (tid == 0) hist[kMaxDigits] = (uint32_t)n;
+    if (tid < kMaxDigits) {
+        uint32_t b = inc - c;
+        for (int q = 0; q < (tid >> 6); ++q) b += wsum[q];
+        hist[tid] = b;
+        uint16_t* rs = run_start + (int64_t)page * kRunStride;
+        rs[tid] = (uint16_t)b;
+        if (tid == kMaxDigits - 1) rs[kMaxDigits] = (uint16_t)n;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kItems; ++k)
+        if (tid + 1024 * k < n) {
+            const uint32_t dg = (key[k] >> kRowBits) & (uint32_t)(kMaxDigits - 1);
+            const uint32_t h0 = hist[dg], q = (hist[dg + 1] - h0) >> 5;
+            uint32_t at = rank[k];
+            if (q > 1u && at < q << 5) {
+                const uint32_t hi = (uint32_t)(((float)at + 0.5f) * __builtin_amdgcn_rcpf((float)q));
+                at = (at - hi * q) * 32u + hi;
+            }
+            at += h0;
+            sv[at] = val[k];
+            sk[at] = (uint16_t)(key[k] & (uint32_t)(kRows - 1));
+        }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {
+        const int i = tid + 1024 * k;
+        if (i < n) vals[first + i] = sv[i];
+    }
+#pragma unroll
+    for (int k = 0; k < kItems; ++k) {
+        const int i = tid + 1024 * k;
+        if (i < n) {
+            const float2 f = pair_value(sv[i]);
+            keys[first + i] = (uint32_t)sk[i] |
+                              (__float_as_uint(f.x) >> 23 & 255u) << kRowBits |
+                              (__float_as_uint(f.y) >> 23 & 255u) << (kRowBits + 8);
+        }
+    }
+}
+
+// Runs of one bucket in pages [p0, p1) of a level.  A wave takes every 16th
+// pair of pages: its lanes look 64 runs up at once, and each half of the wave
+// then reads its page's run, 32 pairs a load, eight pairs of pages in flight
+// together.  body.load(base, i): pair base + i of the arrays (base is the
+// same for the wave); body.use(payload).  Returns the pairs of the runs that
+// this lane looked up.
+struct RunSpan {
+    const uint16_t* run_start;   // the level's first page, at the bucket
+    int64_t first;               // the level's first pair
+    int p0, p1;
+};
+
+template <class Body>
+__device__ __forceinline__ uint32_t for_runs(const RunSpan& s, const Body& body) {
+    constexpr int kU = 8;
+    const uint32_t lane = threadIdx.x & 63u, p = lane & 31u, half = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    uint32_t total = 0;
+    for (int b = s.p0 + 2 * wave; b < s.p1; b += 32 * 32) {
+        const int mine = b + 32 * (int)(lane >> 1) + (int)(lane & 1u);
+        uint32_t both = 0;   // two neighbouring 16-bit entries: start, end
+        if (mine < s.p1) __builtin_memcpy(&both, s.run_start + (int64_t)mine * kRunStride, 4);
+        total += (both >> 16) - (both & 0xffffu);
+        const int pairs = (s.p1 - b + 31) / 32 < 32 ? (s.p1 - b + 31) / 32 : 32;
+        for (int q = 0; q < pairs; q += kU) {
+            const int64_t base0 = s.first + (int64_t)(b + 32 * q) * kPage;
+            typename Body::Payload v[kU];
+            uint32_t run[kU];
+            bool longer = false;
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)both, (2 * (q + u)) & 63);
+                const uint32_t d1 = (uint32_t)__builtin_amdgcn_readlane((int)both, (2 * (q + u) + 1) & 63);
+                longer = longer || (d0 >> 16) - (d0 & 0xffffu) > 32u || (d1 >> 16) - (d1 & 0xffffu) > 32u;
+                run[u] = half ? d1 : d0;
+                const uint32_t i = (run[u] & 0xffffu) + p;
+                if (i < run[u] >> 16)
+                    v[u] = body.load(base0 + (int64_t)(u * 32 * kPage), i + half * (uint32_t)kPage);
+            }
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                if ((run[u] & 0xffffu) + p < run[u] >> 16) body.use(v[u]);
+            if (!longer) continue;
+#pragma unroll 1
+            for (int u = 0; u < kU; ++u) {
+                const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)both, (2 * (q + u)) & 63);
+                const uint32_t d1 = (uint32_t)__builtin_amdgcn_readlane((int)both, (2 * (q + u) + 1) & 63);
+                const uint32_t d = half ? d1 : d0, e = d >> 16;
+                const int64_t base = base0 + (int64_t)(u * 32 * kPage);
+                for (uint32_t i = (d & 0xffffu) + p + 32u; i < e; i += 128u) {
+                    typename Body::Payload w[4];
+#pragma unroll
+                    for (uint32_t c = 0; c < 4; ++c)
+                        if (i + 32u * c < e) w[c] = body.load(base, i + 32u * c + half * (uint32_t)kPage);
+#pragma unroll
+                    for (uint32_t c = 0; c < 4; ++c)
+                        if (i + 32u * c < e) body.use(w[c]);
+                }
+            }
+        }
+    }
+    return total;
+}
+
+// The rows' largest exponents.
+struct RunMax {
+    using Payload = uint32_t;
+    const uint32_t* keys;
+    uint32_t* mx;
+    __device__ __forceinline__ uint32_t load(int64_t base, uint32_t i) const {
+        return (keys + base)[i];
+    }
+    __device__ __forceinline__ void use(uint32_t w) const {
+        const uint32_t row = w & (uint32_t)(kRows - 1);
+        atomicMax(&mx[row], w >> kRowBits & 255u);
+        atomicMax(&mx[kRows + row], w >> (kRowBits + 8));
+    }
+};
+
+// v as a multiple of its row's grid, 2^(e - 126 - Q) with e the row's largest
+// exponent: the low bits of v + c, c = 1.5 * 2^52 grid steps, less c's.
+// ck = (897 + 52 - Q) << 20 | 0x80000: c's high word is (e << 20) + ck.
+__device__ __forceinline__ unsigned long long grid_steps(float v, uint32_t e, uint32_t ck) {
+    const uint32_t ch = (e << 20) + ck;
+    const double x = (double)v + __hiloint2double((int)ch, 0);
+    return (unsigned long long)((uint32_t)__double2hiint(x) - ch) << 32 |
+           (uint32_t)__double2loint(x);
+}
+
+// A value added to a row with an infinity or NaN: flags (1 NaN, 2 +inf,
+// 4 -inf) in place of the sum.
+__device__ __forceinline__ void add_special(float v, unsigned long long* acc) {
+    const uint32_t b = __float_as_uint(v);
+    if ((b & 0x7f800000u) != 0x7f800000u) return;
+    const uint32_t f = (b & 0x7fffffu) ? 1u : ((b >> 31) ? 4u : 2u);
+    atomicOr(reinterpret_cast<uint32_t*>(acc), f);
+}
+
+// The values added up; kSpecial: some row of the bucket holds an infinity or
+// NaN.
+template <class VT, bool kSpecial>
+struct RunAdd {
+    struct Payload {
+        uint32_t w;
+        VT v;
+    };
+    const uint32_t* keys;
+    const VT* vals;
+    const uint16_t* ex;
+    unsigned long long* acc;
+    uint32_t ck;
+    __device__ __forceinline__ Payload load(int64_t base, uint32_t i) const {
+        return Payload{(keys + base)[i], (vals + base)[i]};
+    }
+    __device__ __forceinline__ void use(const Payload& p) const {
+        const float2 v = pair_value(p.v);
+        const uint32_t row = p.w & (uint32_t)(kRows - 1);
+        const uint32_t e = ex[row], e0 = e & 255u, e1 = e >> 8;
+        if (kSpecial && e0 == 255u) add_special(v.x, &acc[row]);
+        else atomicAdd(&acc[row], grid_steps(v.x, e0, ck));
+        if (kSpecial && e1 == 255u) add_special(v.y, &acc[kRows + row]);
+        else atomicAdd(&acc[kRows + row], grid_steps(v.y, e1, ck));
+    }
+};
+
+// The sum of a row: its steps times the grid.
+__device__ __forceinline__ double row_sum(unsigned long long a, uint32_t e, int Q) {
+    if (e == 255u) {
+        const uint32_t f = (uint32_t)a;
+        const double inf = __hiloint2double(0x7ff00000, 0);
+        return f == 2u ? inf : (f == 4u ? -inf : __hiloint2double(0x7ff80000, 0));
+    }
+    return ldexp((double)(long long)a, (int)e - 126 - Q);
+}
+
+// One block per work unit: a bucket of 8192 rows, or a slice of its level's
+// pages.  Two passes over the bucket's runs: the largest exponent of each
+// row (LDS max over the key words), then the values, as whole
+// numbers of their row's grid, added into 64-bit integers in LDS.  With at
+// most 2^b pairs in the unit, the grid is 2^-Q of the row's largest binade,
+// Q = min(50, 61 - b), so the integer sums cannot overflow and are exact in
+// any order: no sort, no barrier between the additions, and the same bits on
+// every run.  A value's rounding to the grid (2^-45 of the row's largest at
+// 10^5 pairs a unit; none for values within 2^-21 of it) is far below that
+// of a float sum.
+// 1024 threads and 144 KB of LDS (the first pass's maxima lie where the sums
+// go, and are packed to 16 bits a row before the second): one block a CU.
+template <class VT>
+__global__ void __launch_bounds__(1024) k_page_reduce(TableLevels t,
+                                                      const PagePlan* __restrict__ plan,
+                                                      const uint32_t* __restrict__ keys,
+                                                      const VT* __restrict__ vals,
+                                                      const uint16_t* __restrict__ run_start,
+                                                      float* __restrict__ out,
+                                                      double2* __restrict__ partial) {
+    __shared__ unsigned long long acc[2 * kRows];
+    __shared__ uint16_t ex[kRows];
+    __shared__ uint32_t pairs;
+    uint32_t* mx = reinterpret_cast<uint32_t*>(acc);
+    const int tid = (int)threadIdx.x;
+    // blocks b, b + 8, ... share an XCD: 32 neighbouring units at a time, whose
+    // runs share cache lines
+    const int bx = (int)blockIdx.x & 7, by = (int)blockIdx.x >> 3;
+    const int u = ((by >> 5) * 8 + bx) * 32 + (by & 31);
+    if (u >= plan->unit_base[t.L]) return;
+    int l = t.L - 1;
+    while (l > 0 && u >= plan->unit_base[l - 1]) --l;
+    const int D = level_digits(t, l), S = plan->slices[l];
+    const int v = u - plan->unit_base[l];
+    const int slice = v / D, d = v - slice * D;
+    const int pb = plan->page_base[l], np = plan->page_base[l + 1] - pb;
+    RunSpan s;
+    s.run_start = run_start + (int64_t)pb * kRunStride + d;
+    s.first = plan->level_start[l];
+    s.p0 = (int)((int64_t)np * slice / S);
+    s.p1 = (int)((int64_t)np * (slice + 1) / S);
+    for (int q = tid; q < 2 * kRows; q += 1024) mx[q] = 0u;
+    if (tid == 0) pairs = 0u;
+    __syncthreads();
+    const uint32_t mine = wave_scan(for_runs(s, RunMax{keys, mx}));
+    if ((tid & 63) == 63) atomicAdd(&pairs, mine);
+    __syncthreads();
+    bool special = false;
+    for (int q = tid; q < kRows; q += 1024) {
+        const uint32_t e0 = mx[q], e1 = mx[kRows + q];
+        special = special || e0 == 255u || e1 == 255u;
+        ex[q] = (uint16_t)(e0 | e1 << 8);
+    }
+    special = __syncthreads_or(special) != 0;
+    for (int q = tid; q < 2 * kRows; q += 1024) acc[q] = 0ull;
+    const int b = pairs > 1u ? 32 - __clz((int)(pairs - 1u)) : 0;
+    const int Q = 61 - b < 50 ? 61 - b : 50;
+    const uint32_t ck = (uint32_t)(897 + 52 - Q) << 20 | 0x80000u;
+    __syncthreads();
+    if (special) for_runs(s, RunAdd<VT, true>{keys, vals, ex, acc, ck});
+    else for_runs(s, RunAdd<VT, false>{keys, vals, ex, acc, ck});
+    __syncthreads();
+    const uint32_t rows = t.offset[l + 1] - t.offset[l];
+    double2* dst = partial + ((int64_t)(plan->slot_base[l] + d * S + slice) << kRowBits);
+#pragma unroll
+    for (int r = 0; r < kRows / 1024; ++r) {
+        const int q = tid + 1024 * r;
+        const uint32_t e = ex[q];
+        const double x = row_sum(acc[q], e & 255u, Q), y = row_sum(acc[kRows + q], e >> 8, Q);
+        const uint32_t row = (uint32_t)d * kRows + q;
+        if (S > 1) dst[q] = make_double2(x, y);
+        else if (row < rows)
+            *reinterpret_cast<float2*>(out + 2 * ((int64_t)t.offset[l] + row)) =
+                make_float2((float)x, (float)y);
+    }
+}
+
+// Sliced levels: each row is the sum of its slices' partials in order.
+__global__ void __launch_bounds__(256) k_page_combine(TableLevels t,
+                                                      const PagePlan* __restrict__ plan,
+                                                      const double2* __restrict__ partial,
+                                                      float* __restrict__ out) {
+    const uint32_t all = (uint32_t)plan->row_base[t.L];
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < all; i += gridDim.x * 256u) {
+        int l = 0;
+        while (i >= (uint32_t)plan->row_base[l + 1]) ++l;
+        const uint32_t q = i - (uint32_t)plan->row_base[l];
+        const int S = plan->slices[l];
+        const double2* src = partial +
+                             ((int64_t)(plan->slot_base[l] + (int)(q >> kRowBits) * S) << kRowBits) +
+                             (q & (uint32_t)(kRows - 1));
+        double a = 0.0, b = 0.0;
+#pragma unroll 4
+        for (int j = 0; j < S; ++j) {
+            const double2 p = src[(int64_t)j << kRowBits];
+            a += p.x;
+            b += p.y;
+        }
+        *reinterpret_cast<float2*>(out + 2 * ((int64_t)t.offset[l] + q)) =
+            make_float2((float)a, (float)b);
+    }
+}
+
+template <class VT>
+static int run_paged(TableReduceWs& w, const am_grid_desc* g, float* dtable, hipStream_t s) {
+    const TableLevels t = table_levels(g);
+    VT* vals = reinterpret_cast<VT*>(w.vals[0]);
+    {
+        KernelTimer kt_("radix_sort", s);
+        hipLaunchKernelGGL(k_page_plan, dim3(1), dim3(64), 0, s, t, w.level_start, w.plan);
+        AM_LAUNCH_CHECK();
+        hipLaunchKernelGGL((k_page_partition<VT>), dim3((unsigned)page_bound(w.m, t.L)), dim3(1024),
+                           0, s, t, w.plan, w.keys[0], vals, w.run_start);
+        AM_LAUNCH_CHECK();
+    }
+    KernelTimer kt_("seg_reduce", s);
+    // units <= buckets + pairs / unit pairs (both unit sizes of k_page_plan)
+    const int64_t least = w.m / kUnitLeast, most = w.m / kUnitMost;
+    const int64_t units = table_digits(g) + (least < 1024 ? least : (most > 1024 ? most : 1024)) + 2;
+    const unsigned grid = (unsigned)(ceil_div(units, 256) * 256);   // whole groups of 8 x 32
+    hipLaunchKernelGGL((k_page_reduce<VT>), dim3(grid), dim3(1024), 0, s, t, w.plan, w.keys[0], vals,
+                       w.run_start, dtable, w.partial2);
+    AM_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_page_combine, dim3(2048), dim3(256), 0, s, t, w.plan, w.partial2, dtable);
+    AM_LAUNCH_CHECK();
+    return AM_OK;
+}
+
 template <class VT>
 static int run_bucketed(TableReduceWs& w, uint32_t n_entries, float* dtable, hipStream_t s) {
     uint32_t* ks = w.keys[0];
@@ -575,8 +1040,13 @@ static int run_f(TableReduceWs& w, uint32_t n_entries, float* dtable, hipStream_
     return AM_OK;
 }
 
-int table_reduce_run(TableReduceWs& w, int F, uint32_t n_entries, float* dtable,
+int table_reduce_run(TableReduceWs& w, const am_grid_desc* g, float* dtable,
                      hipStream_t stream) {
+    const int F = g->n_features;
+    const uint32_t n_entries = g->n_entries;
+    if (w.paged)
+        return w.half_vals ? run_paged<uint32_t>(w, g, dtable, stream)
+                           : run_paged<uint2>(w, g, dtable, stream);
     if (F == 2 && w.n_buckets > 0) {
         if (w.begin_bit > kMaxBucketBits) {
             set_error("bucket bits %d above %d", w.begin_bit, kMaxBucketBits);
