@@ -17,26 +17,12 @@
 //                recompute form), back-propagates it on MFMA and writes the
 //                encode gradient to HBM; MLP weight gradients are per-wave
 //                register accumulators summed in a fixed order;
-//   k_geo_pairs  turns the encode gradients into table-gradient pairs:
-//     1. per lane and level, the evaluations of a cluster (base + 6 FD, or
-//        the 6 curvature points) are merged into the cell B of the cluster
-//        centre with a star stencil: an evaluation in B adds its 8 corners,
-//        one in a face neighbour of B adds the 4 corners of the shared face
-//        and emits its 4 far corners, any other emits its 8 corners;
-//     2. B's corner sums are merged with equal-B lanes of the same lane
-//        group (neighbouring samples of a ray) by a segmented reduction in a
-//        fixed shuffle tree;
-//     3. the same kernel in count mode makes these decisions from positions
-//        alone first; an integer prefix sum of the per-tile counts gives
-//        each tile its first pair, so the pairs land compacted, and a stable
-//        radix sort + fixed-order segmented reduce gives dtable.
-#include "hashgrid_dev.h"
+//   pairs.hip    turns the encode gradients into table-gradient pairs,
+//   table_grad.hip adds them up into dtable.
 #include "mlp_dev.h"
-#include "table_grad.h"
+#include "pairs.h"
 #include "field_common.h"
 #include <mutex>
-#include <type_traits>
-#include <rocprim/device/device_scan.hpp>
 
 namespace am {
 // Row stride (floats) of the 64-column weight matrices in LDS (W2 and the
@@ -50,38 +36,6 @@ constexpr int kWLd = 67;
 namespace am {
 
 using mlp::krow;
-
-struct GeoArgs {
-    GridArgs g;
-    float r, inv2r, eps, inv_eps, inv_pi;
-    int with_grad, with_laplace, recontract, active;
-    int n_in, n_out, act;
-    float beta;
-    int w1, b1, w2, b2, wo, bo, ld1, lds_floats;  // LDS offsets (floats)
-    // output tiles of 16 rows (n_out <= 16 * out_tiles); the rows of tiles
-    // >= 1 are features only, read by the base evaluation alone
-    int out_tiles;
-    int64_t pw1, pb1, pw2, pb2, pwo, pbo, n_params;
-    int n_evals;  // 1, 7 or 13
-    int prec;     // AM_PREC_FP32 / AM_PREC_MIXED
-    // analytic-gradient mode: the base evaluation carries d enc / d x and
-    // grad = d sdf / d x through the MLP; no FD evaluations.  Slots: curv0 =
-    // first curvature evaluation (7 FD mode, 1 analytic), n_dx = stored
-    // position-derivative slots (the analytic base, then the 6 curvature
-    // evaluations), genc_slots = encode-gradient slots per tile (n_evals, and
-    // 3 more in analytic mode: u * scale * g_x along each axis).
-    int analytic, curv0, n_dx, dx_curv0, genc_slots;
-    // Evaluation order: kernel sample n is the caller's sample order[n]
-    // (nullptr: the caller's order).  Inputs (positions, curvature
-    // directions, upstream gradients) and outputs are addressed in the
-    // caller's order; the forward's saved values (FD values, stored
-    // encodings) and the encode gradients in the kernels' order.
-    const int32_t* order;
-};
-
-__device__ __forceinline__ int64_t caller_row(const GeoArgs& a, int64_t n, bool valid) {
-    return (a.order && valid) ? (int64_t)a.order[n] : n;
-}
 
 // Row-space column of the SDF MLP first layer for lane-group level slots:
 // K-step s < 2LJ -> level k + 4(s/2), feature s%2; s == 2LJ -> xyz[k].
@@ -140,10 +94,6 @@ struct GeoEval {
     v4f out;
     float dx[DX ? LJ : 1][2][3];
 };
-
-__device__ __forceinline__ float pick3(const float v[3], int k) {
-    return k == 0 ? v[0] : (k == 1 ? v[1] : v[2]);
-}
 
 // Encode of this lane's level slots at contracted point x (e.xb[0..2LJ),
 // and with DX the position derivatives e.dx).
@@ -284,102 +234,6 @@ __device__ __forceinline__ void geo_eval_b(const GeoArgs& a, const float* sm, co
     else geo_encode<LJ, NH, DX>(a, lv, table, x, e);
     geo_mlp_hidden<LJ, NH, DX, PR>(a, sm, x, e);
 }
-
-__device__ __forceinline__ float contract1(float v, const GeoArgs& a) { return (v + a.r) * a.inv2r; }
-
-__device__ __forceinline__ float clampr(float v, float r) { return fminf(fmaxf(v, -r), r); }
-
-// Offset point j (axis j/2, sign + for even j) around `base` (world units,
-// as the reference adds the offsets to it), clamped and contracted; mask =
-// the clamp passed the coordinate through.
-__device__ __forceinline__ void offset_point(const GeoArgs& a, const float base[3], int j,
-                                             float x[3], bool mask[3]) {
-    const int ax = j >> 1;
-    const float off = (j & 1) ? -a.eps : a.eps;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const float v = base[d] + (d == ax ? off : 0.0f);
-        mask[d] = v >= -a.r && v <= a.r;
-        x[d] = contract1(clampr(v, a.r), a);
-    }
-}
-
-__device__ __forceinline__ void normalize3(const float v[3], float out[3]) {
-    const float n = sqrtf((v[0] * v[0] + v[1] * v[1]) + v[2] * v[2]);
-    const float d = fmaxf(n, 1e-12f);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) out[q] = v[q] / d;
-}
-
-// Backward of y = v / max(|v|, 1e-12) (F.normalize).
-__device__ __forceinline__ void normalize3_bwd(const float v[3], const float g[3], float out[3]) {
-    const float n = sqrtf((v[0] * v[0] + v[1] * v[1]) + v[2] * v[2]);
-    const float d = fmaxf(n, 1e-12f);
-    const float gv = g[0] * v[0] + g[1] * v[1] + g[2] * v[2];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        float r = g[q] / d;
-        if (n >= 1e-12f) r -= gv / (d * d) * (v[q] / n);
-        out[q] = r;
-    }
-}
-
-__device__ __forceinline__ void cross3(const float a[3], const float b[3], float c[3]) {
-    c[0] = a[1] * b[2] - a[2] * b[1];
-    c[1] = a[2] * b[0] - a[0] * b[2];
-    c[2] = a[0] * b[1] - a[1] * b[0];
-}
-
-// Per-sample state rebuilt from the 12 stored SDF values (all lanes of the
-// sample hold it).
-struct GeoSample {
-    float P[3], x0[3];
-    float grad[3], n[3];
-    float rn[3], ps[3], grad_s[3], ns[3], dot;
-};
-
-__device__ __forceinline__ void diff_pair(float* acc3, int j, float v) {
-    // acc[j/2] = f+ then f+ - f- : bit-identical to the single subtraction
-    const int ax = j >> 1;
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-        if (d == ax) acc3[d] = (j & 1) ? acc3[d] - v : v;
-}
-
-__device__ __forceinline__ void finish_grad(const GeoArgs& a, float g[3]) {
-#pragma unroll
-    for (int d = 0; d < 3; ++d) g[d] = (0.5f * g[d]) * a.inv_eps;
-}
-
-// grad -> normal -> tangent -> shifted point.
-__device__ __forceinline__ void geo_tangent(const GeoArgs& a, const float* __restrict__ randn,
-                                            int64_t n, bool valid, GeoSample& s) {
-    float rd[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) rd[d] = valid ? randn[3 * n + d] : 1.0f;
-    normalize3(rd, s.rn);
-    float t[3];
-    cross3(s.n, s.rn, t);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const float base = a.recontract ? s.x0[d] : s.P[d];
-        s.ps[d] = base + t[d] * a.eps;
-    }
-}
-
-// Precision forms of the fused field (template PR).  Mixed: the table rows
-// are read in fp16 and the table-gradient pair values are stored in fp16
-// (summed in fp32); the SDF MLP stays fp32 in both forms, because the
-// central differences of the FD normal divide each evaluation's rounding
-// by eps (bf16 activations there gave normals off by 0.3 on average at the
-// Neuralangelo shapes, while a fixed fp16 rounding of the table keeps the
-// field smooth).
-// Table storage of a precision form: fp32 rows, or fp16 rows (mixed form).
-template <int PR>
-using TableT = typename std::conditional<PR == mlp::kF32, float2, __half2>::type;
-// Table-gradient pair values: fp32, or fp16 (mixed form, loss-scaled).
-template <int PR>
-using PairV = typename std::conditional<PR == mlp::kF32, Vals<2>, ValsH<2>>::type;
 
 // sdf and feature outputs of the base evaluation: output tile 0 from e.out,
 // the feature rows of tiles >= 1 (n_out > 16) from the last hidden layer.
@@ -660,7 +514,7 @@ __device__ __forceinline__ v4f go_row0(float g) {
 
 // MLP backward of one evaluation with output gradient `go` (D tile rows =
 // outputs): accumulates weight gradients, stores the encode gradient of the
-// lane's level slots to genc (LDS, slot-major [LJ][2][64]) and, with DX,
+// lane's level slots to genc (the slot's place of genc_lane) and, with DX,
 // returns the contracted-position gradient (summed over the 4 lane groups).
 template <int LJ, int NH, bool DX, int PR>
 __device__ __forceinline__ void geo_eval_bwd(const GeoArgs& a, const float* sm,
@@ -708,8 +562,8 @@ __device__ __forceinline__ void geo_eval_bwd(const GeoArgs& a, const float* sm,
     const mlp::FragV gb{gin};  // gb[s] = gradient of B fragment s
 #pragma unroll
     for (int j = 0; j < LJ; ++j) {
-        genc[(2 * j) * 64 + l] = gb[2 * j];
-        genc[(2 * j + 1) * 64 + l] = gb[2 * j + 1];
+        genc[j * 512] = gb[2 * j];
+        genc[j * 512 + 64] = gb[2 * j + 1];
     }
     if constexpr (DX) {
         float gp[3] = {0.0f, 0.0f, 0.0f};
@@ -866,434 +720,14 @@ __device__ __forceinline__ void geo_eval_bwd_an(const GeoArgs& a, const float* s
     const mlp::FragV gb{gin}, ub{uin};
 #pragma unroll
     for (int j = 0; j < LJ; ++j) {
-        genc[(2 * j) * 64 + l] = gb[2 * j];
-        genc[(2 * j + 1) * 64 + l] = gb[2 * j + 1];
+        genc[j * 512] = gb[2 * j];
+        genc[j * 512 + 64] = gb[2 * j + 1];
         const int level = k + 4 * j;
         const float sc = level < a.g.L ? lv[level].scale : 0.0f;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            gext[d * LJ * 128 + (2 * j) * 64 + l] = ub[2 * j] * sc * gx[d];
-            gext[d * LJ * 128 + (2 * j + 1) * 64 + l] = ub[2 * j + 1] * sc * gx[d];
-        }
-    }
-}
-
-// ---- pair emission with merging ----
-// The pairs of a tile at one level go to [keys, keys + limit): limit is the
-// count the count pass found for them; the emit pass makes the same
-// decisions, and never writes past limit.  Each lane group (16 lanes, one
-// level) has its own.
-template <class VT>
-struct EmitTile {
-    uint32_t* keys;   // the tile's first pair at the level (keys)
-    VT* vals;         // the same (values); atomic form: the table gradient
-    int cursor;       // group-uniform write position
-    int limit;        // pairs reserved
-};
-
-// Atomic form (flag "table_atomic"): the "pair array" is the table gradient
-// itself, [n_entries] rows of 2 floats, and each pair is added into its row
-// with hardware float atomics: no count pass, no sort, no host read, but the
-// summation order varies from run to run (the tcnn hash-grid backward's
-// semantics).
-struct AtomicRow {
-    float v[2];
-};
-template <class VT>
-constexpr bool kAtomicPairs = std::is_same<VT, AtomicRow>::value;
-
-// Lanes with `on` write K pairs (rows, values); COUNT only advances the
-// cursor.
-__device__ __forceinline__ void set_pair(Vals<2>& v, float a, float b) {
-    v.v[0] = a;
-    v.v[1] = b;
-}
-__device__ __forceinline__ void set_pair(ValsH<2>& v, float a, float b) {
-    v.v[0] = __float2half_rn(a);
-    v.v[1] = __float2half_rn(b);
-}
-__device__ __forceinline__ void set_pair(AtomicRow& v, float a, float b) {   // type-checks only
-    v.v[0] = a;
-    v.v[1] = b;
-}
-
-// The lane group's K * n pairs (n lanes on) fill [cursor, cursor + K n)
-// corner-major: pair c of the lane of rank r goes to cursor + c n + r, so each
-// store instruction writes consecutive addresses across the group's lanes.
-template <int K, bool COUNT, class VT>
-__device__ __forceinline__ void emit_pairs(EmitTile<VT>& et, bool on, const uint32_t rows[K],
-                                           const float vals[2 * K]) {
-    if constexpr (kAtomicPairs<VT>) {
-        static_assert(!COUNT, "the atomic form has no count pass");
-        if (on) {
-#pragma unroll
-            for (int c = 0; c < K; ++c) {
-                float* row = et.vals[rows[c]].v;
-                unsafeAtomicAdd(row, vals[2 * c]);
-                unsafeAtomicAdd(row + 1, vals[2 * c + 1]);
-            }
-        }
-        return;
-    }
-    const int l = lane_id(), k = l >> 4;
-    const uint64_t mask = __ballot(on);
-    const uint32_t half = (k & 2) ? (uint32_t)(mask >> 32) : (uint32_t)mask;
-    const uint32_t group = ((k & 1) ? half >> 16 : half) & 0xffffu;
-    const int n_on = __popc(group);
-    if (!COUNT && on && et.cursor + K * n_on <= et.limit) {
-        const int off = et.cursor + __popc(group & ((1u << (l & 15)) - 1u));
-#pragma unroll
-        for (int c = 0; c < K; ++c) {
-            et.keys[off + c * n_on] = rows[c];
-            VT v;
-            set_pair(v, vals[2 * c], vals[2 * c + 1]);
-            et.vals[off + c * n_on] = v;
-        }
-    }
-    et.cursor += K * n_on;
-}
-
-// The 8 corner rows of `cell` at level `lp` (corner c = cell + bits of c).
-__device__ __forceinline__ void corner_rows(const LevelParams& lp, const uint32_t cell[3],
-                                            uint32_t rows[8]) {
-    cell_rows(lp, cell, rows);
-}
-
-// Corner i (0..3) of the face of a cell with bit `ax` fixed to `b`.
-__device__ __forceinline__ int face_corner(int i, int ax, int b) {
-    const int low = i & ((1 << ax) - 1);
-    return low | (b << ax) | ((i >> ax) << (ax + 1));
-}
-
-
-// Position of cluster evaluation q (0..n-1) for this lane.
-template <int CL>
-__device__ __forceinline__ void cluster_point(const GeoArgs& a, const GeoSample& s, int q,
-                                              float x[3]) {
-    bool inb[3];
-    if (CL == 0) {  // base, then FD 0..5
-        if (q == 0) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d) x[d] = s.x0[d];
-        } else {
-            offset_point(a, s.P, q - 1, x, inb);
-        }
-    } else {        // curvature 0..5
-        offset_point(a, s.ps, q, x, inb);
-    }
-}
-
-// Centre of a cluster: the base point (FD cluster) or the tangent-shifted
-// point (curvature cluster; not itself evaluated), clamped and contracted as
-// its offsets are.
-template <int CL>
-__device__ __forceinline__ void cluster_center(const GeoArgs& a, const GeoSample& s, float x[3]) {
-#pragma unroll
-    for (int d = 0; d < 3; ++d) x[d] = CL == 0 ? s.x0[d] : contract1(clampr(s.ps[d], a.r), a);
-}
-
-// Lane p + D (p - 1) of the lane's 16-lane row (a DPP row shift: no LDS
-// traffic); lanes whose source lies outside the row get 0 and must not use it.
-template <int D>
-__device__ __forceinline__ uint32_t row_down(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x100 + D, 0xf, 0xf, false);
-}
-__device__ __forceinline__ uint32_t row_up1(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);
-}
-
-// One step of the suffix segmented sum over a 16-lane row: a lane that is
-// not the end of its segment adds the accumulators of lane p + D (and takes
-// over its end flag) when that lane is in the row.
-template <int D>
-__device__ __forceinline__ void merge_step(int p, float acc[16], bool& end) {
-    float o[16];
-#pragma unroll
-    for (int c = 0; c < 16; ++c)
-        o[c] = __int_as_float(
-            __builtin_amdgcn_update_dpp(0, __float_as_int(acc[c]), 0x100 + D, 0xf, 0xf, false));
-    const bool oend = row_down<D>((uint32_t)end) != 0u;
-    if (!end && p + D < 16) {
-#pragma unroll
-        for (int c = 0; c < 16; ++c) acc[c] += o[c];
-        end = oend;
-    }
-}
-
-// Reduces the stored encode gradients of one cluster of evaluations at level
-// slot j into (row, value) pairs with a star-stencil merge.  B = the cell of
-// the cluster centre; an evaluation whose cell C
-//   * is B adds its 8 corner values into B's accumulators,
-//   * is B +- e_axis (a face neighbour, the usual case of an offset of about
-//     one cell) adds its 4 corners on the shared face into B's accumulators
-//     and emits its 4 far corners,
-//   * is anything else emits its 8 corners.
-// B's accumulators are then merged with equal-B lanes of the same lane group
-// (neighbouring samples of a ray) by a segmented sum in a fixed shuffle
-// tree, and the segment head emits them.  Every sum has a fixed order.
-// genc_base: LDS [eval][LJ][2][64] of this wave; the cluster's q-th
-// evaluation is genc slot slot0 + q.  COUNT: positions only (no gradients);
-// the cursor advances by the lane group's pairs.
-template <int LJ, int CL, bool COUNT, class VT>
-__device__ __forceinline__ void flush_cluster(const GeoArgs& a, const LevelParams& lp, bool on,
-                                              const GeoSample& s, const float* genc_base, int j,
-                                              int n_q, int slot0, EmitTile<VT>& et) {
-    const int l = lane_id(), p = l & 15;
-    {
-        uint32_t B[3];
-        {
-            float xc[3];
-            cluster_center<CL>(a, s, xc);
-            const LevelPos pb = level_pos(lp, xc);
-#pragma unroll
-            for (int d = 0; d < 3; ++d) B[d] = pb.c[d];
-        }
-        bool touched = false;
-        float acc[16];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) acc[q] = 0.0f;
-        // encode gradients one evaluation ahead: each load pair is issued
-        // before the previous evaluation's pair stores, so its latency
-        // overlaps that evaluation's work instead of stalling every one
-        // (carrying it across level slots too measured no better: more
-        // registers)
-        float g0n = 0.0f, g1n = 0.0f;
-        if constexpr (!COUNT) {
-            g0n = genc_base[(slot0 * LJ + j) * 128 + l];
-            g1n = genc_base[(slot0 * LJ + j) * 128 + 64 + l];
-        }
-#pragma unroll 1
-        for (int q = 0; q < n_q; ++q) {
-            const float g0 = g0n, g1 = g1n;
-            if constexpr (!COUNT) {
-                if (q + 1 < n_q) {
-                    g0n = genc_base[((slot0 + q + 1) * LJ + j) * 128 + l];
-                    g1n = genc_base[((slot0 + q + 1) * LJ + j) * 128 + 64 + l];
-                }
-            }
-            float x[3];
-            cluster_point<CL>(a, s, q, x);
-            const LevelPos pp = level_pos(lp, x);
-            // classify C - B
-            int ax = -1, sgn = 0, nz = 0;
-            bool unit = true;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const int dd = (int)(pp.c[d] - B[d]);
-                if (dd != 0) {
-                    ++nz;
-                    ax = d;
-                    sgn = dd;
-                    unit = unit && (dd == 1 || dd == -1);
-                }
-            }
-            const bool same = nz == 0;
-            const bool adj = nz == 1 && unit;
-            const int axm = ax < 0 ? 0 : ax;
-            const int far_bit = sgn > 0 ? 1 : 0;  // C's corners off B's face
-            touched = touched || same || adj;
-            // all 8 corners of C on their own
-            {
-                const bool em = on && !same && !adj;
-                uint32_t rows[8];
-                float v[16];
-                if (!COUNT && em) corner_rows(lp, pp.c, rows);
-                if (!COUNT && em) {
-#pragma unroll
-                    for (int c = 0; c < 8; ++c) {
-                        const float w = corner_weight(pp, c);
-                        v[2 * c] = w * g0;
-                        v[2 * c + 1] = w * g1;
-                    }
-                }
-                emit_pairs<8, COUNT, VT>(et, em, rows, v);
-            }
-            // the 4 far corners of a face neighbour
-            {
-                const bool em = on && adj;
-                uint32_t rows[4];
-                float v[8];
-                if (!COUNT && em) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int c = face_corner(i, axm, far_bit);
-                        rows[i] = lp.offset + grid_row(lp, pp.c[0] + (c & 1),
-                                                       pp.c[1] + ((c >> 1) & 1),
-                                                       pp.c[2] + ((c >> 2) & 1));
-                    }
-                }
-                if (!COUNT && em) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int c = face_corner(i, axm, far_bit);
-                        const float w = corner_weight(pp, c);
-                        v[2 * i] = w * g0;
-                        v[2 * i + 1] = w * g1;
-                    }
-                }
-                emit_pairs<4, COUNT, VT>(et, em, rows, v);
-            }
-            // into B: corner t of B is corner t of C (same) or corner
-            // t ^ (1 << ax) of C when t lies on the shared face (adj)
-            if constexpr (!COUNT) {
-#pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const bool take = same || (adj && ((t >> axm) & 1) == far_bit);
-                    const int c = same ? t : (t ^ (1 << axm));
-                    const float w = corner_weight(pp, c);
-                    if (take) {
-                        acc[2 * t] = __fmaf_rn(w, g0, acc[2 * t]);
-                        acc[2 * t + 1] = __fmaf_rn(w, g1, acc[2 * t + 1]);
-                    }
-                }
-                // analytic mode, base evaluation (always in B): the gradient
-                // term u * scale * grad(w_c) . g_x of each corner
-                if (CL == 0 && a.analytic && q == 0) {
-                    float ex[3][2];
-#pragma unroll
-                    for (int d = 0; d < 3; ++d)
-#pragma unroll
-                        for (int f = 0; f < 2; ++f)
-                            ex[d][f] = genc_base[((a.n_evals + d) * LJ + j) * 128 + f * 64 + l];
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-#pragma unroll
-                        for (int f = 0; f < 2; ++f) {
-                            const float dv = (corner_dweight(pp, t, 0) * ex[0][f] +
-                                              corner_dweight(pp, t, 1) * ex[1][f]) +
-                                             corner_dweight(pp, t, 2) * ex[2][f];
-                            acc[2 * t + f] += dv;
-                        }
-                    }
-                }
-            }
-        }
-        // B: merge equal cells of neighbouring lanes (same lane group),
-        // suffix segmented sum in a fixed tree, segment head emits.
-        const uint32_t INV = 0xFFFFFFFFu;
-        const bool live = on && touched;
-        const uint32_t key0 = live ? B[0] : INV, key1 = live ? B[1] : INV,
-                       key2 = live ? B[2] : INV;
-        const uint32_t n0 = row_down<1>(key0), n1 = row_down<1>(key1), n2 = row_down<1>(key2);
-        bool end = (p == 15) || !(n0 == key0 && n1 == key1 && n2 == key2) || key0 == INV;
-        if constexpr (!COUNT) {
-            merge_step<1>(p, acc, end);
-            merge_step<2>(p, acc, end);
-            merge_step<4>(p, acc, end);
-            merge_step<8>(p, acc, end);
-        }
-        const uint32_t u0 = row_up1(key0), u1 = row_up1(key1), u2 = row_up1(key2);
-        const bool head = live && (p == 0 || !(u0 == key0 && u1 == key1 && u2 == key2));
-        uint32_t rows[8];
-        if (!COUNT && head) corner_rows(lp, B, rows);
-        emit_pairs<8, COUNT, VT>(et, head, rows, acc);
-    }
-}
-
-// Rebuilds the per-sample state (grad, normal, tangent, curvature terms) of
-// the lane's sample from the 12 stored values (6 FD values, or the analytic
-// grad in the first 3, then the 6 curvature values).  n: the kernels' index
-// (stored values), m: the caller's index (positions, directions).
-__device__ __forceinline__ void geo_rebuild(const GeoArgs& a, const float* __restrict__ pts,
-                                            const float* __restrict__ randn,
-                                            const float* __restrict__ fdv, int64_t n, int64_t m,
-                                            bool valid, GeoSample& s) {
-#pragma unroll
-    for (int d = 0; d < 3; ++d) s.P[d] = valid ? pts[3 * m + d] : 0.0f;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) s.x0[d] = contract1(s.P[d], a);
-    if (a.with_grad) {
-        float g[3] = {0.0f, 0.0f, 0.0f};
-        if (a.analytic) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d) g[d] = valid ? fdv[n * 12 + d] : 0.0f;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 6; ++j) diff_pair(g, j, valid ? fdv[n * 12 + j] : 0.0f);
-            finish_grad(a, g);
-        }
-#pragma unroll
-        for (int d = 0; d < 3; ++d) s.grad[d] = g[d];
-        normalize3(s.grad, s.n);
-    }
-    if (a.with_laplace) {
-        geo_tangent(a, randn, m, valid, s);
-        float gs[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int j = 0; j < 6; ++j) diff_pair(gs, j, valid ? fdv[n * 12 + 6 + j] : 0.0f);
-        finish_grad(a, gs);
-#pragma unroll
-        for (int d = 0; d < 3; ++d) s.grad_s[d] = gs[d];
-        normalize3(s.grad_s, s.ns);
-        s.dot = (s.n[0] * s.ns[0] + s.n[1] * s.ns[1]) + s.n[2] * s.ns[2];
-    }
-}
-
-// Encode-gradient slots of a tile in HBM (written by the backward, read by
-// the pair pass): slot 0 base, 1-6 FD, 7-12 curvature; a slot is [LJ][2][64]
-// floats (level slot, feature, lane).
-__host__ __device__ inline int64_t geo_genc_floats(int64_t tiles, int n_evals, int LJ) {
-    return tiles * n_evals * LJ * 128;
-}
-
-// Pair pass.  COUNT: the number of (row, value) pairs each tile of 16
-// samples emits at each level, from positions alone (counts[level * tiles +
-// tile]).  Otherwise: the same decisions with the encode gradients, the pairs
-// written from offsets[level * tiles + tile] on (one stream per level, never
-// past the tile's count; a different count sets status[1]).
-template <int LJ, bool COUNT, class VT>
-__global__ void __launch_bounds__(256) k_geo_pairs(
-    GeoArgs a, const float* __restrict__ pts, const float* __restrict__ randn, int64_t N,
-    const float* __restrict__ fdv, const float* __restrict__ genc, uint32_t* __restrict__ keys,
-    VT* __restrict__ vals, const int64_t* __restrict__ offsets, int64_t* __restrict__ counts,
-    int64_t* __restrict__ status, int64_t capacity) {
-    __shared__ LevelParams lv[AM_MAX_LEVELS];
-#pragma unroll
-    for (int q = 0; q < AM_MAX_LEVELS; ++q)
-        if ((int)threadIdx.x == q && q < a.g.L) lv[q] = a.g.lv[q];
-    __syncthreads();
-    const int l = lane_id(), p = l & 15, k = l >> 4;
-    const int nw = blockDim.x >> 6, wave = threadIdx.x >> 6;
-    const int64_t n_tiles = (N + 15) / 16;
-    for (int64_t tile = (int64_t)blockIdx.x * nw + wave; tile < n_tiles;
-         tile += (int64_t)gridDim.x * nw) {
-        const int64_t n = tile * 16 + p;
-        const bool valid = n < N;
-        GeoSample s;
-        geo_rebuild(a, pts, randn, fdv, n, caller_row(a, n, valid), valid, s);
-        const float* gt = COUNT ? nullptr : genc + tile * a.genc_slots * LJ * 128;
-#pragma unroll 1
-        for (int j = 0; j < LJ; ++j) {
-            const int level = k + 4 * j;
-            const bool there = level < a.g.L;
-            const bool on = valid && level < a.active;
-            const int64_t entry = level * n_tiles + tile;
-            LevelParams lp{};
-            if (there) lp = lv[level];
-            EmitTile<VT> et{nullptr, nullptr, 0, 0};
-            if constexpr (kAtomicPairs<VT>) {
-                et.vals = vals;
-            } else if constexpr (!COUNT) {
-                if (there) {
-                    const int64_t off = offsets[entry];
-                    const int64_t room = capacity - off;
-                    int64_t lim = counts[entry];
-                    if (lim > room) {   // cut at the arrays' capacity, flagged
-                        lim = room > 0 ? room : 0;
-                        if (p == 0) status[1] = 1;
-                    }
-                    et = EmitTile<VT>{keys + off, vals + off, 0, (int)lim};
-                }
-            }
-            if (a.with_laplace)
-                flush_cluster<LJ, 1, COUNT>(a, lp, on, s, gt, j, 6, a.curv0, et);
-            flush_cluster<LJ, 0, COUNT>(a, lp, on, s, gt, j, a.with_grad && !a.analytic ? 7 : 1, 0,
-                                        et);
-            if constexpr (COUNT) {
-                if (there && p == 0) counts[entry] = et.cursor;
-            } else if constexpr (!kAtomicPairs<VT>) {
-                if (there && p == 0 && et.cursor != et.limit) status[1] = 1;
-            }
+            gext[d * LJ * 512 + j * 512] = ub[2 * j] * sc * gx[d];
+            gext[d * LJ * 512 + j * 512 + 64] = ub[2 * j + 1] * sc * gx[d];
         }
     }
 }
@@ -1345,7 +779,7 @@ __device__ __forceinline__ void geo_bwd_body(
         const int64_t m = caller_row(a, n, valid);
         // this tile's encode-gradient slots (0 base, then FD and curvature, or
         // curvature and the three analytic extra slots)
-        float* genc = genc_g + tile * a.genc_slots * LJ * 128;
+        float* genc = genc_g + genc_lane(a, tile, LJ, l);
         GeoSample s;
         geo_rebuild(a, pts, randn, fdv, n, m, valid, s);
         // upstream gradients of this sample
@@ -1403,7 +837,7 @@ __device__ __forceinline__ void geo_bwd_body(
                                                         a.curv0 + j, a.dx_curv0 + j, x, e);
                 float gpos[3];
                 geo_eval_bwd<LJ, NH, true, mlp::kF32>(a, sm, e, go_row0(gf), scratch, G,
-                                                      genc + (a.curv0 + j) * LJ * 128, gpos);
+                                                      genc + (a.curv0 + j) * LJ * 512, gpos);
 #pragma unroll
                 for (int d = 0; d < 3; ++d)
                     if (inb[d]) g_ps[d] += gpos[d] * a.inv2r;
@@ -1428,7 +862,7 @@ __device__ __forceinline__ void geo_bwd_body(
                                                     s.x0, e);
             const OutExt ext{g_feature, m, fdim, valid, ext_acc};
             geo_eval_bwd_an<LJ, NH>(a, sm, lv, e, go, gx, scratch, G, genc,
-                                    genc + a.n_evals * LJ * 128, a.out_tiles > 1 ? &ext : nullptr);
+                                    genc + a.n_evals * LJ * 512, a.out_tiles > 1 ? &ext : nullptr);
         } else if (a.with_grad) {
             float gn2g[3];
             normalize3_bwd(s.grad, gnrm, gn2g);
@@ -1444,7 +878,7 @@ __device__ __forceinline__ void geo_bwd_body(
                 geo_eval_b<LJ, NH, false, ST, mlp::kF32>(a, sm, lv, table, store, tile, n_tiles,
                                                          1 + j, 0, x, e);
                 geo_eval_bwd<LJ, NH, false, mlp::kF32>(a, sm, e, go_row0(gf), scratch, G,
-                                                       genc + (1 + j) * LJ * 128, nullptr);
+                                                       genc + (1 + j) * LJ * 512, nullptr);
             }
         }
     }
@@ -1543,38 +977,6 @@ template <int LJ, bool ST, int PR, bool AN>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_geo_bwd_o2(AM_GEO_BWD_PARAMS) {
     geo_bwd_body<LJ, 1, ST, PR, AN>(AM_GEO_BWD_ARGS);
-}
-
-// Sentinel keys and zero values in [status[0], bound): the unused tail of
-// pair arrays carved for the worst-case bound (sorted form).
-template <class VT>
-__global__ void k_pair_tail(uint32_t* __restrict__ keys, VT* __restrict__ vals,
-                            const int64_t* __restrict__ status, int64_t bound, uint32_t sentinel) {
-    const int64_t first = status[0];
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = first + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < bound;
-         i += stride) {
-        keys[i] = sentinel;
-        VT v;
-        set_pair(v, 0.0f, 0.0f);
-        vals[i] = v;
-    }
-}
-
-// status[0] = number of pairs; status[1] = 0, set by the emit pass on a
-// count mismatch; level_start = the level streams' bounds.
-__global__ void k_pair_streams(const int64_t* __restrict__ offsets,
-                               const int64_t* __restrict__ counts, int64_t tiles, int L,
-                               int64_t* __restrict__ status, int64_t* __restrict__ level_start) {
-    const int l = threadIdx.x;
-    if (l < L) level_start[l] = offsets[l * tiles];
-    if (l == L) {
-        const int64_t last = L * tiles - 1;
-        const int64_t n = offsets[last] + counts[last];
-        level_start[L] = n;
-        status[0] = n;
-        status[1] = 0;
-    }
 }
 
 // ------------------------------------------------------------------------
@@ -1689,17 +1091,6 @@ static int geo_fwd_launch(const GeoArgs& a, const float* pts, const float* randn
                                                       normal, feature, laplace, fdv, nullptr, s);
 }
 
-template <int LJ>
-static int geo_count_launch(const GeoArgs& a, const float* pts, const float* randn, int64_t n,
-                            const float* fdv, int64_t* counts, hipStream_t s) {
-    KernelTimer kt_("pair_count", s);
-    hipLaunchKernelGGL((k_geo_pairs<LJ, true, Vals<2>>), dim3(count_blocks(n)), dim3(256), 0, s, a,
-                       pts, randn, n, fdv, nullptr, nullptr, nullptr, nullptr, counts, nullptr,
-                       (int64_t)0);
-    AM_LAUNCH_CHECK();
-    return AM_OK;
-}
-
 // The backward's workspace before the pair arrays: the pair count is only
 // known after the count pass, so the sort buffers are carved afterwards
 // from the rest (sized for the worst case by the size query).
@@ -1709,47 +1100,28 @@ struct GeoBwdWs {
     float* genc;
     float* partial;
     float* ctmp;
-    int64_t* counts;
-    int64_t* offsets;
-    int64_t entries;   // count / offset entries: levels x tiles
-    int64_t* status;
-    int64_t* level_start;
-    void* scan_tmp;
-    size_t scan_bytes;
+    PairHead pairs;
 };
 
-static void carve_geo_bwd_head(WsCarver& c, const GeoArgs& a, int LJ, int64_t n, bool need_fdv,
-                               GeoBwdWs* w) {
+static void carve_geo_bwd_head(WsCarver& c, const GeoArgs& a, const am_grid_desc* g, int LJ,
+                               int64_t n, bool need_fdv, GeoBwdWs* w) {
     const int waves = bwd_blocks(n) * 4;
     const int64_t tiles = (n + 15) / 16;
-    const int64_t entries = tiles * a.g.L;
     w->fdv = need_fdv ? c.take<float>((size_t)n * 12 + 1) : nullptr;
     w->sdf_tmp = need_fdv ? c.take<float>((size_t)n + 1) : nullptr;
     w->genc = c.take<float>((size_t)geo_genc_floats(tiles, a.genc_slots, LJ) + 1);
     w->partial = c.take<float>((size_t)waves * a.n_params);
     w->ctmp = c.take<float>((size_t)colsum_tmp_floats(waves, a.n_params) + 1);
-    w->counts = c.take<int64_t>((size_t)entries + 1);
-    w->offsets = c.take<int64_t>((size_t)entries + 1);
-    w->entries = entries;
-    w->status = c.take<int64_t>(2);
-    w->level_start = c.take<int64_t>(AM_MAX_LEVELS + 1);
-    size_t sb = 0;
-    rocprim::exclusive_scan(nullptr, sb, (const int64_t*)nullptr, (int64_t*)nullptr, (int64_t)0,
-                            (size_t)(entries > 0 ? entries : 1), rocprim::plus<int64_t>(), 0,
-                            false);
-    w->scan_bytes = sb;
-    w->scan_tmp = c.take<char>(sb + 256);
+    pairs_carve(c, a, g, n, &w->pairs);
 }
 
-// Most pairs a tile can emit, per lane and level slot.  FD cluster: the
-// base point is always in B, so 6 x 8 + 8 for B = 56; analytic or without
-// gradient: the base alone, 8.  Curvature cluster (its centre is not
-// evaluated): 6 x 8 = 48 with B untouched; with one point in a face
-// neighbour of B, 5 x 8 + 4 far corners + 8 for B = 52 (the most); more
-// points in or beside B emit less.
-static int64_t geo_max_pairs(const GeoArgs& a, int LJ, int64_t n) {
-    const int64_t per_slot = (a.with_grad && !a.analytic ? 56 : 8) + (a.with_laplace ? 52 : 0);
-    return (n + 15) / 16 * (per_slot * LJ * 64);
+// The pair arrays for a count pass's capacity (pages, or pairs).
+static int carve_pairs(WsCarver& c, const GeoArgs& a, const am_grid_desc* g, const PairHead& h,
+                       int64_t capacity, TablePages* tp, TableReduceWs* tw) {
+    const bool half = a.prec == AM_PREC_MIXED;
+    if (!h.paged) return table_reduce_carve(c, g, capacity, tw, half);
+    table_pages_carve(c, capacity, half, tp);
+    return AM_OK;
 }
 
 // Consistency flags of recent backward calls.  The emit pass flags a tile
@@ -1830,7 +1202,7 @@ static int geo_bwd_launch_t(const GeoArgs& a, const am_grid_desc* g, const float
     AM_CHECK_ARG(!store || !need_fdv, "a stored encoding needs the stored FD values too");
     WsCarver c(ws, ws_bytes);
     GeoBwdWs w;
-    carve_geo_bwd_head(c, a, LJ, n, need_fdv, &w);
+    carve_geo_bwd_head(c, a, g, LJ, n, need_fdv, &w);
     if (!c.ok()) return workspace_short(c.used, ws_bytes);
     const float* fdv = fdv_in;
     if (need_fdv) {  // recompute the stored SDF values with a forward pass
@@ -1869,68 +1241,36 @@ static int geo_bwd_launch_t(const GeoArgs& a, const am_grid_desc* g, const float
         // atomic form: the pairs are added into the zeroed table gradient
         if (int rc = fill_f32(dtable, (int64_t)g->n_entries * 2, 0.0f, s)) return rc;
         if (int rc = launch_bwd()) return rc;
-        {
-            KernelTimer kt_("pair_atomic", s);
-            hipLaunchKernelGGL((k_geo_pairs<LJ, false, AtomicRow>), dim3(pair_blocks(n)),
-                               dim3(256), 0, s, a, pts, randn, n, fdv, w.genc, nullptr,
-                               reinterpret_cast<AtomicRow*>(dtable), nullptr, nullptr, nullptr,
-                               (int64_t)0);
-        }
-        AM_LAUNCH_CHECK();
+        if (int rc = pairs_atomic(a, LJ, pts, randn, n, fdv, w.genc, dtable, s)) return rc;
         return colsum_f32(w.partial, waves, a.n_params, dparams, w.ctmp, s);
     }
-    // 1. pairs per level and tile, 2. exclusive prefix sum -> each one's first pair
-    if (int rc = geo_count_launch<LJ>(a, pts, randn, n, fdv, w.counts, s)) return rc;
-    size_t sb = w.scan_bytes;
-    hipError_t e = rocprim::exclusive_scan(w.scan_tmp, sb, w.counts, w.offsets, (int64_t)0,
-                                           (size_t)w.entries, rocprim::plus<int64_t>(), s, false);
-    if (e != hipSuccess) {
-        set_error("tile-count scan failed: %s", hipGetErrorString(e));
-        return AM_ERR_HIP;
-    }
-    hipLaunchKernelGGL(k_pair_streams, dim3(1), dim3(64), 0, s, w.offsets, w.counts, tiles, a.g.L,
-                       w.status, w.level_start);
-    AM_LAUNCH_CHECK();
+    // 1. the pairs each part of the emission makes, 2. their prefix sums
+    if (int rc = pairs_count(a, LJ, pts, randn, n, fdv, w.pairs, s)) return rc;
     // 3. the pair arrays.  Sync-free form (flag "sdf_bwd_sync_free"): arrays
     // of the worst-case pair bound, no host read (the reduction reads the
     // streams' bounds on the device).  Otherwise one host read of the pair
     // count carves the arrays for exactly that many pairs.  A workspace too
     // small is rejected here, before any output is written, with
     // am_last_workspace_need() = what this call needs.
-    const int64_t max_pairs = geo_max_pairs(a, LJ, n);
     const bool bounded = flag_value("sdf_bwd_sync_free", 0) != 0;
-    int64_t st[2] = {0, 0};
+    int64_t st[3] = {pairs_bound(a, w.pairs, LJ, n), 0, 0};
     if (!bounded) {
-        AM_HIP(hipMemcpyAsync(st, w.status, sizeof(st), hipMemcpyDeviceToHost, s));
+        AM_HIP(hipMemcpyAsync(st, w.pairs.status, sizeof(st), hipMemcpyDeviceToHost, s));
         AM_HIP(hipStreamSynchronize(s));
         timer_units("host_syncs", 1);
     }
     if (int rc = collect_flags(false)) return rc;
+    TablePages tp;
     TableReduceWs tw;
-    const int64_t capacity = bounded ? max_pairs : st[0];
-    if (int rc = table_reduce_carve(c, g, capacity, &tw, PR == mlp::kBF16)) return rc;
+    if (int rc = carve_pairs(c, a, g, w.pairs, st[0], &tp, &tw)) return rc;
     if (!c.ok()) return workspace_short(c.used, ws_bytes);
-    if (tw.paged) tw.level_start = w.level_start;
-    if (bounded && !tw.paged && max_pairs > 0) {   // the sorted form's unused tail
-        const int64_t want = ceil_div(max_pairs, 256);
-        hipLaunchKernelGGL((k_pair_tail<PairV<PR>>), dim3((unsigned)(want < 16384 ? want : 16384)),
-                           dim3(256), 0, s, tw.keys[0], reinterpret_cast<PairV<PR>*>(tw.vals[0]),
-                           w.status, max_pairs, table_sentinel(tw.end_bit));
-        AM_LAUNCH_CHECK();
-    }
     if (int rc = launch_bwd()) return rc;
-    {
-        KernelTimer kt_("pair_emit", s);
-        hipLaunchKernelGGL((k_geo_pairs<LJ, false, PairV<PR>>), dim3(pair_blocks(n)), dim3(256), 0,
-                           s, a, pts, randn, n, fdv, w.genc, tw.keys[0],
-                           reinterpret_cast<PairV<PR>*>(tw.vals[0]), w.offsets, w.counts, w.status,
-                           capacity);
-    }
-    AM_LAUNCH_CHECK();
     if (int rc = colsum_f32(w.partial, waves, a.n_params, dparams, w.ctmp, s)) return rc;
-    if (!bounded) timer_units("table_pairs", capacity);
-    if (int rc = table_reduce_run(tw, g, dtable, s)) return rc;
-    return arm_flag(w.status + 1, s);
+    if (!bounded) timer_units("table_pairs", st[2]);
+    if (int rc = pairs_reduce(a, LJ, g, pts, randn, n, fdv, w.genc, w.pairs, tp, tw, bounded, dtable,
+                              s))
+        return rc;
+    return arm_flag(w.pairs.status + 1, s);
 }
 
 template <int LJ, int NH>
@@ -2016,9 +1356,10 @@ extern "C" size_t am_sdf_bwd_workspace_size(const am_grid_desc* g, const am_mlp_
     if (make_geo_args(g, m, sd, &a, &LJ) || n < 0) return 0;
     WsCarver c(nullptr, 0);
     GeoBwdWs w;
-    carve_geo_bwd_head(c, a, LJ, n, true, &w);
+    carve_geo_bwd_head(c, a, g, LJ, n, true, &w);
+    TablePages tp;
     TableReduceWs tw;
-    if (table_reduce_carve(c, g, geo_max_pairs(a, LJ, n), &tw)) return 0;
+    if (carve_pairs(c, a, g, w.pairs, pairs_bound(a, w.pairs, LJ, n), &tp, &tw)) return 0;
     return c.used + 256;
 }
 

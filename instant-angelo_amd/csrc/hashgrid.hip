@@ -3,7 +3,7 @@
 // models/network_utils.py:40-66,83-93).
 #include <cmath>
 #include "hashgrid_dev.h"
-#include "table_grad.h"
+#include "page_dev.h"
 
 namespace am {
 
@@ -173,10 +173,67 @@ static int hg_fwd(const GridArgs& ga, const float* x, int64_t n, const float* ta
     return AM_OK;
 }
 
-// First pair of each level's stream of k_hg_emit.
-__global__ void k_hg_streams(int L, int active, int64_t per_level, int64_t* __restrict__ start) {
-    const int l = threadIdx.x;
-    if (l <= L) start[l] = per_level * (l < active ? l : active);
+// Paged form (two features): one block per page, kPage / 8 points at one
+// level, their eight pairs each put into the LDS page and written partitioned
+// by bucket (page_flush).
+constexpr int kPagePoints = kPage / 8;
+
+__global__ void __launch_bounds__(kPageThreads) k_hg_pages(
+    GridArgs g, const float* __restrict__ x, int64_t n, int64_t per_level,
+    const float* __restrict__ dy, const int32_t* __restrict__ order, uint32_t* __restrict__ keys,
+    uint2* __restrict__ vals, uint16_t* __restrict__ run_start) {
+    extern __shared__ char smem[];
+    __shared__ LevelParams lvs;
+    PageLds<uint2>& pg = *reinterpret_cast<PageLds<uint2>*>(smem);
+    const int tid = (int)threadIdx.x;
+    const int l = (int)(blockIdx.x / per_level);
+    const int64_t first = (int64_t)(blockIdx.x % per_level) * kPagePoints;
+    if (tid <= kMaxDigits) pg.hist[tid] = 0u;
+#pragma unroll
+    for (int q = 0; q < AM_MAX_LEVELS; ++q)
+        if (q == l && tid == 0) lvs = g.lv[q];
+    __syncthreads();
+    LevelParams lp = lvs;
+    lp.offset = 0u;   // rows within the level
+    const int np = n - first < kPagePoints ? (int)(n - first) : kPagePoints;
+    for (int q = tid; q < np; q += kPageThreads) {
+        const int64_t i = order ? (int64_t)order[first + q] : first + q;   // the caller's row
+        const float xi[3] = {x[3 * i], x[3 * i + 1], x[3 * i + 2]};
+        const LevelPos p = level_pos(lp, xi);
+        uint32_t rows[8];
+        cell_rows(lp, p.c, rows);
+        const float g0 = dy[(i * g.L + l) * 2], g1 = dy[(i * g.L + l) * 2 + 1];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const float w = corner_weight(p, c);
+            pg.keys[c * np + q] = rows[c];
+            put_pair(pg.vals[c * np + q], w * g0, w * g1);
+        }
+    }
+    page_flush(pg, 8 * np, blockIdx.x, keys, vals, run_start);
+}
+
+static int hg_bwd_pages(const GridArgs& ga, const am_grid_desc* g, const float* x, int64_t n,
+                        const float* dy, int active, float* dtable, void* ws, size_t ws_bytes,
+                        const int32_t* order, hipStream_t s) {
+    const int64_t per_level = ceil_div(n, kPagePoints);
+    WsCarver c(ws, ws_bytes);
+    TablePages w;
+    table_pages_carve(c, per_level * active, false, &w);
+    if (!c.ok()) return workspace_short(c.used, ws_bytes);
+    const size_t lds = sizeof(PageLds<uint2>);
+    AM_HIP(hipFuncSetAttribute((const void*)k_hg_pages, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds));
+    {
+        KernelTimer kt_("hg_emit", s);
+        hipLaunchKernelGGL(k_hg_pages, dim3((unsigned)w.pages), dim3(kPageThreads), lds, s, ga, x, n,
+                           per_level, dy, order, w.keys, reinterpret_cast<uint2*>(w.vals),
+                           w.run_start);
+    }
+    AM_LAUNCH_CHECK();
+    timer_units("encode_table_pairs", n * active * 8);
+    if (int rc = table_pages_plan(w, g, nullptr, 0, active, per_level, s)) return rc;
+    return table_pages_run(w, g, dtable, s);
 }
 
 template <int F>
@@ -191,6 +248,8 @@ static int hg_bwd(const GridArgs& ga, const am_grid_desc* g, const float* x, int
     if (dtable) {
         const int64_t m = n * active * 8;
         if (m == 0) return fill_f32(dtable, (int64_t)g->n_entries * F, 0.0f, s);
+        if (table_paged(g))
+            return hg_bwd_pages(ga, g, x, n, dy, active, dtable, ws, ws_bytes, order, s);
         WsCarver c(ws, ws_bytes);
         TableReduceWs w;
         int rc = table_reduce_carve(c, g, m, &w);
@@ -204,11 +263,6 @@ static int hg_bwd(const GridArgs& ga, const am_grid_desc* g, const float* x, int
         }
         AM_LAUNCH_CHECK();
         timer_units("encode_table_pairs", w.m);
-        if (w.paged) {
-            hipLaunchKernelGGL(k_hg_streams, dim3(1), dim3(64), 0, s, ga.L, active, n * 8,
-                               w.level_start);
-            AM_LAUNCH_CHECK();
-        }
         return table_reduce_run(w, g, dtable, s);
     }
     return AM_OK;
@@ -304,6 +358,11 @@ extern "C" size_t am_hashgrid_bwd_workspace_size(const am_grid_desc* g, int64_t 
                                                  int32_t active_levels) {
     if (check_grid(g) || n < 0 || active_levels < 0 || active_levels > g->n_levels) return 0;
     WsCarver c(nullptr, 0);
+    if (table_paged(g)) {
+        TablePages w;
+        table_pages_carve(c, ceil_div(n, kPagePoints) * active_levels, false, &w);
+        return c.used + 256;
+    }
     TableReduceWs w;
     if (table_reduce_carve(c, g, n * active_levels * 8, &w)) return 0;
     return c.used + 256;

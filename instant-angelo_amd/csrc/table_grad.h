@@ -3,12 +3,12 @@
 // pair written 0, the same bits on every run.
 //
 // Paged form (two features a row, at most 2^21 rows a level: every grid of
-// the workloads).  The emitters write one stream of pairs per level.  A
-// stream is cut into pages of kPage pairs; each page is partitioned in place
-// (in LDS) by its pairs' bucket of 2^13 rows, with a table of where each
-// bucket's run starts, and one block per bucket then gathers its runs from
-// the level's pages and adds them up in LDS.  The additions are exact (see
-// k_page_reduce), so their order does not matter.
+// the workloads).  The emitting kernels collect the pairs of one level in
+// LDS, a page at a time, and write each page partitioned by its pairs' bucket
+// of 2^13 rows, with a table of where each bucket's run starts; one block per
+// bucket then gathers its runs from the level's pages and adds them up in
+// LDS.  The additions are exact (see k_page_reduce), so their order does not
+// matter.  Every pair is written once and its value read once.
 //
 // Sorted form (other feature counts, larger levels): stable radix sort of the
 // pairs by row, then a fixed-order segmented reduce.  Two-feature tables sort
@@ -17,8 +17,8 @@
 // per bucket finishes the job with an in-wave stable split sort and a
 // segmented scan into per-row accumulators in LDS.
 //
-// The emitters write pairs into carve.keys[0] / carve.vals[0] (keys: table
-// rows).
+// There the emitters write pairs into keys[0] / vals[0].  Keys equal to the
+// sentinel mark empty slots; they sort last and are skipped.
 #pragma once
 #include <hip/hip_fp16.h>
 #include "am_common.h"
@@ -59,11 +59,6 @@ struct TableReduceWs {
     int begin_bit;          // key bits sorted: [begin_bit, end_bit)
     int end_bit;
     bool half_vals;  // values are ValsH<F> instead of Vals<F>
-    bool paged;      // paged form: the fields below
-    uint16_t* run_start;    // [pages][kRunStride] first pair of each bucket's run
-    double2* partial2;      // [slots][8192 rows] sums of sliced buckets
-    struct PagePlan* plan;
-    int64_t* level_start;   // [levels + 1] first pair of each level's stream
 };
 
 // Rows of the levels: level l owns [offset[l], offset[l + 1]).
@@ -73,10 +68,9 @@ struct TableLevels {
 };
 TableLevels table_levels(const am_grid_desc* g);
 
-// What the paged kernels read of the streams (made on the device from
-// level_start, so that no host read is needed).
+// What the reduction reads of the pages (made on the device, so that no host
+// read is needed).
 struct PagePlan {
-    int64_t level_start[AM_MAX_LEVELS + 1];
     int32_t page_base[AM_MAX_LEVELS + 1];   // first page of each level
     int32_t unit_base[AM_MAX_LEVELS + 1];   // first work unit of each level (finest level first)
     int32_t slices[AM_MAX_LEVELS];          // slices of each of the level's buckets
@@ -84,6 +78,29 @@ struct PagePlan {
     int32_t row_base[AM_MAX_LEVELS + 1];    // first combined row of a sliced level
 };
 
+struct TablePages {
+    int64_t pages;       // the arrays' capacity
+    uint32_t* keys;      // [pages][kPage]
+    void* vals;          // the same: float2, or half2 (half_vals)
+    uint16_t* run_start; // [pages][kRunStride]
+    double2* partial;    // [slots][8192 rows] sums of sliced buckets
+    PagePlan* plan;
+    bool half_vals;
+};
+
+// Whether the paged form takes the grid.
+bool table_paged(const am_grid_desc* g);
+void table_pages_carve(WsCarver& c, int64_t pages, bool half_vals, TablePages* out);
+// Where the pages of each level begin: the level's `units` emitting blocks'
+// exclusive scan (high 24 bits: pages), unit = level * units + block, levels
+// from `active` on empty; or (scan == nullptr) `per_level` pages for each of
+// the `active` levels.
+int table_pages_plan(TablePages& w, const am_grid_desc* g, const uint64_t* scan, int64_t units,
+                     int active, int64_t per_level, hipStream_t s);
+// Reduces the pages; dtable [n_entries, 2] fully overwritten.
+int table_pages_run(TablePages& w, const am_grid_desc* g, float* dtable, hipStream_t s);
+
+// ---- sorted form ----
 // Bucket bits of the bucketed form: the low key bits left unsorted (at most
 // 9, so a wave's accumulators span at most 512 rows).
 int table_bucket_bits(int end_bit);
@@ -93,18 +110,16 @@ int table_bucket_bits(int end_bit);
 int table_key_bits(uint32_t n_entries);
 static inline uint32_t table_sentinel(int end_bit) { return (uint32_t)((1ull << end_bit) - 1ull); }
 
-// Carves the reduction workspace for m pairs out of `c`.  Returns the sort's
-// temp byte count through TableReduceWs (0 when c has no base pointer: size
-// query; the sort size query needs a device).
+// Carves the sorted form's workspace for m pairs out of `c`.  Returns the
+// sort's temp byte count through TableReduceWs (0 when c has no base pointer:
+// size query; the sort size query needs a device).
 int table_reduce_carve(WsCarver& c, const am_grid_desc* g, int64_t m, TableReduceWs* out,
                        bool half_vals = false);
 
 // Writes v to p[0..n) on `stream` (a fill kernel, safe under graph capture).
 int fill_f32(float* p, int64_t n, float v, hipStream_t stream);
 
-// Reduces the pairs; dtable [n_entries, F] fully overwritten.  Paged form:
-// w.level_start holds the level streams' bounds (at most w.m pairs); sorted
-// form: exactly w.m pairs (sentinel keys allowed).
+// Runs sort + segmented reduce; dtable [n_entries, F] fully overwritten.
 int table_reduce_run(TableReduceWs& w, const am_grid_desc* g, float* dtable, hipStream_t stream);
 
 }  // namespace am

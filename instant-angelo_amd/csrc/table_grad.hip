@@ -2,7 +2,7 @@
 // radix sort with a fixed-order segmented reduce (see table_grad.h).
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
-#include "table_grad.h"
+#include "page_dev.h"
 
 namespace am {
 
@@ -13,18 +13,13 @@ constexpr int64_t kUnitItems = 16384;   // sorted items per work unit (256 chunk
 static int64_t bucket_slots(int64_t m) { return 2 * (m / kUnitItems) + 1; }
 
 // ---- paged form ----
-constexpr int kPage = 6144;          // pairs a page (two blocks' LDS a CU)
-constexpr int kRowBits = 13;         // rows a bucket: its sums fill the LDS
-constexpr int kRows = 1 << kRowBits;
-constexpr int kMaxDigits = 256;      // buckets a level: 2^21 rows
-constexpr int kRunStride = kMaxDigits + 2;
 // Pairs of a work unit: a level's buckets are cut into slices of about this
 // many pairs where they hold more (coarse levels), fewer when the whole
 // gradient makes less than about 1024 units of the most.
 constexpr int64_t kUnitMost = 1 << 19;
 constexpr int64_t kUnitLeast = 16384;
 
-static bool table_paged(const am_grid_desc* g) {
+bool table_paged(const am_grid_desc* g) {
     if (g->n_features != 2) return false;
     for (int l = 0; l < g->n_levels; ++l)
         if (g->size[l] > (uint32_t)kMaxDigits * kRows) return false;
@@ -40,8 +35,6 @@ TableLevels table_levels(const am_grid_desc* g) {
     }
     return t;
 }
-
-static int64_t page_bound(int64_t m, int L) { return m / kPage + L; }
 
 // Units of sliced levels: a level of n pairs and D buckets has
 // S = ceil(n / (D U)) slices, D S <= 2 n / U where S > 1.
@@ -120,18 +113,6 @@ int table_reduce_carve(WsCarver& c, const am_grid_desc* g, int64_t m, TableReduc
     w.m = m;
     w.end_bit = table_key_bits(n_entries);
     w.half_vals = half_vals;
-    w.paged = table_paged(g);
-    if (w.paged) {
-        const size_t vb = half_vals ? 4 : 8;
-        w.keys[0] = c.take<uint32_t>((size_t)m + 1);
-        w.vals[0] = c.take<char>((size_t)(m + 1) * vb);
-        w.run_start = c.take<uint16_t>((size_t)page_bound(m, g->n_levels) * kRunStride);
-        w.partial2 = c.take<double2>((size_t)slot_bound(m) << kRowBits);
-        w.plan = c.take<PagePlan>(1);
-        w.level_start = c.take<int64_t>(AM_MAX_LEVELS + 1);
-        *out = w;
-        return AM_OK;
-    }
     const size_t vbytes = (size_t)F * (half_vals ? sizeof(__half) : sizeof(float));
     w.keys[0] = c.take<uint32_t>((size_t)m);
     w.keys[1] = c.take<uint32_t>((size_t)m);
@@ -538,165 +519,47 @@ __device__ __forceinline__ int level_digits(const TableLevels& t, int l) {
     return (int)((t.offset[l + 1] - t.offset[l] + (uint32_t)kRows - 1u) >> kRowBits);
 }
 
-// Inclusive sum over the wave's lanes.
-__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = __shfl_up(v, d, 64);
-        if ((int)(threadIdx.x & 63) >= d) v += o;
-    }
-    return v;
-}
-
-// One wave, lane = level: pages, slices and work units of the streams.
-__global__ void k_page_plan(TableLevels t, const int64_t* __restrict__ level_start,
-                            PagePlan* __restrict__ plan) {
+// One wave, lane = level: page bounds, slices and work units.
+__global__ void k_page_plan(TableLevels t, const uint64_t* __restrict__ scan, int64_t units,
+                            int active, int64_t per_level, PagePlan* __restrict__ plan) {
     const int l = threadIdx.x;
     const bool on = l < t.L;
-    const int64_t s = on ? level_start[l] : 0, e = on ? level_start[l + 1] : 0;
-    const int64_t total = level_start[t.L] - level_start[0];
+    auto first_page = [&](int q) -> int64_t {
+        if (q > active) q = active;
+        return scan ? (int64_t)(scan[q * units] >> 40) : q * per_level;
+    };
+    const int64_t p = on ? first_page(l) : 0, n = on ? (first_page(l + 1) - p) * kPage : 0;
+    const int64_t total = first_page(t.L) * kPage;
     int64_t unit = total / 1024;
     unit = unit < kUnitLeast ? kUnitLeast : (unit > kUnitMost ? kUnitMost : unit);
-    const int64_t n = e - s;
     const int D = on ? level_digits(t, l) : 0;
-    const uint32_t pages = (uint32_t)((n + kPage - 1) / kPage);
     int64_t S = on ? (n + D * unit - 1) / (D * unit) : 0;
     if (on && S < 1) S = 1;
-    const uint32_t units = (uint32_t)(D * S);
-    const uint32_t slots = S > 1 ? units : 0u;
+    const uint32_t all = (uint32_t)(D * S);
+    const uint32_t slots = S > 1 ? all : 0u;
     const uint32_t rows = S > 1 ? t.offset[l + 1] - t.offset[l] : 0u;   // combined afterwards
-    const uint32_t ps = wave_scan(pages), us = wave_scan(units), ss = wave_scan(slots),
-                   rs = wave_scan(rows);
-    const uint32_t all = __shfl(us, 63, 64);
+    const uint32_t us = wave_scan(all), ss = wave_scan(slots), rs = wave_scan(rows);
+    const uint32_t sum = __shfl(us, 63, 64);
     if (on) {
-        plan->level_start[l] = s;
-        plan->page_base[l] = (int32_t)(ps - pages);
+        plan->page_base[l] = (int32_t)p;
         // finest level first: its buckets hold the most pairs
-        plan->unit_base[l] = (int32_t)(all - us);
+        plan->unit_base[l] = (int32_t)(sum - us);
         plan->slices[l] = (int32_t)S;
         plan->slot_base[l] = (int32_t)(ss - slots);
         plan->row_base[l] = (int32_t)(rs - rows);
         if (l == t.L - 1) {
-            plan->level_start[l + 1] = e;
-            plan->page_base[l + 1] = (int32_t)ps;
+            plan->page_base[l + 1] = (int32_t)(p + n / kPage);
             plan->row_base[l + 1] = (int32_t)rs;
         }
-        if (l == 0) plan->unit_base[t.L] = (int32_t)all;
+        if (l == 0) plan->unit_base[t.L] = (int32_t)sum;
     }
 }
 
-__device__ __forceinline__ float2 pair_value(uint2 v) {
-    return make_float2(__uint_as_float(v.x), __uint_as_float(v.y));
-}
-__device__ __forceinline__ float2 pair_value(uint32_t v) {
-    return __half22float2(__builtin_bit_cast(__half2, v));
-}
-
-__device__ __forceinline__ uint32_t pair_word(uint2 v, int w) { return w ? v.y : v.x; }
-__device__ __forceinline__ uint32_t pair_word(uint32_t v, int) { return v; }
-
-// Partitions one page in place by its pairs' bucket (row >> 13 within the
-// level): a bucket's run holds its pairs in any order (the reduce's sums do
-// not depend on it), so each pair's place comes from one LDS counter; in runs
-// of 64 pairs or more, pairs that arrive together (neighbouring samples,
-// often of one row) are set a load apart, so that the reduce's LDS additions
-// seldom meet in one row (runs of 16 equal rows: reduce 0.80 -> 0.34 ms for
-// 60 M pairs).  The key words then hold the row within the bucket (bits 0-12)
-// and the two values' exponents (13-20, 21-28).  Bound by memory: 12 bytes in
-// and 12 out a pair, 0.29 ms for 60 M pairs (5.0 TB/s).  Two blocks of 1024
-// threads share a CU, one loading while the other scatters; pages twice as
-// long give the reduce longer runs (0.34 -> 0.29 ms) but take 0.40 ms here.
-template <class VT>
-__global__ void __launch_bounds__(1024) k_page_partition(TableLevels t,
-                                                         const PagePlan* __restrict__ plan,
-                                                         uint32_t* __restrict__ keys,
-                                                         VT* __restrict__ vals,
-                                                         uint16_t* __restrict__ run_start) {
-    __shared__ VT sv[kPage];
-    __shared__ __attribute__((aligned(16))) uint16_t sk[kPage];
-    __shared__ uint32_t hist[kMaxDigits + 1];
-    __shared__ uint32_t wsum[kMaxDigits / 64];
-    constexpr int kItems = kPage / 1024;
-    const int page = (int)blockIdx.x, tid = (int)threadIdx.x;
-    if (page >= plan->page_base[t.L]) return;
-    int l = 0;
-    while (page >= plan->page_base[l + 1]) ++l;
-    const int64_t first = plan->level_start[l] + (int64_t)(page - plan->page_base[l]) * kPage;
-    const int64_t left = plan->level_start[l + 1] - first;
-    const int n = left < kPage ? (int)left : kPage;
-    const uint32_t off = t.offset[l];
-    uint32_t key[kItems], rank[kItems];
-    VT val[kItems];
-#pragma unroll
-    for (int k = 0; k < kItems; ++k) {
-        const int i = tid + 1024 * k;
-        if (i < n) {
-            key[k] = keys[first + i] - off;
-            val[k] = vals[first + i];
-        }
-    }
-    if (tid < kMaxDigits) hist[tid] = 0u;
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kItems; ++k)
-        if (tid + 1024 * k < n)
-            rank[k] = atomicAdd(&hist[(key[k] >> kRowBits) & (uint32_t)(kMaxDigits - 1)], 1u);
-    __syncthreads();
-    uint32_t c = 0, inc = 0;
-    if (tid < kMaxDigits) {
-        c = hist[tid];
-        inc = wave_scan(c);
-        if ((tid & 63) == 63) wsum[tid >> 6] = inc;
-    }
-    __syncthreads();
-    if (tid == 0) hist[kMaxDigits] = (uint32_t)n;
-    if (tid < kMaxDigits) {
-        uint32_t b = inc - c;
-        for (int q = 0; q < (tid >> 6); ++q) b += wsum[q];
-        hist[tid] = b;
-        uint16_t* rs = run_start + (int64_t)page * kRunStride;
-        rs[tid] = (uint16_t)b;
-        if (tid == kMaxDigits - 1) rs[kMaxDigits] = (uint16_t)n;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kItems; ++k)
-        if (tid + 1024 * k < n) {
-            const uint32_t dg = (key[k] >> kRowBits) & (uint32_t)(kMaxDigits - 1);
-            const uint32_t h0 = hist[dg], q = (hist[dg + 1] - h0) >> 5;
-            uint32_t at = rank[k];
-            if (q > 1u && at < q << 5) {
-                const uint32_t hi = (uint32_t)(((float)at + 0.5f) * __builtin_amdgcn_rcpf((float)q));
-                at = (at - hi * q) * 32u + hi;
-            }
-            at += h0;
-            sv[at] = val[k];
-            sk[at] = (uint16_t)(key[k] & (uint32_t)(kRows - 1));
-        }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kItems; ++k) {
-        const int i = tid + 1024 * k;
-        if (i < n) vals[first + i] = sv[i];
-    }
-#pragma unroll
-    for (int k = 0; k < kItems; ++k) {
-        const int i = tid + 1024 * k;
-        if (i < n) {
-            const float2 f = pair_value(sv[i]);
-            keys[first + i] = (uint32_t)sk[i] |
-                              (__float_as_uint(f.x) >> 23 & 255u) << kRowBits |
-                              (__float_as_uint(f.y) >> 23 & 255u) << (kRowBits + 8);
-        }
-    }
-}
-
-// Runs of one bucket in pages [p0, p1) of a level.  A wave takes every 16th
-// pair of pages: its lanes look 64 runs up at once, and each half of the wave
-// then reads its page's run, 32 pairs a load, eight pairs of pages in flight
-// together.  body.load(base, i): pair base + i of the arrays (base is the
-// same for the wave); body.use(payload).  Returns the pairs of the runs that
-// this lane looked up.
+// Runs of one bucket in pages [p0, p1) of a level: a wave takes every 16th
+// page.  Its lanes look 64 runs up at once; each run is read by the whole
+// wave, 64 pairs a load, eight runs' loads in flight together.  body.load(base,
+// i): pair base + i of the arrays (base is the same for the wave);
+// body.use(payload).  Returns the pairs of the runs that this lane looked up.
 struct RunSpan {
     const uint16_t* run_start;   // the level's first page, at the bucket
     int64_t first;               // the level's first pair
@@ -706,48 +569,45 @@ struct RunSpan {
 template <class Body>
 __device__ __forceinline__ uint32_t for_runs(const RunSpan& s, const Body& body) {
     constexpr int kU = 8;
-    const uint32_t lane = threadIdx.x & 63u, p = lane & 31u, half = lane >> 5;
+    const uint32_t lane = threadIdx.x & 63u;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     uint32_t total = 0;
-    for (int b = s.p0 + 2 * wave; b < s.p1; b += 32 * 32) {
-        const int mine = b + 32 * (int)(lane >> 1) + (int)(lane & 1u);
+    for (int b = s.p0 + wave; b < s.p1; b += 16 * 64) {
+        const int mine = b + 16 * (int)lane;
         uint32_t both = 0;   // two neighbouring 16-bit entries: start, end
         if (mine < s.p1) __builtin_memcpy(&both, s.run_start + (int64_t)mine * kRunStride, 4);
         total += (both >> 16) - (both & 0xffffu);
-        const int pairs = (s.p1 - b + 31) / 32 < 32 ? (s.p1 - b + 31) / 32 : 32;
-        for (int q = 0; q < pairs; q += kU) {
-            const int64_t base0 = s.first + (int64_t)(b + 32 * q) * kPage;
+        const int runs = (s.p1 - b + 15) / 16 < 64 ? (s.p1 - b + 15) / 16 : 64;
+        for (int q = 0; q < runs; q += kU) {
+            const int64_t base0 = s.first + (int64_t)(b + 16 * q) * kPage;
+            uint32_t st[kU], len[kU];
             typename Body::Payload v[kU];
-            uint32_t run[kU];
             bool longer = false;
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
-                const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)both, (2 * (q + u)) & 63);
-                const uint32_t d1 = (uint32_t)__builtin_amdgcn_readlane((int)both, (2 * (q + u) + 1) & 63);
-                longer = longer || (d0 >> 16) - (d0 & 0xffffu) > 32u || (d1 >> 16) - (d1 & 0xffffu) > 32u;
-                run[u] = half ? d1 : d0;
-                const uint32_t i = (run[u] & 0xffffu) + p;
-                if (i < run[u] >> 16)
-                    v[u] = body.load(base0 + (int64_t)(u * 32 * kPage), i + half * (uint32_t)kPage);
+                const uint32_t d = (uint32_t)__builtin_amdgcn_readlane((int)both, (q + u) & 63);
+                st[u] = d & 0xffffu;
+                len[u] = (d >> 16) - st[u];
+                longer = longer || len[u] > 64u;
+                if (lane < len[u]) v[u] = body.load(base0 + (int64_t)(u * 16 * kPage) + st[u], lane);
             }
 #pragma unroll
             for (int u = 0; u < kU; ++u)
-                if ((run[u] & 0xffffu) + p < run[u] >> 16) body.use(v[u]);
+                if (lane < len[u]) body.use(v[u]);
             if (!longer) continue;
 #pragma unroll 1
             for (int u = 0; u < kU; ++u) {
-                const uint32_t d0 = (uint32_t)__builtin_amdgcn_readlane((int)both, (2 * (q + u)) & 63);
-                const uint32_t d1 = (uint32_t)__builtin_amdgcn_readlane((int)both, (2 * (q + u) + 1) & 63);
-                const uint32_t d = half ? d1 : d0, e = d >> 16;
-                const int64_t base = base0 + (int64_t)(u * 32 * kPage);
-                for (uint32_t i = (d & 0xffffu) + p + 32u; i < e; i += 128u) {
+                const uint32_t d = (uint32_t)__builtin_amdgcn_readlane((int)both, (q + u) & 63);
+                const uint32_t n = (d >> 16) - (d & 0xffffu);
+                const int64_t base = base0 + (int64_t)(u * 16 * kPage) + (d & 0xffffu);
+                for (uint32_t j = 64; j < n; j += 256) {
                     typename Body::Payload w[4];
 #pragma unroll
                     for (uint32_t c = 0; c < 4; ++c)
-                        if (i + 32u * c < e) w[c] = body.load(base, i + 32u * c + half * (uint32_t)kPage);
+                        if (j + 64 * c + lane < n) w[c] = body.load(base + j, 64 * c + lane);
 #pragma unroll
                     for (uint32_t c = 0; c < 4; ++c)
-                        if (i + 32u * c < e) body.use(w[c]);
+                        if (j + 64 * c + lane < n) body.use(w[c]);
                 }
             }
         }
@@ -864,7 +724,7 @@ __global__ void __launch_bounds__(1024) k_page_reduce(TableLevels t,
     const int pb = plan->page_base[l], np = plan->page_base[l + 1] - pb;
     RunSpan s;
     s.run_start = run_start + (int64_t)pb * kRunStride + d;
-    s.first = plan->level_start[l];
+    s.first = (int64_t)pb * kPage;
     s.p0 = (int)((int64_t)np * slice / S);
     s.p1 = (int)((int64_t)np * (slice + 1) / S);
     for (int q = tid; q < 2 * kRows; q += 1024) mx[q] = 0u;
@@ -929,29 +789,44 @@ __global__ void __launch_bounds__(256) k_page_combine(TableLevels t,
     }
 }
 
-template <class VT>
-static int run_paged(TableReduceWs& w, const am_grid_desc* g, float* dtable, hipStream_t s) {
-    const TableLevels t = table_levels(g);
-    VT* vals = reinterpret_cast<VT*>(w.vals[0]);
-    {
-        KernelTimer kt_("radix_sort", s);
-        hipLaunchKernelGGL(k_page_plan, dim3(1), dim3(64), 0, s, t, w.level_start, w.plan);
-        AM_LAUNCH_CHECK();
-        hipLaunchKernelGGL((k_page_partition<VT>), dim3((unsigned)page_bound(w.m, t.L)), dim3(1024),
-                           0, s, t, w.plan, w.keys[0], vals, w.run_start);
-        AM_LAUNCH_CHECK();
-    }
-    KernelTimer kt_("seg_reduce", s);
-    // units <= buckets + pairs / unit pairs (both unit sizes of k_page_plan)
-    const int64_t least = w.m / kUnitLeast, most = w.m / kUnitMost;
-    const int64_t units = table_digits(g) + (least < 1024 ? least : (most > 1024 ? most : 1024)) + 2;
-    const unsigned grid = (unsigned)(ceil_div(units, 256) * 256);   // whole groups of 8 x 32
-    hipLaunchKernelGGL((k_page_reduce<VT>), dim3(grid), dim3(1024), 0, s, t, w.plan, w.keys[0], vals,
-                       w.run_start, dtable, w.partial2);
-    AM_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_page_combine, dim3(2048), dim3(256), 0, s, t, w.plan, w.partial2, dtable);
+void table_pages_carve(WsCarver& c, int64_t pages, bool half_vals, TablePages* out) {
+    TablePages w{};
+    w.pages = pages;
+    w.half_vals = half_vals;
+    w.keys = c.take<uint32_t>((size_t)pages * kPage);
+    w.vals = c.take<char>((size_t)pages * kPage * (half_vals ? 4 : 8));
+    w.run_start = c.take<uint16_t>((size_t)pages * kRunStride + 2);
+    w.partial = c.take<double2>((size_t)slot_bound(pages * kPage) << kRowBits);
+    w.plan = c.take<PagePlan>(1);
+    *out = w;
+}
+
+int table_pages_plan(TablePages& w, const am_grid_desc* g, const uint64_t* scan, int64_t units,
+                     int active, int64_t per_level, hipStream_t s) {
+    hipLaunchKernelGGL(k_page_plan, dim3(1), dim3(64), 0, s, table_levels(g), scan, units, active,
+                       per_level, w.plan);
     AM_LAUNCH_CHECK();
     return AM_OK;
+}
+
+template <class VT>
+static int run_pages(TablePages& w, const am_grid_desc* g, float* dtable, hipStream_t s) {
+    const TableLevels t = table_levels(g);
+    KernelTimer kt_("seg_reduce", s);
+    // units <= buckets + pairs / unit pairs (both unit sizes of k_page_plan)
+    const int64_t m = w.pages * kPage, least = m / kUnitLeast, most = m / kUnitMost;
+    const int64_t units = table_digits(g) + (least < 1024 ? least : (most > 1024 ? most : 1024)) + 2;
+    const unsigned grid = (unsigned)(ceil_div(units, 256) * 256);   // whole groups of 8 x 32
+    hipLaunchKernelGGL((k_page_reduce<VT>), dim3(grid), dim3(1024), 0, s, t, w.plan, w.keys,
+                       reinterpret_cast<const VT*>(w.vals), w.run_start, dtable, w.partial);
+    AM_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_page_combine, dim3(2048), dim3(256), 0, s, t, w.plan, w.partial, dtable);
+    AM_LAUNCH_CHECK();
+    return AM_OK;
+}
+
+int table_pages_run(TablePages& w, const am_grid_desc* g, float* dtable, hipStream_t s) {
+    return w.half_vals ? run_pages<uint32_t>(w, g, dtable, s) : run_pages<uint2>(w, g, dtable, s);
 }
 
 template <class VT>
@@ -1044,9 +919,6 @@ int table_reduce_run(TableReduceWs& w, const am_grid_desc* g, float* dtable,
                      hipStream_t stream) {
     const int F = g->n_features;
     const uint32_t n_entries = g->n_entries;
-    if (w.paged)
-        return w.half_vals ? run_paged<uint32_t>(w, g, dtable, stream)
-                           : run_paged<uint2>(w, g, dtable, stream);
     if (F == 2 && w.n_buckets > 0) {
         if (w.begin_bit > kMaxBucketBits) {
             set_error("bucket bits %d above %d", w.begin_bit, kMaxBucketBits);
