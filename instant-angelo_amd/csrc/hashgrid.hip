@@ -206,11 +206,11 @@ __global__ void __launch_bounds__(kPageThreads) k_hg_pages(
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
             const float w = corner_weight(p, c);
-            pg.keys[c * np + q] = rows[c];
-            put_pair(pg.vals[c * np + q], w * g0, w * g1);
+            page_put(pg, c * np + q, rows[c], w * g0, w * g1);
         }
     }
-    page_flush(pg, 8 * np, blockIdx.x, keys, vals, run_start);
+    page_flush(pg, 8 * np, (lp.size_flags & kSizeMask) <= (uint32_t)kSpreadDigits * kRows, blockIdx.x,
+               keys, vals, run_start);
 }
 
 static int hg_bwd_pages(const GridArgs& ga, const am_grid_desc* g, const float* x, int64_t n,

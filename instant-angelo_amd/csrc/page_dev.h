@@ -22,13 +22,6 @@ __device__ __forceinline__ float2 pair_value(uint2 v) {
 __device__ __forceinline__ float2 pair_value(uint32_t v) {
     return __half22float2(__builtin_bit_cast(__half2, v));
 }
-__device__ __forceinline__ void put_pair(uint2& v, float a, float b) {
-    v = make_uint2(__float_as_uint(a), __float_as_uint(b));
-}
-__device__ __forceinline__ void put_pair(uint32_t& v, float a, float b) {
-    v = __builtin_bit_cast(uint32_t, __halves2half2(__float2half_rn(a), __float2half_rn(b)));
-}
-
 // Inclusive sum over the wave's lanes.
 __device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
 #pragma unroll
@@ -41,39 +34,61 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
 
 // The page under construction: pairs in any order (keys: rows within the
 // level).  hist is zero between flushes.
+// Values are kept by word (fp32: the first features, then the second ones;
+// fp16: the pairs).
 template <class VT>
 struct PageLds {
-    VT vals[kPage];
+    uint32_t words[sizeof(VT) / 4][kPage];
     uint32_t keys[kPage];
     uint32_t hist[kMaxDigits + 4];
-    uint32_t wave_pairs[2][16];   // pairs of each wave in a step (two steps in turn)
-    uint32_t general[2];          // evaluations on the general path, by cluster
+    uint32_t cursor;   // pairs put so far
 };
+
+__device__ __forceinline__ void page_put(PageLds<uint2>& s, int at, uint32_t row, float a, float b) {
+    s.keys[at] = row;
+    s.words[0][at] = __float_as_uint(a);
+    s.words[1][at] = __float_as_uint(b);
+}
+__device__ __forceinline__ void page_put(PageLds<uint32_t>& s, int at, uint32_t row, float a,
+                                         float b) {
+    s.keys[at] = row;
+    s.words[0][at] =
+        __builtin_bit_cast(uint32_t, __halves2half2(__float2half_rn(a), __float2half_rn(b)));
+}
+__device__ __forceinline__ uint2 page_value(const PageLds<uint2>& s, int i) {
+    return make_uint2(s.words[0][i], s.words[1][i]);
+}
+__device__ __forceinline__ uint32_t page_value(const PageLds<uint32_t>& s, int i) {
+    return s.words[0][i];
+}
 
 // Partitions the LDS page's n pairs by bucket and writes them to page `page`.
 // The runs hold their pairs in any order (the reduce's sums do not depend on
-// it), so each pair's place comes from one LDS counter; in runs of 128 pairs
-// or more, pairs that arrive together (neighbouring samples, often of one
-// row) are set a wave's load apart, so that the reduce's LDS additions seldom
-// meet in one row (for 60 M pairs in runs of 16 equal rows: 0.80 -> 0.34 ms).
-// Called by all kPageThreads threads.
+// it), so each pair's place comes from one LDS counter.  spread (levels of
+// few buckets, whose runs are long and full of repeated rows): pairs that
+// arrive together, neighbouring samples often of one row, are set a wave's
+// load apart, so that the reduce's LDS additions seldom meet in one row (60 M
+// pairs in runs of 16 equal rows: reduce 0.80 -> 0.34 ms).  The second
+// features move after the others, to hold few registers beside the caller's.
+// Bound by LDS operations.  Called by all kPageThreads threads; leaves the
+// page empty.
 template <class VT>
-__device__ __forceinline__ void page_flush(PageLds<VT>& s, int n, int64_t page,
+__device__ __forceinline__ void page_flush(PageLds<VT>& s, int n, bool spread, int64_t page,
                                            uint32_t* __restrict__ keys, VT* __restrict__ vals,
                                            uint16_t* __restrict__ run_start) {
     constexpr int kItems = kPage / kPageThreads;
-    const int tid = (int)threadIdx.x;
-    uint32_t key[kItems], at[kItems];
-    VT val[kItems];
+    int tid = (int)threadIdx.x;
+    asm volatile("" : "+v"(tid));   // keeps its addresses out of the caller's loop registers
+    uint32_t key[kItems], at[kItems], first[kItems];   // first: words[0]
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kItems; ++k) {
         const int i = tid + kPageThreads * k;
         if (i < n) {
             key[k] = s.keys[i];
-            val[k] = s.vals[i];
             at[k] = atomicAdd(&s.hist[(key[k] >> kRowBits) & (uint32_t)(kMaxDigits - 1)], 1u);
         }
+        if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
     __syncthreads();
     if (tid < 64) {   // four counters a lane
@@ -94,6 +109,7 @@ __device__ __forceinline__ void page_flush(PageLds<VT>& s, int n, int64_t page,
         if (tid == 63) {
             s.hist[kMaxDigits] = (uint32_t)n;
             rs[kMaxDigits] = (uint16_t)n;
+            s.cursor = 0u;
         }
     }
     __syncthreads();
@@ -101,19 +117,41 @@ __device__ __forceinline__ void page_flush(PageLds<VT>& s, int n, int64_t page,
     for (int k = 0; k < kItems; ++k)
         if (tid + kPageThreads * k < n) {
             const uint32_t d = (key[k] >> kRowBits) & (uint32_t)(kMaxDigits - 1);
-            const uint32_t h0 = s.hist[d], q = (s.hist[d + 1] - h0) >> 6;
+            const uint32_t h0 = s.hist[d];
             uint32_t r = at[k];
-            if (q > 1u && r < q << 6) {   // r = a q + b -> 64 b + a
-                const uint32_t a = (uint32_t)(((float)r + 0.5f) * __builtin_amdgcn_rcpf((float)q));
-                r = (r - a * q) * 64u + a;
+            if (spread) {
+                const uint32_t q = (s.hist[d + 1] - h0) >> 6;
+                if (q > 1u && r < q << 6) {   // r = a q + b -> 64 b + a
+                    const uint32_t a =
+                        (uint32_t)(((float)r + 0.5f) * __builtin_amdgcn_rcpf((float)q));
+                    r = (r - a * q) * 64u + a;
+                }
             }
             r += h0;
-            const float2 f = pair_value(val[k]);
-            s.keys[r] = (key[k] & (uint32_t)(kRows - 1)) |
-                        (__float_as_uint(f.x) >> 23 & 255u) << kRowBits |
-                        (__float_as_uint(f.y) >> 23 & 255u) << (kRowBits + 8);
-            s.vals[r] = val[k];
+            at[k] = r;
+            const int i = tid + kPageThreads * k;
+            const float2 f = pair_value(page_value(s, i));
+            first[k] = s.words[0][i];
+            key[k] = (key[k] & (uint32_t)(kRows - 1)) |
+                     (__float_as_uint(f.x) >> 23 & 255u) << kRowBits |
+                     (__float_as_uint(f.y) >> 23 & 255u) << (kRowBits + 8);
         }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kItems; ++k)
+        if (tid + kPageThreads * k < n) {
+            s.keys[at[k]] = key[k];
+            s.words[0][at[k]] = first[k];
+        }
+    if constexpr (sizeof(VT) == 8) {
+#pragma unroll
+        for (int k = 0; k < kItems; ++k)
+            if (tid + kPageThreads * k < n) first[k] = s.words[1][tid + kPageThreads * k];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kItems; ++k)
+            if (tid + kPageThreads * k < n) s.words[1][at[k]] = first[k];
+    }
     __syncthreads();
     keys += page * kPage;
     vals += page * kPage;
@@ -122,11 +160,15 @@ __device__ __forceinline__ void page_flush(PageLds<VT>& s, int n, int64_t page,
         const int i = tid + kPageThreads * k;
         if (i < n) {
             keys[i] = s.keys[i];
-            vals[i] = s.vals[i];
+            vals[i] = page_value(s, i);
         }
+        if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
     if (tid <= kMaxDigits) s.hist[tid] = 0u;
     __syncthreads();
 }
+
+// Levels of at most this many buckets spread their runs.
+constexpr int kSpreadDigits = 96;
 
 }  // namespace am

@@ -52,9 +52,14 @@ __device__ __forceinline__ void merge_step(int p, float acc[16], bool& end) {
 // the cluster's cell serve all its evaluations.  Along axis d only the d
 // coordinate of an offset evaluation differs from the centre's: one position,
 // one comparison and two weights each.  (A sample outside the box has its
-// offset points clamped in the other axes too: such lanes, and offsets
-// beyond one cell, take the general path, all 8 corners of each evaluation.)
-constexpr int kPairSteps = 26;   // per cluster: 6 far faces, 6 general, 1 centre cell
+// offset points clamped in the other axes too: such lanes are classified by
+// whole cells, in the general steps that also take the offsets beyond one
+// cell.)
+// An emission step puts at most 4 pairs a lane.  Per cluster: the far faces of
+// the 6 offset evaluations; their general steps, two each (corners 0-3 or the
+// far face, corners 4-7); the centre cell's two.
+constexpr int kClusterSteps = 19;   // counted: 6, 6 + 6, 1 (both halves alike)
+constexpr int kPairSteps = 2 * kClusterSteps;
 
 __device__ __forceinline__ LevelParams scalar_level(const LevelParams& lp) {
     LevelParams r;
@@ -96,6 +101,46 @@ __device__ __forceinline__ ClusterCell cluster_cell(const GeoArgs& a, const Leve
     return ClusterCell{level_pos(lp, xc), CL == 0 && out};
 }
 
+// Corner i (0..3) of the face of a cell with bit `ax` fixed to `b`.
+__device__ __forceinline__ int face_corner(int i, int ax, int b) {
+    const int low = i & ((1 << ax) - 1);
+    return low | (b << ax) | ((i >> ax) << (ax + 1));
+}
+
+// Offset evaluation j against the centre's cell by whole cells: `same` cell,
+// a face neighbour along `axis` (`adj`; `up`: on its high side), or neither.
+struct CellClass {
+    LevelPos pos;
+    bool same, adj, up;
+    int axis;
+};
+
+__device__ __forceinline__ CellClass classify(const GeoArgs& a, const LevelParams& lp,
+                                              const float P[3], int j, const uint32_t B[3]) {
+    float x[3];
+    bool inb[3];
+    offset_point(a, P, j, x, inb);
+    CellClass r;
+    r.pos = level_pos(lp, x);
+    int nz = 0;
+    bool unit = true;
+    r.axis = 0;
+    r.up = false;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int dd = (int)(r.pos.c[d] - B[d]);
+        if (dd != 0) {
+            ++nz;
+            r.axis = d;
+            r.up = dd > 0;
+            unit = unit && (dd == 1 || dd == -1);
+        }
+    }
+    r.same = nz == 0;
+    r.adj = nz == 1 && unit;
+    return r;
+}
+
 // Whether this lane's accumulators start a run of equal cells in its 16 lanes.
 __device__ __forceinline__ bool cell_head(const uint32_t B[3], bool live, bool* end) {
     const uint32_t INV = 0xFFFFFFFFu;
@@ -124,23 +169,41 @@ __device__ __forceinline__ void count_cluster(const GeoArgs& a, const LevelParam
             const bool adj = !cc.general && (dd == 1 || dd == -1);
             touched = touched || same || adj;
             const uint32_t nf = (uint32_t)__popcll(__ballot(on && adj));
-            const uint32_t ng = (uint32_t)__popcll(__ballot(on && !same && !adj));
+            const uint32_t ng = (uint32_t)__popcll(__ballot(on && !cc.general && !same && !adj));
             if (lane_id() == 0) {
                 if (nf) atomicAdd(&tot[j], 4u * nf);
-                if (ng) atomicAdd(&tot[6 + j], 4u * ng);
+                if (ng) {
+                    atomicAdd(&tot[6 + j], 4u * ng);
+                    atomicAdd(&tot[12 + j], 4u * ng);
+                }
+            }
+        }
+        if (CL == 0 && __builtin_expect(__ballot(on && cc.general) != 0, 0)) {
+#pragma unroll 1
+            for (int j = 0; j < 6; ++j) {
+                const CellClass cl = classify(a, lp, P, j, cc.pos.c);
+                const bool mine = on && cc.general && !cl.same;
+                const uint32_t ng = (uint32_t)__popcll(__ballot(mine && !cl.adj));
+                const uint32_t na = (uint32_t)__popcll(__ballot(mine && cl.adj));
+                if (lane_id() == 0 && ng + na) {
+                    atomicAdd(&tot[6 + j], 4u * (ng + na));
+                    atomicAdd(&tot[12 + j], 4u * ng);
+                }
             }
         }
     }
     const uint32_t nh =
         (uint32_t)__popcll(__ballot(cell_head(cc.pos.c, on && touched, nullptr)));
-    if (lane_id() == 0 && nh) atomicAdd(&tot[12], 4u * nh);
+    if (lane_id() == 0 && nh) atomicAdd(&tot[18], 4u * nh);
 }
 
 // Count pass: per unit (level, block of 1024 samples), the pairs of each
-// emission step, from positions alone.  steps[unit][13 c + s]: cluster c
-// (0: curvature, 1: base and FD), step s (0-5 far faces, 6-11 half a general
-// evaluation's, 12 half the centre cell's).  Also keeps the cluster centres
-// for the emission.
+// emission step, from positions alone.  steps[unit][kClusterSteps c + s]:
+// cluster c (0: curvature, 1: base and FD), step s (0-5 far faces, 6-11 the
+// general evaluations' first halves, 12-17 their second, 18 half the centre
+// cell's).  Also keeps the cluster centres
+// for the emission.  A block covers levels blockIdx.y, + gridDim.y, ...: all
+// of them when the sample blocks alone fill the chip (page_count_split).
 __global__ void __launch_bounds__(1024) k_page_count(GeoArgs a, const float* __restrict__ pts,
                                                      const float* __restrict__ randn, int64_t N,
                                                      const float* __restrict__ fdv,
@@ -159,21 +222,23 @@ __global__ void __launch_bounds__(1024) k_page_count(GeoArgs a, const float* __r
     const bool on = n < N;
     GeoSample s;
     geo_rebuild(a, pts, randn, fdv, n, caller_row(a, n, on), on, s);
+    if (blockIdx.y == 0) {
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        centers[d * row + n] = s.P[d];
-        if (a.with_laplace) centers[(3 + d) * row + n] = s.ps[d];
+        for (int d = 0; d < 3; ++d) {
+            centers[d * row + n] = s.P[d];
+            if (a.with_laplace) centers[(3 + d) * row + n] = s.ps[d];
+        }
     }
     const bool fd = a.with_grad && !a.analytic;
-    for (int l = 0; l < a.active; ++l) {
+    for (int l = (int)blockIdx.y; l < a.active; l += (int)gridDim.y) {
         const LevelParams lp = scalar_level(lv[l]);
         if (a.with_laplace) count_cluster<1>(a, lp, s.ps, on, true, tot + l * kPairSteps);
-        count_cluster<0>(a, lp, s.P, on, fd, tot + l * kPairSteps + 13);
+        count_cluster<0>(a, lp, s.P, on, fd, tot + l * kPairSteps + kClusterSteps);
     }
     __syncthreads();
     for (int q = tid; q < a.active * kPairSteps; q += 1024) {
         const int l = q / kPairSteps;
-        steps[((int64_t)l * gridDim.x + blockIdx.x) * kPairSteps + (q - l * kPairSteps)] = tot[q];
+        if (l % (int)gridDim.y == (int)blockIdx.y) steps[((int64_t)l * gridDim.x + blockIdx.x) * kPairSteps + (q - l * kPairSteps)] = tot[q];
     }
 }
 
@@ -182,56 +247,106 @@ __global__ void __launch_bounds__(1024) k_page_count(GeoArgs a, const float* __r
 __global__ void k_unit_pages(const uint32_t* __restrict__ steps, int64_t units,
                              uint64_t* __restrict__ out) {
     const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (u > units) return;
+    if (u >= units) return;
     uint64_t pages = 0, pairs = 0;
     uint32_t cursor = 0;
-    if (u < units) {
-        const uint32_t* st = steps + u * kPairSteps;
-        for (int q = 0; q < kPairSteps; ++q) {
-            const int s = q % 13;
-            for (int h = 0; h < (s < 6 ? 1 : 2); ++h) {
-                if (cursor + st[q] > (uint32_t)kPage) {
-                    ++pages;
-                    cursor = 0;
-                }
-                cursor += st[q];
-                pairs += st[q];
+    const uint32_t* st = steps + u * kPairSteps;
+    for (int c = 0; c < 2; ++c, st += kClusterSteps)
+        for (int q = 0; q < 20; ++q) {   // far faces, general halves, centre cell's halves
+            const uint32_t n =
+                st[q < 6 ? q : (q < 18 ? 6 + ((q & 1) ? 6 : 0) + ((q - 6) >> 1) : 18)];
+            if (cursor + n > (uint32_t)kPage) {
+                ++pages;
+                cursor = 0;
             }
+            cursor += n;
+            pairs += n;
         }
-        if (cursor) ++pages;
-    }
+    if (cursor) ++pages;
     out[u] = pages << 40 | pairs;
 }
 
-__global__ void k_page_status(const uint64_t* __restrict__ scan, int64_t units,
-                              int64_t* __restrict__ status) {
-    if (threadIdx.x == 0) {
-        status[0] = (int64_t)(scan[units] >> 40);
+// Exclusive scan of the units' pages and pairs, and the totals.  One block: a
+// unit is 1024 samples of a level, so a thread has few (4.8 M points: 74).
+__global__ void __launch_bounds__(1024) k_unit_scan(const uint64_t* __restrict__ in, int64_t units,
+                                                    uint64_t* __restrict__ scan,
+                                                    int64_t* __restrict__ status) {
+    __shared__ uint64_t wave_sum[16];
+    const int tid = (int)threadIdx.x;
+    const int64_t each = (units + 1023) / 1024;
+    const int64_t u0 = tid * each < units ? tid * each : units;
+    const int64_t u1 = u0 + each < units ? u0 + each : units;
+    uint64_t sum = 0;
+    for (int64_t u = u0; u < u1; ++u) sum += in[u];
+    uint64_t incl = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint64_t o = __shfl_up((unsigned long long)incl, d, 64);
+        if ((tid & 63) >= d) incl += o;
+    }
+    if ((tid & 63) == 63) wave_sum[tid >> 6] = incl;
+    __syncthreads();
+    uint64_t at = incl - sum, total = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        if (w < tid >> 6) at += wave_sum[w];
+        total += wave_sum[w];
+    }
+    for (int64_t u = u0; u < u1; ++u) {
+        scan[u] = at;
+        at += in[u];
+    }
+    if (tid == 0) {
+        scan[units] = total;
+        status[0] = (int64_t)(total >> 40);
         status[1] = 0;
-        status[2] = (int64_t)(scan[units] & ((1ull << 40) - 1ull));
+        status[2] = (int64_t)(total & ((1ull << 40) - 1ull));
     }
 }
 
-// Row of a corner from its per-axis terms (x, or the products with the hash
-// primes or strides).
-__device__ __forceinline__ uint32_t term_row(const LevelParams& lp, uint32_t x, uint32_t y,
-                                             uint32_t z) {
-    const bool hashed = (lp.size_flags & kHashedBit) != 0u;
-    return wrap_row(hashed ? (x ^ y ^ z) : (x + y + z), lp.size_flags);
+// Four rows of a level from a corner face: terms a (fixed), b0 / b1 and c0 / c1
+// (x, or the products with the hash primes or strides; their order does not
+// matter).
+__device__ __forceinline__ void face_rows(const LevelParams& lp, uint32_t a, uint32_t b0,
+                                          uint32_t b1, uint32_t c0, uint32_t c1, uint32_t r[4]) {
+    if (lp.size_flags & kHashedBit) {
+        r[0] = a ^ b0 ^ c0;
+        r[1] = a ^ b1 ^ c0;
+        r[2] = a ^ b0 ^ c1;
+        r[3] = a ^ b1 ^ c1;
+    } else {
+        r[0] = a + b0 + c0;
+        r[1] = a + b1 + c0;
+        r[2] = a + b0 + c1;
+        r[3] = a + b1 + c1;
+    }
+    if (lp.size_flags & kPow2Bit) {
+        const uint32_t m = (lp.size_flags & kSizeMask) - 1u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] &= m;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = wrap_row(r[i], lp.size_flags);
+    }
 }
 
 // Emission: one block per unit collects the unit's pairs in an LDS page,
 // step by step (all lanes' far faces of one offset evaluation, at most 4096
-// pairs), and writes each page partitioned (page_flush).  A step costs one
-// barrier: the waves' pair counts are exchanged through LDS and each wave
-// places its own.  Writing pairs straight into partitioned pages spares
+// pairs), and writes each page partitioned (page_flush).  The counted steps
+// say beforehand which steps share a page, so the waves run through them
+// without meeting, each taking its place from one LDS counter, and meet only
+// to write a page.  Writing pairs straight into partitioned pages spares
 // writing them once unpartitioned and reading them back.  LDS (148 KB) holds
-// it to one block of 16 waves a CU; bound by VALU issue.
+// it to one block of 16 waves a CU; bound by VALU issue in the steps and by
+// LDS operations in the flushes.  940 k samples, 16 levels, 13 evaluations:
+// 2.43 ms, and a forward and backward 11.3 ms, where writing level streams and
+// partitioning them in a pass of its own took 13.57 ms.
 template <int LJ, class VT>
 __global__ void __launch_bounds__(1024) k_pair_pages(GeoArgs a, const float* __restrict__ centers,
                                                      int64_t N, int64_t blocks,
                                                      const float* __restrict__ genc,
                                                      const uint64_t* __restrict__ scan,
+                                                     const uint32_t* __restrict__ steps,
                                                      int64_t capacity, uint32_t* __restrict__ keys,
                                                      VT* __restrict__ vals,
                                                      uint16_t* __restrict__ run_start,
@@ -252,7 +367,7 @@ __global__ void __launch_bounds__(1024) k_pair_pages(GeoArgs a, const float* __r
         return;
     }
     if (tid <= kMaxDigits) pg.hist[tid] = 0u;
-    if (tid < 2) pg.general[tid] = 0u;
+    if (tid == 0) pg.cursor = 0u;
     __shared__ LevelParams lvs;
 #pragma unroll
     for (int q = 0; q < AM_MAX_LEVELS; ++q)
@@ -262,76 +377,44 @@ __global__ void __launch_bounds__(1024) k_pair_pages(GeoArgs a, const float* __r
     const int64_t n = sb * 1024 + tid, row = blocks * 1024;
     const bool on = n < N;
     int64_t page = page0;
-    int cursor = 0, par = 0;
+    int cursor = 0;
+    const bool spread = (lp.size_flags & kSizeMask) <= (uint32_t)kSpreadDigits * kRows;
     auto flush = [&]() {
         if (page < page_end)
-            page_flush(pg, cursor, page, keys, vals, run_start);
+            page_flush(pg, cursor, spread, page, keys, vals, run_start);
         else
             __syncthreads();
         ++page;
         cursor = 0;
     };
-    // place of this lane's first of 4 pairs (they go n_on apart); the block's
-    // pairs of the step; starts a new page when they do not fit
-    auto reserve = [&](bool put, int& n_on, int& at) -> int {
-        const uint64_t mask = __ballot(put);
-        n_on = __popcll(mask);
-        if (lane == 0) pg.wave_pairs[par][wave] = 4u * (uint32_t)n_on;
-        __syncthreads();
-        uint32_t v = pg.wave_pairs[par][p];
-        par ^= 1;
-        v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);
-        v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
-        v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
-        v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
-        const int total = __builtin_amdgcn_readlane((int)v, 15);
-        const int before = __builtin_amdgcn_readlane((int)v, wave) - 4 * n_on;
-        if (cursor + total > kPage) flush();
-        at = cursor + before +
-             (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                            __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-        cursor += total;
-        return total;
-    };
-    auto put4 = [&](int at, int n_on, const uint32_t r[4], const float v[8]) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            pg.keys[at + i * n_on] = r[i];
-            put_pair(pg.vals[at + i * n_on], v[2 * i], v[2 * i + 1]);
-        }
-    };
     const bool hashed = (lp.size_flags & kHashedBit) != 0u;
-    const uint32_t mul[3] = {1u, hashed ? 2654435761u : lp.res, hashed ? 805459861u : lp.res * lp.res};
-    // this lane's encode gradients: slot s, feature f at gl[s * LJ * 512 + f * 64]
-    const float* gl = genc + (n >> 6) * a.genc_slots * (int64_t)(LJ * 512) + level * 128 + lane;
+    const uint32_t my = hashed ? 2654435761u : lp.res, mz = hashed ? 805459861u : lp.res * lp.res;
+    // the wave's encode gradients: slot s, feature f at gl[s * LJ * 512 + f * 64 + lane]
+    const float* gl = genc + (sb * 16 + wave) * a.genc_slots * (int64_t)(LJ * 512) + level * 128;
+    const float* cen = centers + sb * 1024;
     const bool fd = a.with_grad && !a.analytic;
 
 #pragma unroll 1
     for (int c = a.with_laplace ? 0 : 1; c < 2; ++c) {
         const bool curv = c == 0;
         const bool offsets = curv || fd;
-        const int slot0 = curv ? a.curv0 : 1;   // the offset evaluations' first slot
+        const float* go = gl + (curv ? a.curv0 : 1) * (LJ * 512);   // the offset evaluations
         float P[3];
 #pragma unroll
-        for (int d = 0; d < 3; ++d) P[d] = on ? centers[(curv ? 3 + d : d) * row + n] : 0.0f;
-        float g[6][2];
-        if (offsets && on) {
-#pragma unroll
-            for (int j = 0; j < 6; ++j)
-#pragma unroll
-                for (int f = 0; f < 2; ++f) g[j][f] = gl[(slot0 + j) * (LJ * 512) + f * 64];
-        } else {
-#pragma unroll
-            for (int j = 0; j < 6; ++j) g[j][0] = g[j][1] = 0.0f;
-        }
-        const ClusterCell cc = curv ? cluster_cell<1>(a, lp, P) : cluster_cell<0>(a, lp, P);
+        for (int d = 0; d < 3; ++d) P[d] = on ? (cen + (curv ? 3 + d : d) * row)[tid] : 0.0f;
+        ClusterCell cc = curv ? cluster_cell<1>(a, lp, P) : cluster_cell<0>(a, lp, P);
         const uint32_t* B = cc.pos.c;
         float acc[16];
 #pragma unroll
         for (int q = 0; q < 16; ++q) acc[q] = 0.0f;
         bool touched = !curv;
+        float n0 = 0.0f, n1 = 0.0f;   // the next evaluation's gradients, one ahead
+        if (offsets && on) {
+            n0 = go[lane];
+            n1 = go[64 + lane];
+        }
         if (!curv) {   // the base evaluation, always in B
-            const float g0 = on ? gl[0] : 0.0f, g1 = on ? gl[64] : 0.0f;
+            const float g0 = on ? gl[lane] : 0.0f, g1 = on ? gl[64 + lane] : 0.0f;
 #pragma unroll
             for (int t = 0; t < 8; ++t) {
                 const float w = corner_weight(cc.pos, t);
@@ -345,7 +428,7 @@ __global__ void __launch_bounds__(1024) k_pair_pages(GeoArgs a, const float* __r
                 for (int d = 0; d < 3; ++d)
 #pragma unroll
                     for (int f = 0; f < 2; ++f)
-                        ex[d][f] = on ? gl[(a.n_evals + d) * (LJ * 512) + f * 64] : 0.0f;
+                        ex[d][f] = on ? gl[(a.n_evals + d) * (LJ * 512) + f * 64 + lane] : 0.0f;
 #pragma unroll
                 for (int t = 0; t < 8; ++t)
 #pragma unroll
@@ -355,127 +438,189 @@ __global__ void __launch_bounds__(1024) k_pair_pages(GeoArgs a, const float* __r
                                           corner_dweight(cc.pos, t, 2) * ex[2][f];
             }
         }
-        // per-axis terms of B's corners: lo and hi = lo + mul
-        uint32_t lo[3];
+        // per-axis terms of B's corners: lo, and lo plus the axis's factor
+        uint32_t lo[3] = {B[0], B[1] * my, B[2] * mz};
+        // The cluster's steps, one loop body for all (the unrolled form is
+        // larger than the instruction cache): 0-5 the far faces, 6 the general
+        // evaluations' halves, 7 and 8 the centre cell's.
+        const uint32_t* st = steps + unit * kPairSteps + (curv ? 0 : kClusterSteps);
+        // (evaluations with pairs there, and all of a wave with lanes outside the
+        // box, whose evaluations may go into B alone)
+        uint32_t general = offsets && __ballot(on && cc.general) != 0 ? 63u : 0u;
 #pragma unroll
-        for (int d = 0; d < 3; ++d) lo[d] = B[d] * mul[d];
-        uint32_t general = 0u;   // evaluations with lanes on the general path
-        if (offsets) {
-#pragma unroll
-            for (int ax = 0; ax < 3; ++ax) {
-                const int b = ax == 0 ? 1 : 0, e = ax == 2 ? 1 : 2;   // the other axes
-                float w2[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    w2[i] = ((i & 1) ? cc.pos.f[b] : 1.0f - cc.pos.f[b]) *
-                            ((i & 2) ? cc.pos.f[e] : 1.0f - cc.pos.f[e]);
-#pragma unroll
-                for (int sg = 0; sg < 2; ++sg) {
-                    const int j = 2 * ax + sg;
-                    float f;
-                    const int dd = offset_cell(a, lp, P[ax], sg == 1, B[ax], f);
-                    const bool same = on && !cc.general && dd == 0;
-                    const bool adj = on && !cc.general && (dd == 1 || dd == -1);
-                    touched = touched || same || adj;
-                    float v0[4], v1[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        v0[i] = w2[i] * g[j][0];
-                        v1[i] = w2[i] * g[j][1];
-                    }
-                    // weight of B's low and high face of the axis
-                    const bool up = dd == 1;
-                    const float wl = same ? 1.0f - f : f, wh = same ? f : 1.0f - f;
-                    if (same || (adj && !up)) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int t = (i & 1) << b | (i >> 1) << e;
-                            acc[2 * t] = __fmaf_rn(wl, v0[i], acc[2 * t]);
-                            acc[2 * t + 1] = __fmaf_rn(wl, v1[i], acc[2 * t + 1]);
-                        }
-                    }
-                    if (same || (adj && up)) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int t = (i & 1) << b | (i >> 1) << e | 1 << ax;
-                            acc[2 * t] = __fmaf_rn(wh, v0[i], acc[2 * t]);
-                            acc[2 * t + 1] = __fmaf_rn(wh, v1[i], acc[2 * t + 1]);
-                        }
-                    }
-                    // the far face of a face neighbour
-                    int n_on, at;
-                    if (reserve(adj, n_on, at) && adj) {
-                        const uint32_t far = up ? lo[ax] + 2u * mul[ax] : lo[ax] - mul[ax];
-                        const float wf = up ? f : 1.0f - f;
-                        uint32_t r[4];
-                        float v[8];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const uint32_t tb = (i & 1) ? lo[b] + mul[b] : lo[b];
-                            const uint32_t te = (i & 2) ? lo[e] + mul[e] : lo[e];
-                            r[i] = ax == 0 ? term_row(lp, far, tb, te)
-                                           : (ax == 1 ? term_row(lp, tb, far, te)
-                                                      : term_row(lp, tb, te, far));
-                            v[2 * i] = wf * v0[i];
-                            v[2 * i + 1] = wf * v1[i];
-                        }
-                        put4(at, n_on, r, v);
-                    }
-                    if (__ballot(on && !same && !adj) != 0) general |= 1u << j;
-                }
-            }
-            // lanes on the general path: all 8 corners, in two halves
-            if (lane == 0 && general) atomicOr(&pg.general[c], general);
-            __syncthreads();
-            general = (uint32_t)__builtin_amdgcn_readfirstlane((int)pg.general[c]);
+        for (int j = 0; j < 6; ++j) general |= st[6 + j] != 0u ? 1u << j : 0u;
+        bool second = false;     // the second half of a general evaluation
+        bool head = false;
 #pragma unroll 1
-            for (uint32_t left = general; left != 0u; left &= left - 1u) {
-                const int j = __ffs((int)left) - 1;
-                float x[3], f;
-                bool inb[3];
-                offset_point(a, P, j, x, inb);
-                const float Pj = j < 2 ? P[0] : (j < 4 ? P[1] : P[2]);
-                const uint32_t Bj = j < 2 ? B[0] : (j < 4 ? B[1] : B[2]);
-                const int dd = offset_cell(a, lp, Pj, (j & 1) != 0, Bj, f);
-                const bool gen = on && (cc.general || (dd != 0 && dd != 1 && dd != -1));
-                const LevelPos pp = level_pos(lp, x);
-                uint32_t rows[8];
-                cell_rows(lp, pp.c, rows);
-                const float g0 = on ? gl[(slot0 + j) * (LJ * 512)] : 0.0f;
-                const float g1 = on ? gl[(slot0 + j) * (LJ * 512) + 64] : 0.0f;
+        for (int step = offsets ? 0 : 7; step < 9;) {
+            // (what derives from these is formed in each step rather than kept in
+            // registers across the flushes)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
+            for (int d = 0; d < 3; ++d)
+                asm volatile("" : "+v"(cc.pos.f[d]), "+v"(lo[d]), "+v"(P[d]));
+            const int gj = __ffs((int)general) - 1;
+            const int total = (int)st[step < 6 ? step : (step == 6 ? (second ? 12 : 6) + gj : 18)];
+            if (cursor + total > kPage) flush();
+            cursor += total;
+            // the wave's place in the page for its lanes' four pairs each
+            auto place = [&](bool put, uint64_t mask, const uint32_t r[4], const float v[8],
+                             uint32_t base) {
+                const int n_on = __popcll(mask);
+                const int b0 = __builtin_amdgcn_readfirstlane((int)base);
+                if (b0 + 4 * n_on > kPage) {   // more than counted
+                    if (lane == 0) status[1] = 1;
+                } else if (put) {
+                    const int at = b0 + (int)__builtin_amdgcn_mbcnt_hi(
+                                            (uint32_t)(mask >> 32),
+                                            __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        page_put(pg, at + i * n_on, r[i], v[2 * i], v[2 * i + 1]);
+                }
+            };
+            if (__builtin_expect(step == 6, 0)) {   // half a general evaluation
+                const CellClass cl = classify(a, lp, P, gj, B);
+                const bool in_b = on && cc.general && (cl.same || cl.adj) && !second;
+                const bool put = on && ((!cl.same && !cl.adj) || (in_b && cl.adj));
+                const float g0 = on ? go[gj * (LJ * 512) + lane] : 0.0f;
+                const float g1 = on ? go[gj * (LJ * 512) + 64 + lane] : 0.0f;
+                if (in_b) {   // corner t of B: corner t of the cell, or t across the face
+                    touched = true;
+                    float lo_w[3], hi_w[3];
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        const bool flip = cl.adj && cl.axis == d;
+                        lo_w[d] = flip ? cl.pos.f[d] : 1.0f - cl.pos.f[d];
+                        hi_w[d] = flip ? 1.0f - cl.pos.f[d] : cl.pos.f[d];
+                    }
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) {
+                        const float w = ((t & 1 ? hi_w[0] : lo_w[0]) * (t & 2 ? hi_w[1] : lo_w[1])) *
+                                        (t & 4 ? hi_w[2] : lo_w[2]);
+                        if (cl.same || ((t >> cl.axis) & 1) == (int)cl.up) {
+                            acc[2 * t] = __fmaf_rn(w, g0, acc[2 * t]);
+                            acc[2 * t + 1] = __fmaf_rn(w, g1, acc[2 * t + 1]);
+                        }
+                    }
+                }
+                const uint64_t mask = __ballot(put);
+                if (mask != 0) {   // half the cell's 8 corners, or its far face
+                    uint32_t base = 0;
+                    if (lane == 0) base = atomicAdd(&pg.cursor, (uint32_t)(4 * __popcll(mask)));
+                    uint32_t r[4];
                     float v[8];
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const float w = corner_weight(pp, 4 * h + i);
+                        const int t = cl.adj ? face_corner(i, cl.axis, cl.up) : (second ? 4 + i : i);
+                        r[i] = grid_row(lp, cl.pos.c[0] + (uint32_t)(t & 1),
+                                        cl.pos.c[1] + (uint32_t)(t >> 1 & 1),
+                                        cl.pos.c[2] + (uint32_t)(t >> 2));
+                        const float w = corner_weight(cl.pos, t);
                         v[2 * i] = w * g0;
                         v[2 * i + 1] = w * g1;
                     }
-                    int n_on, at;
-                    reserve(gen, n_on, at);
-                    if (gen) put4(at, n_on, rows + 4 * h, v);
+                    place(put, mask, r, v, base);
                 }
+                if (second) general &= general - 1u;
+                second = !second;
+                if (general == 0u) step = 7;
+                continue;
             }
-        }
-        // B: equal cells of neighbouring lanes merged, the head emits
-        bool end;
-        const bool head = cell_head(B, on && touched, &end);
-        merge_step<1>(p, acc, end);
-        merge_step<2>(p, acc, end);
-        merge_step<4>(p, acc, end);
-        merge_step<8>(p, acc, end);
+            // part 1: who puts pairs, and what goes into B
+            bool put = false, up = false;
+            float wfar[4], g0 = n0, g1 = n1;   // far face: weights and gradients
+            if (step < 6) {
+                if (step < 5 && on) {
+                    n0 = go[(step + 1) * (LJ * 512) + lane];
+                    n1 = go[(step + 1) * (LJ * 512) + 64 + lane];
+                }
+                auto near_faces = [&](auto axis) {
+                    constexpr int ax = decltype(axis)::value;
+                    constexpr int b = ax == 0 ? 1 : 0, e = ax == 2 ? 1 : 2;   // the other axes
+                    float f;
+                    const int dd = offset_cell(a, lp, P[ax], (step & 1) != 0, B[ax], f);
+                    const bool same = on && !cc.general && dd == 0;
+                    put = on && !cc.general && (dd == 1 || dd == -1);
+                    touched = touched || same || put;
+                    up = dd == 1;
+                    // weights of the corners on B's low and high faces (the far
+                    // face's are the other face's), as corner_weight forms them
+                    const float fl = same ? 1.0f - f : f, fh = same ? f : 1.0f - f;
+                    const float fb = cc.pos.f[b], fe = cc.pos.f[e];
+                    float wl[4], wh[4];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            int n_on, at;
-            if (reserve(head, n_on, at) && head) {
+                    for (int i = 0; i < 4; ++i) {
+                        const float vb = (i & 1) ? fb : 1.0f - fb, ve = (i & 2) ? fe : 1.0f - fe;
+                        wl[i] = ax == 2 ? (vb * ve) * fl : (fl * vb) * ve;
+                        wh[i] = ax == 2 ? (vb * ve) * fh : (fh * vb) * ve;
+                        wfar[i] = up ? wl[i] : wh[i];
+                    }
+                    if (same || (put && !up)) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int t = (i & 1) << b | (i >> 1) << e;
+                            acc[2 * t] = __fmaf_rn(wl[i], g0, acc[2 * t]);
+                            acc[2 * t + 1] = __fmaf_rn(wl[i], g1, acc[2 * t + 1]);
+                        }
+                    }
+                    if (same || (put && up)) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int t = (i & 1) << b | (i >> 1) << e | 1 << ax;
+                            acc[2 * t] = __fmaf_rn(wh[i], g0, acc[2 * t]);
+                            acc[2 * t + 1] = __fmaf_rn(wh[i], g1, acc[2 * t + 1]);
+                        }
+                    }
+                };
+                if (step < 2) near_faces(std::integral_constant<int, 0>());
+                else if (step < 4) near_faces(std::integral_constant<int, 1>());
+                else near_faces(std::integral_constant<int, 2>());
+            } else {
+                // B: equal cells of neighbouring lanes merged, the head emits
+                if (step == 7) {
+                    bool end;
+                    head = cell_head(B, on && touched, &end);
+                    merge_step<1>(p, acc, end);
+                    merge_step<2>(p, acc, end);
+                    merge_step<4>(p, acc, end);
+                    merge_step<8>(p, acc, end);
+                }
+                put = head;
+            }
+            // part 2: the wave's place in the page, rows and values
+            const uint64_t mask = __ballot(put);
+            if (mask != 0) {
+                uint32_t base = 0;
+                if (lane == 0) base = atomicAdd(&pg.cursor, (uint32_t)(4 * __popcll(mask)));
                 uint32_t r[4];
+                float v[8];
+                if (step < 6) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    r[i] = term_row(lp, (i & 1) ? lo[0] + mul[0] : lo[0],
-                                    (i & 2) ? lo[1] + mul[1] : lo[1],
-                                    h ? lo[2] + mul[2] : lo[2]);
-                put4(at, n_on, r, acc + 8 * h);
+                    for (int i = 0; i < 4; ++i) {
+                        v[2 * i] = wfar[i] * g0;
+                        v[2 * i + 1] = wfar[i] * g1;
+                    }
+                    if (step < 2)
+                        face_rows(lp, up ? lo[0] + 2u : lo[0] - 1u, lo[1], lo[1] + my, lo[2], lo[2] + mz, r);
+                    else if (step < 4)
+                        face_rows(lp, up ? lo[1] + 2u * my : lo[1] - my, lo[0], lo[0] + 1u, lo[2],
+                                  lo[2] + mz, r);
+                    else
+                        face_rows(lp, up ? lo[2] + 2u * mz : lo[2] - mz, lo[0], lo[0] + 1u, lo[1],
+                                  lo[1] + my, r);
+                } else {
+                    face_rows(lp, step == 8 ? lo[2] + mz : lo[2], lo[0], lo[0] + 1u, lo[1],
+                              lo[1] + my, r);
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) v[q] = step == 8 ? acc[8 + q] : acc[q];
+                }
+                place(put, mask, r, v, base);
+            }
+            if (step < 6) {
+                ++step;
+                if (step == 6 && general == 0u) step = 7;
+            } else {
+                ++step;
             }
         }
     }
@@ -563,13 +708,6 @@ __device__ __forceinline__ void corner_rows(const LevelParams& lp, const uint32_
                                             uint32_t rows[8]) {
     cell_rows(lp, cell, rows);
 }
-
-// Corner i (0..3) of the face of a cell with bit `ax` fixed to `b`.
-__device__ __forceinline__ int face_corner(int i, int ax, int b) {
-    const int low = i & ((1 << ax) - 1);
-    return low | (b << ax) | ((i >> ax) << (ax + 1));
-}
-
 
 // Position of cluster evaluation q (0..n-1) for this lane.
 template <int CL>
@@ -874,7 +1012,6 @@ void pairs_carve(WsCarver& c, const GeoArgs& a, const am_grid_desc* g, int64_t n
     PairHead h{};
     h.paged = table_paged(g);
     h.status = c.take<int64_t>(4);
-    size_t sb = 0;
     if (h.paged) {
         const int64_t blocks = ceil_div(n, 1024);
         h.units = blocks * a.active;
@@ -882,19 +1019,17 @@ void pairs_carve(WsCarver& c, const GeoArgs& a, const am_grid_desc* g, int64_t n
         h.steps = c.take<uint32_t>((size_t)h.units * kPairSteps + 1);
         h.unit_pages = c.take<uint64_t>((size_t)h.units + 1);
         h.unit_scan = c.take<uint64_t>((size_t)h.units + 1);
-        rocprim::exclusive_scan(nullptr, sb, (const uint64_t*)nullptr, (uint64_t*)nullptr,
-                                (uint64_t)0, (size_t)h.units + 1, rocprim::plus<uint64_t>(), 0,
-                                false);
     } else {
+        size_t sb = 0;
         h.entries = ceil_div(n, 16) * a.g.L;
         h.counts = c.take<int64_t>((size_t)h.entries + 1);
         h.offsets = c.take<int64_t>((size_t)h.entries + 1);
         rocprim::exclusive_scan(nullptr, sb, (const int64_t*)nullptr, (int64_t*)nullptr, (int64_t)0,
                                 (size_t)(h.entries > 0 ? h.entries : 1), rocprim::plus<int64_t>(),
                                 0, false);
+        h.scan_bytes = sb;
+        h.scan_tmp = c.take<char>(sb + 256);
     }
-    h.scan_bytes = sb;
-    h.scan_tmp = c.take<char>(sb + 256);
     *out = h;
 }
 
@@ -912,36 +1047,46 @@ static void count_launch(const GeoArgs& a, const float* pts, const float* randn,
                        (int64_t)0);
 }
 
+// Few sample blocks leave the chip idle: their levels are split over blocks
+// until there are two a CU (20 k samples: 49 -> 15 us; 65 k: 29 -> 14 us; at
+// 940 k, where nothing is split, 150 us).
+static unsigned page_count_split(int64_t blocks, int active) {
+    const int64_t want = ceil_div(512, blocks);
+    return (unsigned)(want < 1 ? 1 : (want > active ? (active > 0 ? active : 1) : want));
+}
+
 int pairs_count(const GeoArgs& a, int LJ, const float* pts, const float* randn, int64_t n,
                 const float* fdv, PairHead& h, hipStream_t s) {
     KernelTimer kt_("pair_count", s);
-    hipError_t e;
-    size_t sb = h.scan_bytes;
     if (h.paged) {
-        hipLaunchKernelGGL(k_page_count, dim3((unsigned)ceil_div(n, 1024)), dim3(1024), 0, s, a, pts,
-                           randn, n, fdv, h.centers, h.steps);
+        const int64_t blocks = ceil_div(n, 1024);
+        if (blocks > 0) {
+            hipLaunchKernelGGL(k_page_count, dim3((unsigned)blocks, page_count_split(blocks, a.active)),
+                               dim3(1024), 0, s, a, pts, randn, n, fdv, h.centers, h.steps);
+            AM_LAUNCH_CHECK();
+        }
+        if (h.units > 0) {
+            hipLaunchKernelGGL(k_unit_pages, dim3((unsigned)ceil_div(h.units, 256)), dim3(256), 0, s,
+                               h.steps, h.units, h.unit_pages);
+            AM_LAUNCH_CHECK();
+        }
+        hipLaunchKernelGGL(k_unit_scan, dim3(1), dim3(1024), 0, s, h.unit_pages, h.units,
+                           h.unit_scan, h.status);
         AM_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_unit_pages, dim3((unsigned)ceil_div(h.units + 1, 256)), dim3(256), 0, s,
-                           h.steps, h.units, h.unit_pages);
-        AM_LAUNCH_CHECK();
-        e = rocprim::exclusive_scan(h.scan_tmp, sb, h.unit_pages, h.unit_scan, (uint64_t)0,
-                                    (size_t)h.units + 1, rocprim::plus<uint64_t>(), s, false);
-    } else {
-        if (LJ == 2) count_launch<2>(a, pts, randn, n, fdv, h.counts, s);
-        else count_launch<4>(a, pts, randn, n, fdv, h.counts, s);
-        AM_LAUNCH_CHECK();
-        e = rocprim::exclusive_scan(h.scan_tmp, sb, h.counts, h.offsets, (int64_t)0,
-                                    (size_t)h.entries, rocprim::plus<int64_t>(), s, false);
+        return AM_OK;
     }
+    if (LJ == 2) count_launch<2>(a, pts, randn, n, fdv, h.counts, s);
+    else count_launch<4>(a, pts, randn, n, fdv, h.counts, s);
+    AM_LAUNCH_CHECK();
+    size_t sb = h.scan_bytes;
+    hipError_t e = rocprim::exclusive_scan(h.scan_tmp, sb, h.counts, h.offsets, (int64_t)0,
+                                           (size_t)h.entries, rocprim::plus<int64_t>(), s, false);
     if (e != hipSuccess) {
         set_error("pair-count scan failed: %s", hipGetErrorString(e));
         return AM_ERR_HIP;
     }
-    if (h.paged)
-        hipLaunchKernelGGL(k_page_status, dim3(1), dim3(64), 0, s, h.unit_scan, h.units, h.status);
-    else
-        hipLaunchKernelGGL(k_pair_total, dim3(1), dim3(64), 0, s, h.offsets, h.counts, h.entries,
-                           h.status);
+    hipLaunchKernelGGL(k_pair_total, dim3(1), dim3(64), 0, s, h.offsets, h.counts, h.entries,
+                       h.status);
     AM_LAUNCH_CHECK();
     return AM_OK;
 }
@@ -954,7 +1099,7 @@ static int pages_launch(const GeoArgs& a, int64_t n, const float* genc, PairHead
                                (int)sizeof(PageLds<VT>)));
     KernelTimer kt_("pair_emit", s);
     hipLaunchKernelGGL(kern, dim3((unsigned)h.units), dim3(kPageThreads), sizeof(PageLds<VT>), s, a,
-                       h.centers, n, ceil_div(n, 1024), genc, h.unit_scan, tp.pages, tp.keys,
+                       h.centers, n, ceil_div(n, 1024), genc, h.unit_scan, h.steps, tp.pages, tp.keys,
                        reinterpret_cast<VT*>(tp.vals), tp.run_start, h.status);
     AM_LAUNCH_CHECK();
     return AM_OK;
