@@ -90,7 +90,7 @@ __device__ __forceinline__ float dist_next_voxel(const MarchArgs& a, const float
     return fmaxf(t, 0.0f);
 }
 
-// ---- marching, G lanes to a ray ----
+// ---- marching, a wave to a ray ----
 // The rule for one ray (nerfacc 0.3.3): from t0 = near, t1 = t0 + step,
 // t_mid = (t0 + t1) / 2, while t_mid < far and fewer than cap samples (cap 0:
 // no cap): the midpoint's cell occupied -> a sample [t0, t1], then t0 = t1,
@@ -98,89 +98,131 @@ __device__ __forceinline__ float dist_next_voxel(const MarchArgs& a, const float
 // longer grows; unoccupied -> t_mid advances by whole steps to the next voxel
 // boundary (the ray ends when a step no longer advances t), t0 / t1 = t_mid
 // -/+ step / 2.
-// G lanes run it together.  From the group's state (t0, t1, t_mid, j), lane
-// g takes g occupied steps (the same IEEE sequence) and tests its midpoint,
-// so the group's grid loads are in flight together instead of one after
-// another.  The first lane whose state is out of range or unoccupied ends the
-// round: the lanes before it are the next samples; if it is in range, the
-// voxel skip runs from its midpoint.  Samples and counts are those of the
-// one-lane rule, bit for bit.  Outputs ts / te / ri may be null (count
-// only); every lane returns the count.
-template <int G>
-__device__ int march_group(const MarchArgs& a, const float* o, const float* d, float near,
-                           float far, const uint8_t* __restrict__ grid, float* __restrict__ ts,
-                           float* __restrict__ te, int32_t* __restrict__ ri, int32_t ray, int g,
-                           int gbase) {
-    static_assert(G >= 2 && G <= 16 && (64 % G) == 0, "a group is a power of two within a wave");
+// A wave runs it, so the grid loads of up to 64 points are in flight together
+// instead of one after another.  A round takes one of two forms, from the
+// state (t0, t1, t_mid, j):
+//   * inside: lane g takes g occupied steps and tests its midpoint.  The first
+//     lane whose state is out of range or unoccupied ends the run: the lanes
+//     before it are the next samples; if it is in range, the march goes on
+//     outside from its midpoint.
+//   * outside: the midpoints of a run of voxel skips all lie on the sequence
+//     s_0 = t_mid, s_k+1 = s_k + step.  Lane g holds s_g, tests it, and finds
+//     from its own skip target where the skip from s_g lands (`next`); the
+//     chain of skips from s_0 is then followed through the lanes, to the first
+//     midpoint that is occupied (inside from there), out of range or stuck (the
+//     ray ends), or whose skip leaves the lanes (the next round starts where it
+//     lands).
+// Both need the sequence x_0, x_k+1 = fl(x_k + step), and every lane its
+// element at once: within a binade an addition moves by the same d = fl(x_0 +
+// step) - x_0 (but for a tie), so lane k proposes fl(x_0 + k d), checks that
+// fl(its element + step) is the next lane's, and the round uses the lanes up to
+// the first that disagrees (one lane at least).
+// Samples and counts are those of the one-lane rule, bit for bit.  Outputs
+// ts / te / ri may be null (count only); every lane returns the count.
+// Latency-bound: a chain of rounds, a grid load and some hundred instructions
+// each, with few waves a CU.  2048 rays, 128^3 cells, steps of 0.43 cell: 43 us;
+// 16 lanes a ray, serial sequences: 141 us; 4 lanes and one skip a round: 355 us
+// (whole marching call with 256 / 8192 / 262144 rays: 45 / 91 / 695 us, against
+// 182 / 307 / 910 with 4 lanes).
+__device__ __forceinline__ float lane_float(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+__device__ __forceinline__ int march_wave(const MarchArgs& a, const float* o, const float* d,
+                                          float near, float far,
+                                          const uint8_t* __restrict__ grid,
+                                          float* __restrict__ ts, float* __restrict__ te,
+                                          int32_t* __restrict__ ri, int32_t ray) {
+    const int g = lane_id();
+    const float fg = (float)g;
     const float inv[3] = {1.0f / d[0], 1.0f / d[1], 1.0f / d[2]};
-    const float step = a.step;
-    const uint32_t mask = (1u << G) - 1u;
+    const float step = a.step, inv_step = 1.0f / step;
     float t0 = near;
     float t1 = t0 + step;
     float tm = (t0 + t1) * 0.5f;
     int j = 0;
+    bool inside = true;
     while (true) {
-        // this lane's state: g occupied steps ahead
-        float c0 = t0, c1 = t1, cm = tm;
-        bool alive = true;
-        for (int q = 0; q < g; ++q) {
-            const float prev = cm;
-            c0 = c1;
-            c1 = c0 + step;
-            cm = (c0 + c1) * 0.5f;
-            alive = alive && (cm > prev);
-        }
-        const bool cond = alive && cm < far && !(a.cap > 0 && j + g >= a.cap);
+        // this lane's element x of the sequence from t1 (inside: the end of its
+        // interval) or from t_mid, its predecessors, and the lanes that hold
+        const float base = inside ? t1 : tm;
+        const float delta = (base + step) - base;
+        const float x = __fmaf_rn(fg, delta, base);
+        const uint64_t agree = __ballot(x + step == __fmaf_rn(fg + 1.0f, delta, base));
+        const int hold = ~agree == 0 ? 64 : min(__builtin_ctzll(~agree) + 1, 64);
+        const float x1 = __fmaf_rn(fg - 1.0f, delta, base), x2 = __fmaf_rn(fg - 2.0f, delta, base);
+        const float c0 = g == 0 ? t0 : x1;
+        const float cm = !inside ? x : (g == 0 ? tm : (x1 + x) * 0.5f);
+        const bool alive = !inside || g == 0 || cm > (g == 1 ? tm : (x2 + x1) * 0.5f);
+        const bool cond = g < hold && alive && cm < far &&
+                          !(a.cap > 0 && j + (inside ? g : 0) >= a.cap);
         float xyz[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) xyz[k] = __fmaf_rn(cm, d[k], o[k]);
         const bool occ = cond && occupied(a, xyz, grid);
-        const uint32_t bo = (uint32_t)(__ballot(occ) >> gbase) & mask;
-        const uint32_t bc = (uint32_t)(__ballot(cond) >> gbase) & mask;
-        const int m = __builtin_ctz(~bo);   // first lane not an occupied in-range state (G: none)
-        if (g < m && ts) {
-            ts[j + g] = c0;
-            te[j + g] = c1;
-            if (ri) ri[j + g] = ray;
-        }
-        if (m == G) {   // all G were samples: continue from the last lane's successor
-            const float n0 = c1, n1 = n0 + step, nm = (n0 + n1) * 0.5f;
-            const int ok = nm > cm ? 1 : 0;
-            t0 = __shfl(n0, gbase + G - 1, 64);
-            t1 = __shfl(n1, gbase + G - 1, 64);
-            tm = __shfl(nm, gbase + G - 1, 64);
-            const int okg = __shfl(ok, gbase + G - 1, 64);
-            j += G;
-            if (!okg) break;
+        const uint64_t bo = __ballot(occ);
+        if (inside) {
+            // first lane that is not an occupied in-range state
+            const int m = ~bo == 0 ? 64 : __builtin_ctzll(~bo);
+            if (g < m && ts) {
+                ts[j + g] = c0;
+                te[j + g] = x;
+                if (ri) ri[j + g] = ray;
+            }
+            j += m;
+            if (m == hold) {   // all were samples: on from the last lane's successor
+                t0 = lane_float(x, hold - 1);
+                t1 = t0 + step;
+                tm = (t0 + t1) * 0.5f;
+                if (!(tm > lane_float(cm, hold - 1))) break;
+                continue;
+            }
+            if (!(__ballot(cond) >> m & 1u)) break;   // state m ends the march
+            // state m is in range and unoccupied: voxel skips from its midpoint
+            tm = lane_float(cm, m);
+            inside = false;
             continue;
         }
-        j += m;
-        if (!((bc >> m) & 1u)) break;   // state m ends the march
-        // state m is in range and unoccupied: the voxel skip from its midpoint
-        const float tmm = __shfl(cm, gbase + m, 64);
+        const float goal = x + dist_next_voxel(a, xyz, d, inv);
+        // the first element after x not below goal: about where it is, then exactly
+        int next = g + max(1, (int)fminf((goal - x) * inv_step, 64.0f));
+        while (next > g + 1 && !(__fmaf_rn((float)(next - 1), delta, base) < goal)) --next;
+        while (next < 64 && __fmaf_rn((float)next, delta, base) < goal) ++next;
+        // 0: skips to lane `next`; 1: occupied; 2: the ray ends; 3: skips past the lanes
+        const int kind = occ ? 1 : (!cond || !(x + step > x) ? 2 : (next < hold ? 0 : 3));
+        int hop = kind == 0 ? next : g;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) xyz[k] = __fmaf_rn(tmm, d[k], o[k]);
-        const float target = tmm + dist_next_voxel(a, xyz, d, inv);
-        float tt = tmm;
-        bool stuck = false;
-        do {
-            const float nt = tt + step;
-            if (!(nt > tt)) {
-                stuck = true;
-                break;
-            }
-            tt = nt;
-        } while (tt < target);
-        if (stuck) break;
-        tm = tt;
-        t0 = tm - step * 0.5f;
-        t1 = tm + step * 0.5f;
+        for (int q = 0; q < 6; ++q) hop = __shfl(hop, hop, 64);   // 64 skips
+        const int last = __builtin_amdgcn_readfirstlane(hop);
+        const int end = __builtin_amdgcn_readlane(kind, last);
+        if (end == 2) break;
+        if (end == 1) {
+            tm = lane_float(x, last);
+            t0 = tm - step * 0.5f;
+            t1 = tm + step * 0.5f;
+            inside = true;
+        } else {
+            // from the last element: below the target, or the skip's start
+            const float target = lane_float(goal, last);
+            float tt = lane_float(x, hold - 1);
+            bool stuck = false;
+            do {
+                const float nt = tt + step;
+                if (!(nt > tt)) {
+                    stuck = true;
+                    break;
+                }
+                tt = nt;
+            } while (tt < target);
+            if (stuck) break;
+            tm = tt;
+        }
     }
     return j;
 }
 
-// Lanes per ray of every marching kernel (8 measured no faster).
-constexpr int kMarchGroup = 4;
+// Lanes per ray of the background marching (8 measured no faster).
+constexpr int kMarchBgGroup = 4;
 
 // ---- background marching (nerfacc 0.3.3 ray_marching with
 // ContractionType.UN_BOUNDED_SPHERE and a cone angle, as called by
@@ -284,12 +326,12 @@ __global__ void __launch_bounds__(64) k_march_bg_count(MarchBgArgs b,
                                                       const uint8_t* __restrict__ grid,
                                                       int32_t* __restrict__ counts) {
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t i = tid / kMarchGroup;
-    const int g = (int)(tid % kMarchGroup);
+    const int64_t i = tid / kMarchBgGroup;
+    const int g = (int)(tid % kMarchBgGroup);
     if (i >= n) return;
     const float o[3] = {rays[6 * i], rays[6 * i + 1], rays[6 * i + 2]};
     const float d[3] = {rays[6 * i + 3], rays[6 * i + 4], rays[6 * i + 5]};
-    const int j = march_group_bg<kMarchGroup>(b, o, d, t_near[i], t_far[i], grid, nullptr, nullptr,
+    const int j = march_group_bg<kMarchBgGroup>(b, o, d, t_near[i], t_far[i], grid, nullptr, nullptr,
                                               nullptr, (int32_t)i, g, lane_id() - g);
     if (g == 0) counts[i] = j;
 }
@@ -303,8 +345,8 @@ __global__ void __launch_bounds__(64) k_march_bg_fill(MarchBgArgs b, const float
                                                      float* __restrict__ ts,
                                                      float* __restrict__ te) {
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t i = tid / kMarchGroup;
-    const int g = (int)(tid % kMarchGroup);
+    const int64_t i = tid / kMarchBgGroup;
+    const int g = (int)(tid % kMarchBgGroup);
     if (i >= n) return;
     const int32_t base = packed[2 * i];
     const float o[3] = {rays[6 * i], rays[6 * i + 1], rays[6 * i + 2]};
@@ -312,7 +354,7 @@ __global__ void __launch_bounds__(64) k_march_bg_fill(MarchBgArgs b, const float
     MarchBgArgs c = b;
     c.m.cap = packed[2 * i + 1];  // never write past the counted samples
     if (c.m.cap == 0) return;
-    march_group_bg<kMarchGroup>(c, o, d, t_near[i], t_far[i], grid, ts + base, te + base,
+    march_group_bg<kMarchBgGroup>(c, o, d, t_near[i], t_far[i], grid, ts + base, te + base,
                                 ridx + base, (int32_t)i, g, lane_id() - g);
 }
 
@@ -356,22 +398,19 @@ __global__ void k_ray_aabb(const float* __restrict__ rays, int64_t n, float aabb
     aabb_one(o, d, aabb, t_near + i, t_far + i);
 }
 
-__global__ void __launch_bounds__(64) k_march_count(MarchArgs a, const float* __restrict__ rays,
+__global__ void __launch_bounds__(256) k_march_count(MarchArgs a, const float* __restrict__ rays,
                                                    int64_t n, const float* __restrict__ t_near,
                                                    const float* __restrict__ t_far,
                                                    const float* __restrict__ jitter,
                                                    const uint8_t* __restrict__ grid,
                                                    int32_t* __restrict__ counts) {
-    const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t i = tid / kMarchGroup;
-    const int g = (int)(tid % kMarchGroup);
+    const int64_t i = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     if (i >= n) return;
     const float o[3] = {rays[6 * i], rays[6 * i + 1], rays[6 * i + 2]};
     const float d[3] = {rays[6 * i + 3], rays[6 * i + 4], rays[6 * i + 5]};
-    const int j = march_group<kMarchGroup>(a, o, d, ray_near(t_near, jitter, i, a.step), t_far[i],
-                                           grid, nullptr, nullptr, nullptr, (int32_t)i, g,
-                                           lane_id() - g);
-    if (g == 0) counts[i] = j;
+    const int j = march_wave(a, o, d, ray_near(t_near, jitter, i, a.step), t_far[i], grid, nullptr,
+                             nullptr, nullptr, (int32_t)i);
+    if (lane_id() == 0) counts[i] = j;
 }
 
 // packed[i] = (start, count) from counts and their exclusive scan; total.
@@ -385,7 +424,7 @@ __global__ void k_march_pack(const int32_t* __restrict__ counts, const int32_t* 
     if (i == n - 1) total[0] = starts[i] + counts[i];
 }
 
-__global__ void __launch_bounds__(64) k_march_fill(MarchArgs a, const float* __restrict__ rays,
+__global__ void __launch_bounds__(256) k_march_fill(MarchArgs a, const float* __restrict__ rays,
                                                   int64_t n, const float* __restrict__ t_near,
                                                   const float* __restrict__ t_far,
                                                   const float* __restrict__ jitter,
@@ -393,9 +432,7 @@ __global__ void __launch_bounds__(64) k_march_fill(MarchArgs a, const float* __r
                                                   const int32_t* __restrict__ packed,
                                                   int32_t* __restrict__ ridx,
                                                   float* __restrict__ ts, float* __restrict__ te) {
-    const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t i = tid / kMarchGroup;
-    const int g = (int)(tid % kMarchGroup);
+    const int64_t i = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     if (i >= n) return;
     const int32_t base = packed[2 * i];
     const float o[3] = {rays[6 * i], rays[6 * i + 1], rays[6 * i + 2]};
@@ -403,14 +440,14 @@ __global__ void __launch_bounds__(64) k_march_fill(MarchArgs a, const float* __r
     MarchArgs b = a;
     b.cap = packed[2 * i + 1];  // never write past the counted samples
     if (b.cap == 0) return;
-    march_group<kMarchGroup>(b, o, d, ray_near(t_near, jitter, i, a.step), t_far[i], grid,
-                             ts + base, te + base, ridx + base, (int32_t)i, g, lane_id() - g);
+    march_wave(b, o, d, ray_near(t_near, jitter, i, a.step), t_far[i], grid, ts + base, te + base,
+               ridx + base, (int32_t)i);
 }
 
 // Staged marching (a per-ray sample cap is set): the count pass also writes
 // each ray's samples into a cap-strided staging area, and the fill pass
 // copies them to their packed positions instead of marching again.
-__global__ void __launch_bounds__(64) k_march_count_staged(MarchArgs a,
+__global__ void __launch_bounds__(256) k_march_count_staged(MarchArgs a,
                                                           const float* __restrict__ rays, int64_t n,
                                                           const float* __restrict__ t_near,
                                                           const float* __restrict__ t_far,
@@ -419,17 +456,14 @@ __global__ void __launch_bounds__(64) k_march_count_staged(MarchArgs a,
                                                           int32_t* __restrict__ counts,
                                                           float* __restrict__ st0,
                                                           float* __restrict__ st1) {
-    const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t i = tid / kMarchGroup;
-    const int g = (int)(tid % kMarchGroup);
+    const int64_t i = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     if (i >= n) return;
     const float o[3] = {rays[6 * i], rays[6 * i + 1], rays[6 * i + 2]};
     const float d[3] = {rays[6 * i + 3], rays[6 * i + 4], rays[6 * i + 5]};
     const int64_t base = i * (int64_t)a.cap;   // a.cap > 0: samples j < cap
-    const int j = march_group<kMarchGroup>(a, o, d, ray_near(t_near, jitter, i, a.step), t_far[i],
-                                           grid, st0 + base, st1 + base, nullptr, (int32_t)i, g,
-                                           lane_id() - g);
-    if (g == 0) counts[i] = j;
+    const int j = march_wave(a, o, d, ray_near(t_near, jitter, i, a.step), t_far[i], grid,
+                             st0 + base, st1 + base, nullptr, (int32_t)i);
+    if (lane_id() == 0) counts[i] = j;
 }
 
 // One wave per ray: its staged samples to the packed outputs, coalesced.
@@ -541,10 +575,10 @@ extern "C" int am_march_count(const float* rays, int64_t n_rays, const float* t_
     char* stmp = c.take<char>(sb + 256);
     if (!c.ok()) return workspace_short(c.used, workspace_bytes);
     const MarchArgs a = march_args(roi6_host, grid, grid_res, step, cap);
-    const unsigned nb = (unsigned)ceil_div(n_rays * kMarchGroup, 64);
+    const unsigned nb = (unsigned)ceil_div(n_rays, 4);
     {
         KernelTimer kt_("march_count", s);
-        hipLaunchKernelGGL(k_march_count, dim3(nb), dim3(64), 0, s, a, rays, n_rays, t_near, t_far,
+        hipLaunchKernelGGL(k_march_count, dim3(nb), dim3(256), 0, s, a, rays, n_rays, t_near, t_far,
                            jitter, grid, counts);
     }
     AM_LAUNCH_CHECK();
@@ -572,7 +606,7 @@ extern "C" int am_march_fill(const float* rays, int64_t n_rays, const float* t_n
     const MarchArgs a = march_args(roi6_host, grid, grid_res, step, cap);
     {
         KernelTimer kt_("march_fill", to_stream(stream));
-        hipLaunchKernelGGL(k_march_fill, dim3((unsigned)ceil_div(n_rays * kMarchGroup, 64)), dim3(64), 0,
+        hipLaunchKernelGGL(k_march_fill, dim3((unsigned)ceil_div(n_rays, 4)), dim3(256), 0,
                            to_stream(stream), a, rays, n_rays, t_near, t_far, jitter, grid, packed,
                            ray_indices, t_starts, t_ends);
     }
@@ -619,7 +653,7 @@ extern "C" int am_march_count_staged(const float* rays, int64_t n_rays, const fl
     {
         KernelTimer kt_("march_count", s);
         hipLaunchKernelGGL(k_march_count_staged,
-                           dim3((unsigned)ceil_div(n_rays * kMarchGroup, 64)), dim3(64), 0, s, a,
+                           dim3((unsigned)ceil_div(n_rays, 4)), dim3(256), 0, s, a,
                            rays, n_rays, t_near, t_far, jitter, grid, counts, st0, st1);
     }
     AM_LAUNCH_CHECK();
@@ -688,7 +722,7 @@ extern "C" int am_march_bg_count(const float* rays, int64_t n_rays, const float*
     b.cone = cone_angle;
     {
         KernelTimer kt_("march_bg_count", s);
-        hipLaunchKernelGGL(k_march_bg_count, dim3((unsigned)ceil_div(n_rays * kMarchGroup, 64)),
+        hipLaunchKernelGGL(k_march_bg_count, dim3((unsigned)ceil_div(n_rays * kMarchBgGroup, 64)),
                            dim3(64), 0, s,
                            b, rays, n_rays, t_near, t_far, grid, counts);
     }
@@ -720,7 +754,7 @@ extern "C" int am_march_bg_fill(const float* rays, int64_t n_rays, const float* 
     b.cone = cone_angle;
     {
         KernelTimer kt_("march_bg_fill", to_stream(stream));
-        hipLaunchKernelGGL(k_march_bg_fill, dim3((unsigned)ceil_div(n_rays * kMarchGroup, 64)),
+        hipLaunchKernelGGL(k_march_bg_fill, dim3((unsigned)ceil_div(n_rays * kMarchBgGroup, 64)),
                            dim3(64), 0,
                            to_stream(stream), b, rays, n_rays, t_near, t_far, grid, packed,
                            ray_indices, t_starts, t_ends);
