@@ -13,13 +13,16 @@ static inline int field_blocks(int64_t n) {
 // Grids of the SDF forward and of the pair passes (count, emit); their
 // tiles' results do not depend on the grid.  Each is a whole number of
 // rounds of the blocks the device holds at once on 256 CUs (the register
-// counts of the fp32 16-level kernels): the forward two rounds of 512 (two
-// waves a SIMD), the emission two rounds of 768 (three), the count one
-// round of 2048 (eight); a partial last round measured slower.
-static constexpr int kFwdBlocksMax = 1024;
+// counts of the fp32 16-level kernels): the forward two rounds of 768 in the
+// difference form (three waves a SIMD; 1024 blocks: 3.2 ms where 1536 take 2.9),
+// of 512 in analytic mode, one of 2048 without gradient (262 k points: 148 us,
+// 1024 blocks 160); the emission two rounds of 768, the count one round of
+// 2048 (eight); a partial last round measured slower.
+static constexpr int kFwdBlocksNear = 1536;
+static constexpr int kFwdBlocksAnalytic = 1024;
+static constexpr int kFwdBlocksBase = 2048;
 static constexpr int kPairBlocksMax = 1536;
 static constexpr int kCountBlocksMax = 2048;
-static inline int fwd_blocks(int64_t n) { return persistent_blocks((n + 15) / 16, 4, kFwdBlocksMax); }
 static inline int pair_blocks(int64_t n) { return persistent_blocks((n + 15) / 16, 4, kPairBlocksMax); }
 // The backward passes of the SDF and radiance MLPs (over 200 VGPRs: two
 // waves a SIMD, 512 resident blocks) in one round; the grid fixes the

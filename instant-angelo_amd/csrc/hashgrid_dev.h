@@ -78,6 +78,32 @@ __device__ __forceinline__ void cell_rows(const LevelParams& lp, const uint32_t 
     }
 }
 
+// Four rows of a level from a corner face: terms a (fixed), b0 / b1 and c0 / c1
+// (x, or the products with the hash primes or strides; their order does not
+// matter).
+__device__ __forceinline__ void face_rows(const LevelParams& lp, uint32_t a, uint32_t b0,
+                                          uint32_t b1, uint32_t c0, uint32_t c1, uint32_t r[4]) {
+    if (lp.size_flags & kHashedBit) {
+        r[0] = a ^ b0 ^ c0;
+        r[1] = a ^ b1 ^ c0;
+        r[2] = a ^ b0 ^ c1;
+        r[3] = a ^ b1 ^ c1;
+    } else {
+        r[0] = a + b0 + c0;
+        r[1] = a + b1 + c0;
+        r[2] = a + b0 + c1;
+        r[3] = a + b1 + c1;
+    }
+    if (lp.size_flags & kPow2Bit) {
+        const uint32_t m = (lp.size_flags & kSizeMask) - 1u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] &= m;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = wrap_row(r[i], lp.size_flags);
+    }
+}
+
 // Cell and fractional position of x at one level.
 struct LevelPos {
     uint32_t c[3];
@@ -125,18 +151,15 @@ __device__ __forceinline__ float2 load_row2(const __half2* __restrict__ t, uint3
     return __half22float2(t[r]);
 }
 
-// Two-feature level encode (the configuration on the NeuS path).  Optionally
-// returns d enc_f / d x_d (including the level scale) for input gradients.
-template <bool WITH_DX, class TT>
-__device__ __forceinline__ void encode_level_f2(const LevelParams& lp, const float x[3],
-                                                const TT* __restrict__ table, float* out2,
-                                                float (*dx)[3]) {
-    const LevelPos p = level_pos(lp, x);
-    uint32_t rows[8];
-    cell_rows(lp, p.c, rows);
-    float2 v[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) v[c] = load_row2(table, rows[c]);
+__device__ __forceinline__ float2 row2(float2 v) { return v; }
+__device__ __forceinline__ float2 row2(__half2 v) { return __half22float2(v); }
+
+// Two-feature level encode (the configuration on the NeuS path) from the
+// cell's corner rows v[8].  Optionally returns d enc_f / d x_d (including the
+// level scale) for input gradients.
+template <bool WITH_DX>
+__device__ __forceinline__ void blend_level_f2(const LevelParams& lp, const LevelPos& p,
+                                               const float2 v[8], float* out2, float (*dx)[3]) {
     float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
@@ -160,6 +183,19 @@ __device__ __forceinline__ void encode_level_f2(const LevelParams& lp, const flo
             dx[1][d] = s1 * lp.scale;
         }
     }
+}
+
+template <bool WITH_DX, class TT>
+__device__ __forceinline__ void encode_level_f2(const LevelParams& lp, const float x[3],
+                                                const TT* __restrict__ table, float* out2,
+                                                float (*dx)[3]) {
+    const LevelPos p = level_pos(lp, x);
+    uint32_t rows[8];
+    cell_rows(lp, p.c, rows);
+    float2 v[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = load_row2(table, rows[c]);
+    blend_level_f2<WITH_DX>(lp, p, v, out2, dx);
 }
 
 }  // namespace am

@@ -304,32 +304,6 @@ __global__ void __launch_bounds__(1024) k_unit_scan(const uint64_t* __restrict__
     }
 }
 
-// Four rows of a level from a corner face: terms a (fixed), b0 / b1 and c0 / c1
-// (x, or the products with the hash primes or strides; their order does not
-// matter).
-__device__ __forceinline__ void face_rows(const LevelParams& lp, uint32_t a, uint32_t b0,
-                                          uint32_t b1, uint32_t c0, uint32_t c1, uint32_t r[4]) {
-    if (lp.size_flags & kHashedBit) {
-        r[0] = a ^ b0 ^ c0;
-        r[1] = a ^ b1 ^ c0;
-        r[2] = a ^ b0 ^ c1;
-        r[3] = a ^ b1 ^ c1;
-    } else {
-        r[0] = a + b0 + c0;
-        r[1] = a + b1 + c0;
-        r[2] = a + b0 + c1;
-        r[3] = a + b1 + c1;
-    }
-    if (lp.size_flags & kPow2Bit) {
-        const uint32_t m = (lp.size_flags & kSizeMask) - 1u;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] &= m;
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) r[i] = wrap_row(r[i], lp.size_flags);
-    }
-}
-
 // Emission: one block per unit collects the unit's pairs in an LDS page,
 // step by step (all lanes' far faces of one offset evaluation, at most 4096
 // pairs), and writes each page partitioned (page_flush).  The counted steps
