@@ -93,6 +93,9 @@ int64_t colsum_tmp_floats(int64_t rows, int64_t cols) {
     return slices > 1 ? slices * cols : 0;
 }
 
+// Column sums of a slice's rows, in row order.  A few blocks of one load chain a
+// lane: bound by latency, so 16 rows are loaded ahead of their additions (2048
+// partial rows of 3300 parameters, both stages: 24 -> 10 us).
 __global__ void k_colsum(const float* __restrict__ in, int64_t rows, int64_t cols, int64_t slice,
                          float* __restrict__ out) {
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -100,7 +103,15 @@ __global__ void k_colsum(const float* __restrict__ in, int64_t rows, int64_t col
     const int64_t r0 = (int64_t)blockIdx.y * slice;
     const int64_t r1 = r0 + slice < rows ? r0 + slice : rows;
     float s = 0.0f;
-    for (int64_t r = r0; r < r1; ++r) s += in[r * cols + c];
+    int64_t r = r0;
+    for (; r + 16 <= r1; r += 16) {
+        float v[16];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) v[q] = in[(r + q) * cols + c];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) s += v[q];
+    }
+    for (; r < r1; ++r) s += in[r * cols + c];
     out[(int64_t)blockIdx.y * cols + c] = s;
 }
 
