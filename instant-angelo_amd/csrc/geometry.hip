@@ -711,76 +711,33 @@ __host__ __device__ inline int geo_ext_base(const GeoArgs& a) {
     return (a.lds_floats + 4 * 128 * mlp::kScratchLd + 3) & ~3;
 }
 
-// Only the base evaluation has gradients of all output rows; the offset
-// evaluations' have the SDF row alone.  With one hidden layer in the difference
-// form (kSplitOut) their output layer is vector arithmetic: gh = Wo[0, :] gf, and
-// a lane sums gf h of its own sample and hidden rows in G.dWo over the tile's
-// evaluations, where 32 of an evaluation's 164 MFMAs and a transpose through LDS
-// multiplied by zeros.  Once a tile, those sums go into row 0 of the dWo tile,
-// which accumulates in a wave-private LDS area, [4 column tiles][64 lanes] v4f:
-// the large terms of a difference's two sides cancel before they meet it.
-// 940 k samples, 16 levels: backward kernel 3.09 -> 2.86 ms; 65 k, 8 levels:
-// 191 -> 167 us.  (Two hidden layers: the LDS area would not fit beside the
-// feature rows'.)
-template <int NH, bool AN>
-constexpr bool kSplitOut = NH == 1 && !AN;
-enum OutForm { kOutWhole, kOutTile, kOutRow };   // G.dWo holds the tile; LDS does; the SDF row
-constexpr int kOutTileFloats = 4 * 64 * 4;
-
 // Output-gradient tile with only row 0 (the SDF) set.
 __device__ __forceinline__ v4f go_row0(float g) {
     const int k = lane_id() >> 4;
     return v4f{k == 0 ? g : 0.0f, 0.0f, 0.0f, 0.0f};
 }
 
-// dWo tile in LDS += go (x) x over the tile's samples.
-__device__ __forceinline__ void out_tile_dw(v4f go, const v4f x[4], float* scratch,
-                                            float* out_tile) {
-    const int l = lane_id();
-    v4f dw[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) dw[t] = *reinterpret_cast<const v4f*>(out_tile + (t * 64 + l) * 4);
-    mlp::mm_dw<1, 4, 16, mlp::FragV, mlp::kF32>(&go, mlp::FragV{x}, scratch, dw);
-#pragma unroll
-    for (int t = 0; t < 4; ++t) *reinterpret_cast<v4f*>(out_tile + (t * 64 + l) * 4) = dw[t];
-}
-
 // MLP backward of one evaluation with output gradient `go` (D tile rows =
 // outputs): accumulates weight gradients, stores the encode gradient of the
 // lane's level slots to genc (the slot's place of genc_lane) and, with DX,
 // returns the contracted-position gradient (summed over the 4 lane groups).
-// OUT, kOutRow: go[0] is the SDF row's gradient of the lane's sample.
-template <int LJ, int NH, bool DX, int PR, OutForm OUT>
+template <int LJ, int NH, bool DX, int PR>
 __device__ __forceinline__ void geo_eval_bwd(const GeoArgs& a, const float* sm,
                                              const GeoEval<LJ, NH, DX>& e, v4f go,
                                              float* scratch, GeoGrad<LJ, NH>& G, float* genc,
-                                             float gpos[3], const OutExt* ext = nullptr,
-                                             float* out_tile = nullptr) {
+                                             float gpos[3], const OutExt* ext = nullptr) {
     constexpr int KS1 = GeoDims<LJ>::KS1, IT1 = GeoDims<LJ>::IT1;
     const int l = lane_id(), k = l >> 4;
     v4f h[4], dh[4];   // last hidden activation and its derivative
     const v4f* zl = NH == 2 ? e.z2 : e.z1;
 #pragma unroll
     for (int t = 0; t < 4; ++t) mlp::act_fb4(a.act, zl[t], a.beta, h[t], dh[t]);
+    mlp::mm_dw<1, 4, 16, mlp::FragV, PR>(&go, mlp::FragV{h}, scratch, G.dWo);
+    G.dbo += go;
     v4f gh[4];
-    if constexpr (OUT == kOutRow) {
-        sdf_row_tiles(a, sm, gh);
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                G.dWo[t][r] = __fmaf_rn(go[0], h[t][r], G.dWo[t][r]);
-                gh[t][r] *= go[0];
-            }
-        G.dbo += go_row0(go[0]);
-    } else {
-        if constexpr (OUT == kOutTile) out_tile_dw(go, h, scratch, out_tile);
-        else mlp::mm_dw<1, 4, 16, mlp::FragV, PR>(&go, mlp::FragV{h}, scratch, G.dWo);
-        G.dbo += go;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) gh[t] = v4f{0, 0, 0, 0};
-        mlp::mm_bwd_in<4, 4, mlp::FragV, PR>(sm + a.wo, kWLd, mlp::FragV{&go}, gh);
-    }
+    for (int t = 0; t < 4; ++t) gh[t] = v4f{0, 0, 0, 0};
+    mlp::mm_bwd_in<4, 4, mlp::FragV, PR>(sm + a.wo, kWLd, mlp::FragV{&go}, gh);
     if constexpr (NH == 2)
         if (ext) out_ext_bwd(a, sm, h, *ext, scratch, gh);
     if constexpr (NH == 2) {
@@ -1003,11 +960,6 @@ __device__ __forceinline__ void geo_bwd_body(
     const int ext_floats = NH == 2 ? (a.out_tiles - 1) * kOutExtFloats : 0;
     float* ext_acc = sm + geo_ext_base(a) + wave * ext_floats;
     for (int q = l; q < ext_floats; q += 64) ext_acc[q] = 0.0f;
-    constexpr bool SPLIT = kSplitOut<NH, AN>;
-    constexpr OutForm kRow = SPLIT ? kOutRow : kOutWhole;
-    float* out_tile = SPLIT ? sm + geo_ext_base(a) + wave * kOutTileFloats : nullptr;
-    if constexpr (SPLIT)
-        for (int q = l; q < kOutTileFloats; q += 64) out_tile[q] = 0.0f;
     mlp::wave_sync();
     const int64_t n_tiles = (N + 15) / 16;
     const int fdim = a.n_out + 3;
@@ -1060,13 +1012,9 @@ __device__ __forceinline__ void geo_bwd_body(
             geo_eval_b<LJ, NH, false, ST, mlp::kF32>(a, sm, lv, table, store, tile, n_tiles, 0, 0,
                                                      s.x0, e);
             const OutExt ext{g_feature, m, fdim, valid, ext_acc};
-            geo_eval_bwd<LJ, NH, false, mlp::kF32, SPLIT ? kOutTile : kOutWhole>(
-                a, sm, e, go, scratch, G, genc, nullptr,
-                                                   a.out_tiles > 1 ? &ext : nullptr, out_tile);
+            geo_eval_bwd<LJ, NH, false, mlp::kF32>(a, sm, e, go, scratch, G, genc, nullptr,
+                                                   a.out_tiles > 1 ? &ext : nullptr);
         }
-        if constexpr (SPLIT)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) G.dWo[t] = v4f{0, 0, 0, 0};
         if (a.with_laplace) {
             const float gl = (valid && g_laplace) ? g_laplace[m] : 0.0f;
             const float lo = -1.0f + 1e-6f, hi = 1.0f - 1e-6f;
@@ -1093,9 +1041,8 @@ __device__ __forceinline__ void geo_bwd_body(
                 geo_eval_b<LJ, NH, true, ST, mlp::kF32>(a, sm, lv, table, store, tile, n_tiles,
                                                         a.curv0 + j, a.dx_curv0 + j, x, e);
                 float gpos[3];
-                const v4f gt = SPLIT ? v4f{gf, 0.0f, 0.0f, 0.0f} : go_row0(gf);
-                geo_eval_bwd<LJ, NH, true, mlp::kF32, kRow>(a, sm, e, gt, scratch, G,
-                                                             genc + (a.curv0 + j) * LJ * 512, gpos);
+                geo_eval_bwd<LJ, NH, true, mlp::kF32>(a, sm, e, go_row0(gf), scratch, G,
+                                                      genc + (a.curv0 + j) * LJ * 512, gpos);
 #pragma unroll
                 for (int d = 0; d < 3; ++d)
                     if (inb[d]) g_ps[d] += gpos[d] * a.inv2r;
@@ -1135,11 +1082,9 @@ __device__ __forceinline__ void geo_bwd_body(
                 GeoEval<LJ, NH, false> e;
                 geo_eval_b<LJ, NH, false, ST, mlp::kF32>(a, sm, lv, table, store, tile, n_tiles,
                                                          1 + j, 0, x, e);
-                const v4f gt = SPLIT ? v4f{gf, 0.0f, 0.0f, 0.0f} : go_row0(gf);
-                geo_eval_bwd<LJ, NH, false, mlp::kF32, kRow>(a, sm, e, gt, scratch, G,
-                                                              genc + (1 + j) * LJ * 512, nullptr);
+                geo_eval_bwd<LJ, NH, false, mlp::kF32>(a, sm, e, go_row0(gf), scratch, G,
+                                                       genc + (1 + j) * LJ * 512, nullptr);
             }
-            if constexpr (SPLIT) out_tile_dw(go_row0(1.0f), G.dWo, scratch, out_tile);
         }
     }
     // per-wave partial gradient row in parameter layout
@@ -1164,11 +1109,6 @@ __device__ __forceinline__ void geo_bwd_body(
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     out[a.pw2 + (16 * ot + 4 * k + r) * 64 + 16 * it + i] = G.dW2[ot * 4 + it][r];
-    }
-    if constexpr (SPLIT) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            G.dWo[t] = *reinterpret_cast<const v4f*>(out_tile + (t * 64 + l) * 4);
     }
 #pragma unroll
     for (int it = 0; it < 4; ++it)
@@ -1483,9 +1423,7 @@ static int geo_bwd_launch_t(const GeoArgs& a, const am_grid_desc* g, const float
     // the backward proper: MLP parameter partials and the encode gradients
     auto launch_bwd = [&]() -> int {
         const size_t lds =
-            (size_t)(geo_ext_base(a) + 4 * (a.out_tiles - 1) * kOutExtFloats +
-                     (NH == 1 && !a.analytic ? 4 * kOutTileFloats : 0)) *
-            sizeof(float);
+            (size_t)(geo_ext_base(a) + 4 * (a.out_tiles - 1) * kOutExtFloats) * sizeof(float);
         AM_CHECK_ARG(lds <= 160 * 1024, "geometry backward needs %zu bytes of LDS", lds);
         auto kern = k_geo_bwd_o2<LJ, true, PR, false>;   // the type of every form's kernel
         if constexpr (NH == 1) {
