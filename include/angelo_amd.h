@@ -67,8 +67,11 @@ int am_timer_units(const char* name, int64_t* units);
  * (default 0): 1 makes am_sdf_bwd add its merged pairs into the table
  * gradient with float atomics (no host read; the summation order
  * varies run to run; measured 3x slower than the pair reduction on a
- * 0.87 M-sample step).  Unknown names return
- * AM_ERR_INVALID. */
+ * 0.87 M-sample step).  "sdf_bwd_count_shift" (default 0, for tests; at most
+ * 64 either way): adds this to one count of am_sdf_bwd's paged form (levels
+ * of at most 2^21 rows), so that the emission's check reports it
+ * (am_sdf_bwd_check).
+ * Unknown names return AM_ERR_INVALID. */
 int am_set_flag(const char* name, int32_t value);
 
 /* ------------------------------------------------------------------------ */

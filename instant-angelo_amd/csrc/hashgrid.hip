@@ -209,7 +209,7 @@ __global__ void __launch_bounds__(kPageThreads) k_hg_pages(
             page_put(pg, c * np + q, rows[c], w * g0, w * g1);
         }
     }
-    page_flush(pg, 8 * np, (lp.size_flags & kSizeMask) <= (uint32_t)kSpreadDigits * kRows, blockIdx.x,
+    page_flush(pg, 8 * np, nullptr, (lp.size_flags & kSizeMask) <= (uint32_t)kSpreadDigits * kRows, blockIdx.x,
                keys, vals, run_start);
 }
 

@@ -71,9 +71,12 @@ __device__ __forceinline__ uint32_t page_value(const PageLds<uint32_t>& s, int i
 // pairs in runs of 16 equal rows: reduce 0.80 -> 0.34 ms).  The second
 // features move after the others, to hold few registers beside the caller's.
 // Bound by LDS operations.  Called by all kPageThreads threads; leaves the
-// page empty.
+// page empty.  mismatch (null: n is what was put): set to 1 when the pairs put
+// (cursor) are not the n counted; only pairs that were both put and counted are
+// written then.
 template <class VT>
-__device__ __forceinline__ void page_flush(PageLds<VT>& s, int n, bool spread, int64_t page,
+__device__ __forceinline__ void page_flush(PageLds<VT>& s, int n, int64_t* __restrict__ mismatch,
+                                           bool spread, int64_t page,
                                            uint32_t* __restrict__ keys, VT* __restrict__ vals,
                                            uint16_t* __restrict__ run_start) {
     constexpr int kItems = kPage / kPageThreads;
@@ -81,6 +84,11 @@ __device__ __forceinline__ void page_flush(PageLds<VT>& s, int n, bool spread, i
     asm volatile("" : "+v"(tid));   // keeps its addresses out of the caller's loop registers
     uint32_t key[kItems], at[kItems], first[kItems];   // first: words[0]
     __syncthreads();
+    if (mismatch) {
+        const int put = __builtin_amdgcn_readfirstlane((int)s.cursor);
+        if (put != n && tid == 0) *mismatch = 1;
+        n = put < n ? put : n;
+    }
 #pragma unroll
     for (int k = 0; k < kItems; ++k) {
         const int i = tid + kPageThreads * k;

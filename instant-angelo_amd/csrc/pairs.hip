@@ -355,7 +355,7 @@ __global__ void __launch_bounds__(1024) k_pair_pages(GeoArgs a, const float* __r
     const bool spread = (lp.size_flags & kSizeMask) <= (uint32_t)kSpreadDigits * kRows;
     auto flush = [&]() {
         if (page < page_end)
-            page_flush(pg, cursor, spread, page, keys, vals, run_start);
+            page_flush(pg, cursor, status + 1, spread, page, keys, vals, run_start);
         else
             __syncthreads();
         ++page;
@@ -1013,6 +1013,23 @@ int64_t pairs_bound(const GeoArgs& a, const PairHead& h, int LJ, int64_t n) {
     return h.units * (lane_pairs(a) * 1024 / (kPage - 4096) + 1);
 }
 
+// Moves one count (flag "sdf_bwd_count_shift"), so that a test can see the
+// emission's check of the counts.  The emission never passes its page's end,
+// however many pairs were counted.
+__global__ void k_shift_count(uint32_t* count, int by) {
+    const int c = (int)*count + by;
+    *count = c < 0 ? 0u : (uint32_t)c;
+}
+
+static int shift_count(uint32_t* count, hipStream_t s) {
+    const int by = flag_value("sdf_bwd_count_shift", 0);
+    if (by == 0) return AM_OK;
+    AM_CHECK_ARG(by >= -64 && by <= 64, "sdf_bwd_count_shift %d", by);
+    hipLaunchKernelGGL(k_shift_count, dim3(1), dim3(1), 0, s, count, by);
+    AM_LAUNCH_CHECK();
+    return AM_OK;
+}
+
 template <int LJ>
 static void count_launch(const GeoArgs& a, const float* pts, const float* randn, int64_t n,
                          const float* fdv, int64_t* counts, hipStream_t s) {
@@ -1040,6 +1057,8 @@ int pairs_count(const GeoArgs& a, int LJ, const float* pts, const float* randn, 
             AM_LAUNCH_CHECK();
         }
         if (h.units > 0) {
+            // (the base cluster's centre cells of the first unit)
+            if (int rc = shift_count(h.steps + 2 * kClusterSteps - 1, s)) return rc;
             hipLaunchKernelGGL(k_unit_pages, dim3((unsigned)ceil_div(h.units, 256)), dim3(256), 0, s,
                                h.steps, h.units, h.unit_pages);
             AM_LAUNCH_CHECK();
