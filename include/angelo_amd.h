@@ -70,7 +70,8 @@ int am_timer_units(const char* name, int64_t* units);
  * 0.87 M-sample step).  "sdf_bwd_count_shift" (default 0, for tests; at most
  * 64 either way): adds this to one count of am_sdf_bwd's paged form (levels
  * of at most 2^21 rows), so that the emission's check reports it
- * (am_sdf_bwd_check).
+ * (am_sdf_bwd_check).  "sdf_bwd_page_cut" (default 0, for tests): takes that
+ * many pages off the paged form's arrays, which reports it the same way.
  * Unknown names return AM_ERR_INVALID. */
 int am_set_flag(const char* name, int32_t value);
 

@@ -1329,18 +1329,23 @@ static int carve_pairs(WsCarver& c, const GeoArgs& a, const am_grid_desc* g, con
                        int64_t capacity, TablePages* tp, TableReduceWs* tw) {
     const bool half = a.prec == AM_PREC_MIXED;
     if (!h.paged) return table_reduce_carve(c, g, capacity, tw, half);
+    const int64_t cut = flag_value("sdf_bwd_page_cut", 0);   // (tests)
+    if (cut > 0) capacity = capacity > cut ? capacity - cut : 0;
     table_pages_carve(c, capacity, half, tp);
     return AM_OK;
 }
 
-// Consistency flags of recent backward calls.  The emit pass flags a tile
-// whose pairs differ from the count pass's; instead of a stream sync per
-// call, each call copies its flag into a pinned host slot behind an event,
-// and later calls (after their own pair-count sync, cheaply) and
-// am_sdf_bwd_check read the slots whose copies have landed.  Every emitted
-// pair stays inside its tile's reserved range and the sort and reduce only
-// index rows below n_entries and items below the count whatever the keys
-// hold, so a mismatch gives a wrong dtable, never a stray access.
+// Consistency flags of recent backward calls.  The emission flags a page
+// (sorted form: a tile) whose pairs are not as many as the count pass found;
+// instead of a stream sync per call, each call copies its flag into a pinned
+// host slot behind an event, and later calls (after their own pair-count sync,
+// cheaply) and am_sdf_bwd_check read the slots whose copies have landed.  A
+// mismatch gives a wrong dtable, never a stray access: pairs stay inside their
+// page, which holds only pairs put and counted, every page that the reduction
+// walks has its run table and lies inside the arrays, and rows are taken modulo
+// the bucket (sorted form: pairs stay inside their tile's reserved range, and
+// the sort and reduce only index rows below n_entries and items below the
+// count whatever the keys hold).
 namespace {
 struct FlagSlot {
     hipEvent_t ev = nullptr;

@@ -176,6 +176,11 @@ __device__ __forceinline__ void page_flush(PageLds<VT>& s, int n, int64_t* __res
     __syncthreads();
 }
 
+// A page without pairs (one that the emission did not reach).
+__device__ __forceinline__ void page_empty(int64_t page, uint16_t* __restrict__ run_start) {
+    if ((int)threadIdx.x <= kMaxDigits) run_start[page * kRunStride + threadIdx.x] = 0;
+}
+
 // Levels of at most this many buckets spread their runs.
 constexpr int kSpreadDigits = 96;
 

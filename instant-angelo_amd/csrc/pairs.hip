@@ -337,6 +337,7 @@ __global__ void __launch_bounds__(1024) k_pair_pages(GeoArgs a, const float* __r
     const int64_t page_end = (int64_t)(scan[unit + 1] >> 40);
     if (page_end == page0) return;
     if (page_end > capacity) {   // never past the arrays
+        for (int64_t q = page0; q < capacity; ++q) page_empty(q, run_start);
         if (tid == 0) status[1] = 1;
         return;
     }
@@ -599,7 +600,10 @@ __global__ void __launch_bounds__(1024) k_pair_pages(GeoArgs a, const float* __r
         }
     }
     if (cursor > 0) flush();
-    if (tid == 0 && page != page_end) status[1] = 1;
+    if (page != page_end) {   // (the page rule on the same steps: not reached)
+        for (; page < page_end; ++page) page_empty(page, run_start);
+        if (tid == 0) status[1] = 1;
+    }
 }
 
 // ---- sorted and atomic forms ----

@@ -519,14 +519,17 @@ __device__ __forceinline__ int level_digits(const TableLevels& t, int l) {
     return (int)((t.offset[l + 1] - t.offset[l] + (uint32_t)kRows - 1u) >> kRowBits);
 }
 
-// One wave, lane = level: page bounds, slices and work units.
+// One wave, lane = level: page bounds (never past the arrays), slices and work
+// units.
 __global__ void k_page_plan(TableLevels t, const uint64_t* __restrict__ scan, int64_t units,
-                            int active, int64_t per_level, PagePlan* __restrict__ plan) {
+                            int active, int64_t per_level, int64_t capacity,
+                            PagePlan* __restrict__ plan) {
     const int l = threadIdx.x;
     const bool on = l < t.L;
     auto first_page = [&](int q) -> int64_t {
         if (q > active) q = active;
-        return scan ? (int64_t)(scan[q * units] >> 40) : q * per_level;
+        const int64_t p = scan ? (int64_t)(scan[q * units] >> 40) : q * per_level;
+        return p < capacity ? p : capacity;
     };
     const int64_t p = on ? first_page(l) : 0, n = on ? (first_page(l + 1) - p) * kPage : 0;
     const int64_t total = first_page(t.L) * kPage;
@@ -804,7 +807,7 @@ void table_pages_carve(WsCarver& c, int64_t pages, bool half_vals, TablePages* o
 int table_pages_plan(TablePages& w, const am_grid_desc* g, const uint64_t* scan, int64_t units,
                      int active, int64_t per_level, hipStream_t s) {
     hipLaunchKernelGGL(k_page_plan, dim3(1), dim3(64), 0, s, table_levels(g), scan, units, active,
-                       per_level, w.plan);
+                       per_level, w.pages, w.plan);
     AM_LAUNCH_CHECK();
     return AM_OK;
 }
