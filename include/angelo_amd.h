@@ -69,7 +69,7 @@ int am_timer_units(const char* name, int64_t* units);
  * varies run to run; measured 3x slower than the pair reduction on a
  * 0.87 M-sample step).  "sdf_bwd_count_shift" (default 0, for tests; at most
  * 64 either way): adds this to one count of am_sdf_bwd's paged form (levels
- * of at most 2^21 rows), so that the emission's check reports it
+ * of at most 2^21 rows, one after another), so that the emission's check reports it
  * (am_sdf_bwd_check).  "sdf_bwd_page_cut" (default 0, for tests): takes that
  * many pages off the paged form's arrays, which reports it the same way.
  * Unknown names return AM_ERR_INVALID. */

@@ -2,17 +2,18 @@
 // backward kernel -> one write per row of the table gradient, rows without a
 // pair written 0, the same bits on every run.
 //
-// Paged form (two features a row, at most 2^21 rows a level: every grid of
-// the workloads).  The emitting kernels collect the pairs of one level in
-// LDS, a page at a time, and write each page partitioned by its pairs' bucket
-// of 2^13 rows, with a table of where each bucket's run starts; one block per
-// bucket then gathers its runs from the level's pages and adds them up in
-// LDS.  The additions are exact (see k_page_reduce), so their order does not
-// matter.  Every pair is written once and its value read once.
+// Paged form (two features a row, at most 2^21 rows a level, the levels one
+// after another: every grid of the workloads).  The emitting kernels collect
+// the pairs of one level in LDS, a page at a time, and write each page
+// partitioned by its pairs' bucket of 2^13 rows, with a table of where each
+// bucket's run starts; one block per bucket then gathers its runs from the
+// level's pages and adds them up in LDS.  The additions are exact (see
+// k_page_reduce), so their order does not matter.  Every pair is written once
+// and its value read once.
 //
-// Sorted form (other feature counts, larger levels): stable radix sort of the
-// pairs by row, then a fixed-order segmented reduce.  Two-feature tables sort
-// only the key bits above `begin_bit`: the pairs of each bucket of
+// Sorted form (other feature counts, larger levels, other layouts): stable
+// radix sort of the pairs by row, then a fixed-order segmented reduce.
+// Two-feature tables sort only the key bits above `begin_bit`: the pairs of each bucket of
 // 2^begin_bit rows are then contiguous and in emission order, and one wave
 // per bucket finishes the job with an in-wave stable split sort and a
 // segmented scan into per-row accumulators in LDS.

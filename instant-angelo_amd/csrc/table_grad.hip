@@ -19,11 +19,20 @@ static int64_t bucket_slots(int64_t m) { return 2 * (m / kUnitItems) + 1; }
 constexpr int64_t kUnitMost = 1 << 19;
 constexpr int64_t kUnitLeast = 16384;
 
+// The buckets of a level are written whole and row 0 on to n_entries by the
+// levels together, so the levels must follow one another as am_grid_init lays
+// them; descriptors with gaps, shared rows or another order take the sorted
+// form, which knows rows alone.
 bool table_paged(const am_grid_desc* g) {
     if (g->n_features != 2) return false;
-    for (int l = 0; l < g->n_levels; ++l)
-        if (g->size[l] > (uint32_t)kMaxDigits * kRows) return false;
-    return true;
+    uint64_t next = 0;
+    for (int l = 0; l < g->n_levels; ++l) {
+        if (g->offset[l] != next || g->size[l] == 0u ||
+            g->size[l] > (uint32_t)kMaxDigits * kRows)
+            return false;
+        next += g->size[l];
+    }
+    return next == g->n_entries;
 }
 
 TableLevels table_levels(const am_grid_desc* g) {
