@@ -1331,7 +1331,7 @@ static int carve_pairs(WsCarver& c, const GeoArgs& a, const am_grid_desc* g, con
     if (!h.paged) return table_reduce_carve(c, g, capacity, tw, half);
     const int64_t cut = flag_value("sdf_bwd_page_cut", 0);   // (tests)
     if (cut > 0) capacity = capacity > cut ? capacity - cut : 0;
-    table_pages_carve(c, capacity, half, tp);
+    table_pages_carve(c, g, capacity, half, tp);
     return AM_OK;
 }
 

@@ -219,7 +219,7 @@ static int hg_bwd_pages(const GridArgs& ga, const am_grid_desc* g, const float* 
     const int64_t per_level = ceil_div(n, kPagePoints);
     WsCarver c(ws, ws_bytes);
     TablePages w;
-    table_pages_carve(c, per_level * active, false, &w);
+    table_pages_carve(c, g, per_level * active, false, &w);
     if (!c.ok()) return workspace_short(c.used, ws_bytes);
     const size_t lds = sizeof(PageLds<uint2>);
     AM_HIP(hipFuncSetAttribute((const void*)k_hg_pages, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -232,8 +232,7 @@ static int hg_bwd_pages(const GridArgs& ga, const am_grid_desc* g, const float* 
     }
     AM_LAUNCH_CHECK();
     timer_units("encode_table_pairs", n * active * 8);
-    if (int rc = table_pages_plan(w, g, nullptr, 0, active, per_level, s)) return rc;
-    return table_pages_run(w, g, dtable, s);
+    return table_pages_run(w, g, nullptr, 0, active, per_level, dtable, s);
 }
 
 template <int F>
@@ -360,7 +359,7 @@ extern "C" size_t am_hashgrid_bwd_workspace_size(const am_grid_desc* g, int64_t 
     WsCarver c(nullptr, 0);
     if (table_paged(g)) {
         TablePages w;
-        table_pages_carve(c, ceil_div(n, kPagePoints) * active_levels, false, &w);
+        table_pages_carve(c, g, ceil_div(n, kPagePoints) * active_levels, false, &w);
         return c.used + 256;
     }
     TableReduceWs w;

@@ -1144,8 +1144,7 @@ int pairs_reduce(const GeoArgs& a, int LJ, const am_grid_desc* g, const float* p
                          : pages_launch<4, uint2>(a, n, genc, h, tp, s);
         if (rc) return rc;
     }
-    rc = table_pages_plan(tp, g, h.unit_scan, ceil_div(n, 1024), a.active, 0, s);
-    return rc ? rc : table_pages_run(tp, g, dtable, s);
+    return table_pages_run(tp, g, h.unit_scan, ceil_div(n, 1024), a.active, 0, dtable, s);
 }
 
 int pairs_atomic(const GeoArgs& a, int LJ, const float* pts, const float* randn, int64_t n,

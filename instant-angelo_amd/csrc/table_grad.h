@@ -62,21 +62,41 @@ struct TableReduceWs {
     bool half_vals;  // values are ValsH<F> instead of Vals<F>
 };
 
-// Rows of the levels: level l owns [offset[l], offset[l + 1]).
+// Rows of the levels: level l owns [offset[l], offset[l + 1]).  Its buckets:
+// from bucket[l] on, n_buckets in all.
 struct TableLevels {
     int32_t L;
     uint32_t offset[AM_MAX_LEVELS + 1];
+    int32_t bucket[AM_MAX_LEVELS];
+    int32_t n_buckets;
 };
 TableLevels table_levels(const am_grid_desc* g);
 
-// What the reduction reads of the pages (made on the device, so that no host
-// read is needed).
+// What the reduction does (made on the device from the pages' run tables, so
+// that no host read is needed).
 struct PagePlan {
-    int32_t page_base[AM_MAX_LEVELS + 1];   // first page of each level
-    int32_t unit_base[AM_MAX_LEVELS + 1];   // first work unit of each level (finest level first)
-    int32_t slices[AM_MAX_LEVELS];          // slices of each of the level's buckets
-    int32_t slot_base[AM_MAX_LEVELS];       // first partial slot of a sliced level
-    int32_t row_base[AM_MAX_LEVELS + 1];    // first combined row of a sliced level
+    int32_t n_units, n_merges;
+};
+// A bucket's pairs, or (slices > 1) those of every slices-th page, the slice-th
+// on.
+struct __attribute__((aligned(32))) PageUnit {
+    int64_t page;            // the first of them
+    int32_t runs, slices;    // pages, and from one to the next
+    int32_t bucket;          // within its level
+    uint32_t row, rows;      // the bucket's first row, and how many
+    int32_t slot;            // partial slot (slices > 1)
+};
+
+// Where the pages of each level begin, on the device: the level's `units`
+// emitting blocks' exclusive scan (high 24 bits: pages), unit = level * units +
+// block, levels from `active` on empty; or (scan == nullptr) `per_level` pages
+// for each of the `active` levels.  Never past the arrays' `capacity`.
+struct PageSource {
+    const uint64_t* scan;
+    int64_t units;
+    int32_t active;
+    int64_t per_level;
+    int64_t capacity;
 };
 
 struct TablePages {
@@ -85,21 +105,22 @@ struct TablePages {
     void* vals;          // the same: float2, or half2 (half_vals)
     uint16_t* run_start; // [pages][kRunStride]
     double2* partial;    // [slots][8192 rows] sums of sliced buckets
+    int32_t chunks;      // parts of a level's pages counted by a block each (0: few pages)
+    uint32_t* pairs;     // [chunks][n_buckets] pairs of the buckets
     PagePlan* plan;
+    PageUnit* units;     // [max_units]
+    PageUnit* merges;    // [n_buckets] those of several slices, or of no pair (slices 0)
+    int64_t max_units;
     bool half_vals;
 };
 
 // Whether the paged form takes the grid.
 bool table_paged(const am_grid_desc* g);
-void table_pages_carve(WsCarver& c, int64_t pages, bool half_vals, TablePages* out);
-// Where the pages of each level begin: the level's `units` emitting blocks'
-// exclusive scan (high 24 bits: pages), unit = level * units + block, levels
-// from `active` on empty; or (scan == nullptr) `per_level` pages for each of
-// the `active` levels.
-int table_pages_plan(TablePages& w, const am_grid_desc* g, const uint64_t* scan, int64_t units,
-                     int active, int64_t per_level, hipStream_t s);
-// Reduces the pages; dtable [n_entries, 2] fully overwritten.
-int table_pages_run(TablePages& w, const am_grid_desc* g, float* dtable, hipStream_t s);
+void table_pages_carve(WsCarver& c, const am_grid_desc* g, int64_t pages, bool half_vals,
+                       TablePages* out);
+// Reduces the pages (of PageSource); dtable [n_entries, 2] fully overwritten.
+int table_pages_run(TablePages& w, const am_grid_desc* g, const uint64_t* scan, int64_t units,
+                    int active, int64_t per_level, float* dtable, hipStream_t s);
 
 // ---- sorted form ----
 // Bucket bits of the bucketed form: the low key bits left unsorted (at most

@@ -13,11 +13,22 @@ constexpr int64_t kUnitItems = 16384;   // sorted items per work unit (256 chunk
 static int64_t bucket_slots(int64_t m) { return 2 * (m / kUnitItems) + 1; }
 
 // ---- paged form ----
-// Pairs of a work unit: a level's buckets are cut into slices of about this
-// many pairs where they hold more (coarse levels), fewer when the whole
-// gradient makes less than about 1024 units of the most.
+// Pairs of a work unit: a bucket of more than half as many again is cut into
+// slices of about this many, a 1216th of all pairs between the two bounds: with
+// what the buckets round up, just under five rounds of 256 blocks.  Fewer, longer
+// units end raggedly; one more than a round starts another; more units write
+// and merge more partial sums.  Reduce and merge with 768 / 960 / 1024 / 1216 /
+// 1440 / 2048 units: 940 k samples, 16 levels 1930 / 1925 / 1911 / 1827 / 1760 /
+// 1776 us; 480 k, 4 levels 576 / 584 / 667 / 586 / 659 / 774; 240 k, 16 levels
+// of 2^19 rows 438 / 469 / - / 420 / 441 / -.  65 k samples, 8 levels, with
+// 16384 / 32768 pairs at least: 133 / 95 us.
 constexpr int64_t kUnitMost = 1 << 19;
-constexpr int64_t kUnitLeast = 16384;
+constexpr int64_t kUnitLeast = 32768;
+constexpr int64_t kUnits = 1216;
+__host__ __device__ inline int64_t unit_pairs(int64_t total) {
+    const int64_t u = total / kUnits;
+    return u < kUnitLeast ? kUnitLeast : (u > kUnitMost ? kUnitMost : u);
+}
 
 // The buckets of a level are written whole and row 0 on to n_entries by the
 // levels together, so the levels must follow one another as am_grid_init lays
@@ -42,21 +53,20 @@ TableLevels table_levels(const am_grid_desc* g) {
         t.offset[l] = g->offset[l];
         t.offset[l + 1] = g->offset[l] + g->size[l];
     }
+    for (int l = 0; l < g->n_levels; ++l) {
+        t.bucket[l] = t.n_buckets;
+        t.n_buckets += (int32_t)ceil_div(g->size[l], kRows);
+    }
     return t;
 }
 
-// Units of sliced levels: a level of n pairs and D buckets has
-// S = ceil(n / (D U)) slices, D S <= 2 n / U where S > 1.
-static int64_t slot_bound(int64_t m) {
-    const int64_t a = 2 * (m / kUnitLeast), b = 2 * (m / kUnitMost);
-    return (a < 2048 ? a : (b > 2048 ? b : 2048)) + 2;
+// At most n / U for the unit U of any number n of pairs up to m.
+static int64_t units_of(int64_t m) {
+    const int64_t a = m / kUnitLeast, b = m / kUnitMost;
+    return (a < kUnits ? a : (b > kUnits ? b : kUnits)) + 1;
 }
-
-static int64_t table_digits(const am_grid_desc* g) {
-    int64_t d = 0;
-    for (int l = 0; l < g->n_levels; ++l) d += ceil_div(g->size[l], kRows);
-    return d;
-}
+// A sliced bucket of n > 1.5 U pairs has S = ceil(n / U) <= 1.5 n / U slices.
+static int64_t slot_bound(int64_t m) { return 3 * units_of(m) / 2 + 1; }
 
 int table_key_bits(uint32_t n_entries) {
     int b = 1;
@@ -528,54 +538,162 @@ __device__ __forceinline__ int level_digits(const TableLevels& t, int l) {
     return (int)((t.offset[l + 1] - t.offset[l] + (uint32_t)kRows - 1u) >> kRowBits);
 }
 
-// One wave, lane = level: page bounds (never past the arrays), slices and work
-// units.
-__global__ void k_page_plan(TableLevels t, const uint64_t* __restrict__ scan, int64_t units,
-                            int active, int64_t per_level, int64_t capacity,
-                            PagePlan* __restrict__ plan) {
-    const int l = threadIdx.x;
-    const bool on = l < t.L;
-    auto first_page = [&](int q) -> int64_t {
-        if (q > active) q = active;
-        const int64_t p = scan ? (int64_t)(scan[q * units] >> 40) : q * per_level;
-        return p < capacity ? p : capacity;
-    };
-    const int64_t p = on ? first_page(l) : 0, n = on ? (first_page(l + 1) - p) * kPage : 0;
-    const int64_t total = first_page(t.L) * kPage;
-    int64_t unit = total / 1024;
-    unit = unit < kUnitLeast ? kUnitLeast : (unit > kUnitMost ? kUnitMost : unit);
-    const int D = on ? level_digits(t, l) : 0;
-    int64_t S = on ? (n + D * unit - 1) / (D * unit) : 0;
-    if (on && S < 1) S = 1;
-    const uint32_t all = (uint32_t)(D * S);
-    const uint32_t slots = S > 1 ? all : 0u;
-    const uint32_t rows = S > 1 ? t.offset[l + 1] - t.offset[l] : 0u;   // combined afterwards
-    const uint32_t us = wave_scan(all), ss = wave_scan(slots), rs = wave_scan(rows);
-    const uint32_t sum = __shfl(us, 63, 64);
-    if (on) {
-        plan->page_base[l] = (int32_t)p;
-        // finest level first: its buckets hold the most pairs
-        plan->unit_base[l] = (int32_t)(sum - us);
-        plan->slices[l] = (int32_t)S;
-        plan->slot_base[l] = (int32_t)(ss - slots);
-        plan->row_base[l] = (int32_t)(rs - rows);
-        if (l == t.L - 1) {
-            plan->page_base[l + 1] = (int32_t)(p + n / kPage);
-            plan->row_base[l + 1] = (int32_t)rs;
+__device__ __forceinline__ int64_t first_page(const PageSource& src, int level) {
+    const int q = level < src.active ? level : src.active;
+    const int64_t p = src.scan ? (int64_t)(src.scan[q * src.units] >> 40) : q * src.per_level;
+    return p < src.capacity ? p : src.capacity;
+}
+
+constexpr int kMostChunks = 16;
+
+// Pairs of each bucket in a part of its level's pages, from the run tables.
+// Block (part, level); 1024 threads: the buckets, four pages at a time.
+__global__ void __launch_bounds__(1024) k_bucket_pairs(TableLevels t, PageSource src,
+                                                       const uint16_t* __restrict__ run_start,
+                                                       uint32_t* __restrict__ pairs) {
+    __shared__ uint32_t part[4][kMaxDigits];
+    const int l = (int)blockIdx.y, d = (int)threadIdx.x & (kMaxDigits - 1), q = (int)threadIdx.x >> 8;
+    const int64_t p0 = first_page(src, l), np = first_page(src, l + 1) - p0;
+    const int64_t a = p0 + np * blockIdx.x / gridDim.x, b = p0 + np * (blockIdx.x + 1) / gridDim.x;
+    const int D = level_digits(t, l);
+    uint32_t sum = 0;
+    if (d < D) {
+#pragma unroll 8
+        for (int64_t p = a + q; p < b; p += 4) {
+            const uint16_t* rs = run_start + p * kRunStride + d;
+            sum += (uint32_t)rs[1] - (uint32_t)rs[0];
         }
-        if (l == 0) plan->unit_base[t.L] = (int32_t)sum;
+    }
+    part[q][d] = sum;
+    __syncthreads();
+    if (q == 0 && d < D)
+        pairs[(int64_t)blockIdx.x * t.n_buckets + t.bucket[l] + d] =
+            (part[0][d] + part[1][d]) + (part[2][d] + part[3][d]);
+}
+
+// Exclusive sum over the block's 1024 threads, and the total.
+__device__ __forceinline__ uint64_t block_scan(uint64_t v, uint64_t* wave_sum, uint64_t* total) {
+    const int tid = (int)threadIdx.x;
+    uint64_t incl = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint64_t o = __shfl_up((unsigned long long)incl, d, 64);
+        if ((tid & 63) >= d) incl += o;
+    }
+    if ((tid & 63) == 63) wave_sum[tid >> 6] = incl;
+    __syncthreads();
+    uint64_t at = incl - v, all = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        if (w < tid >> 6) at += wave_sum[w];
+        all += wave_sum[w];
+    }
+    __syncthreads();
+    *total = all;
+    return at;
+}
+
+// The work units: each bucket's pairs cut into slices by its own load, so that
+// samples that crowd in few cells are spread over the chip like any others.
+// With slices by the level's mean load the fullest bucket of a fine level was
+// one block's: 940 k samples within 0.002 of a point, 2^21 rows a level, reduce
+// 7.6 -> 3.3 ms, within 0.1: 2.76 -> 2.52; 2 M points of the stand-alone grid
+// within 0.4 % of the box 29.5 -> 5.3 ms.  Spread samples pay 5 to 10 us for
+// the counts (20 k samples: 85 -> 90 us in all).  Buckets without pairs have no
+// unit; the merge writes their zeros.
+__global__ void __launch_bounds__(1024) k_page_plan(TableLevels t, PageSource src,
+                                                    const uint16_t* __restrict__ run_start,
+                                                    const uint32_t* __restrict__ pairs, int chunks,
+                                                    PagePlan* __restrict__ plan,
+                                                    PageUnit* __restrict__ units,
+                                                    PageUnit* __restrict__ merges) {
+    constexpr int kMost = AM_MAX_LEVELS * kMaxDigits;
+    __shared__ uint64_t n[kMost + 1];   // pairs, then the scan
+    __shared__ uint64_t wave_sum[16];
+    const int tid = (int)threadIdx.x, each = (t.n_buckets + 1023) / 1024;
+    // four waves to a level, whose parameters are scalars
+    const int quarter = __builtin_amdgcn_readfirstlane(tid >> 8), d = tid & (kMaxDigits - 1);
+    uint64_t sum = 0, total;
+    if (chunks > 0) {
+        for (int i = tid; i < t.n_buckets; i += 1024) {
+            uint64_t v = 0;
+#pragma unroll
+            for (int c = 0; c < kMostChunks; ++c)
+                v += c < chunks ? pairs[(int64_t)c * t.n_buckets + i] : 0u;
+            n[i] = v;
+            sum += v;
+        }
+    } else {   // few pages: from the run tables themselves
+        for (int l = quarter; l < t.L; l += 4) {
+            if (d >= level_digits(t, l)) continue;
+            const int64_t p1 = first_page(src, l + 1);
+            uint64_t v = 0;
+            for (int64_t p = first_page(src, l); p < p1; ++p) {
+                const uint16_t* rs = run_start + p * kRunStride + d;
+                v += (uint32_t)rs[1] - (uint32_t)rs[0];
+            }
+            n[t.bucket[l] + d] = v;
+            sum += v;
+        }
+    }
+    block_scan(sum, wave_sum, &total);
+    const uint64_t U = (uint64_t)unit_pairs((int64_t)total);
+    // units | partial slots << 24 | merges << 48
+    auto counts = [&](uint64_t m) -> uint64_t {
+        if (m != 0u && m <= U + U / 2u) return 1u;
+        const uint64_t S = m >> 32 ? (m + U - 1u) / U
+                                   : (uint32_t)m / (uint32_t)U + ((uint32_t)m % (uint32_t)U != 0u);
+        return S | S << 24 | 1ull << 48;
+    };
+    const int i0 = tid * each < t.n_buckets ? tid * each : t.n_buckets;
+    const int i1 = i0 + each < t.n_buckets ? i0 + each : t.n_buckets;
+    uint64_t mine = 0;
+    for (int i = i0; i < i1; ++i) mine += n[i] = counts(n[i]);
+    uint64_t at = block_scan(mine, wave_sum, &total);
+    for (int i = i0; i < i1; ++i) {
+        const uint64_t c = n[i];
+        n[i] = at;
+        at += c;
+    }
+    if (tid == 0) {
+        n[t.n_buckets] = total;
+        plan->n_units = (int32_t)(total & 0xffffffu);
+        plan->n_merges = (int32_t)(total >> 48);
+    }
+    __syncthreads();
+    for (int l = quarter; l < t.L; l += 4) {
+        if (d >= level_digits(t, l)) continue;
+        const uint64_t a = n[t.bucket[l] + d], b = n[t.bucket[l] + d + 1];
+        const int64_t p0 = first_page(src, l);
+        const int pages = (int)(first_page(src, l + 1) - p0), first = (int)(a & 0xffffffu);
+        const uint32_t left = t.offset[l + 1] - t.offset[l] - (uint32_t)d * kRows;
+        PageUnit w;
+        w.slices = (int)(b & 0xffffffu) - first;
+        w.bucket = d;
+        w.row = t.offset[l] + (uint32_t)d * kRows;
+        w.rows = left < (uint32_t)kRows ? left : (uint32_t)kRows;
+        w.page = p0;
+        w.slot = (int)(a >> 24 & 0xffffffu);
+        w.runs = 0;
+        if (a >> 48 != b >> 48) merges[a >> 48] = w;
+        for (int q = 0; q < w.slices; ++q) {   // every slices-th page from the q-th on
+            w.runs = (pages - q + w.slices - 1) / w.slices;
+            units[first + q] = w;
+            ++w.page;
+            ++w.slot;
+        }
     }
 }
 
-// Runs of one bucket in pages [p0, p1) of a level: a wave takes every 16th
-// page.  Its lanes look 64 runs up at once; each run is read by the whole
+// Runs of one bucket in every step-th page of a level: a wave takes every 16th
+// of them.  Its lanes look 64 runs up at once; each run is read by the whole
 // wave, 64 pairs a load, eight runs' loads in flight together.  body.load(base,
 // i): pair base + i of the arrays (base is the same for the wave);
 // body.use(payload).  Returns the pairs of the runs that this lane looked up.
 struct RunSpan {
-    const uint16_t* run_start;   // the level's first page, at the bucket
-    int64_t first;               // the level's first pair
-    int p0, p1;
+    const uint16_t* run_start;   // the first page, at the bucket
+    int64_t first;               // the first page's first pair
+    int runs, step;              // pages, and from one to the next
 };
 
 template <class Body>
@@ -583,15 +701,17 @@ __device__ __forceinline__ uint32_t for_runs(const RunSpan& s, const Body& body)
     constexpr int kU = 8;
     const uint32_t lane = threadIdx.x & 63u;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int64_t apart = (int64_t)s.step * (16 * kPage);   // a wave's runs
     uint32_t total = 0;
-    for (int b = s.p0 + wave; b < s.p1; b += 16 * 64) {
+    for (int b = wave; b < s.runs; b += 16 * 64) {
         const int mine = b + 16 * (int)lane;
         uint32_t both = 0;   // two neighbouring 16-bit entries: start, end
-        if (mine < s.p1) __builtin_memcpy(&both, s.run_start + (int64_t)mine * kRunStride, 4);
+        if (mine < s.runs)
+            __builtin_memcpy(&both, s.run_start + (int64_t)mine * s.step * kRunStride, 4);
         total += (both >> 16) - (both & 0xffffu);
-        const int runs = (s.p1 - b + 15) / 16 < 64 ? (s.p1 - b + 15) / 16 : 64;
+        const int runs = (s.runs - b + 15) / 16 < 64 ? (s.runs - b + 15) / 16 : 64;
         for (int q = 0; q < runs; q += kU) {
-            const int64_t base0 = s.first + (int64_t)(b + 16 * q) * kPage;
+            int64_t base0 = s.first + (int64_t)b * s.step * kPage + q * apart;
             uint32_t st[kU], len[kU];
             typename Body::Payload v[kU];
             bool longer = false;
@@ -601,17 +721,19 @@ __device__ __forceinline__ uint32_t for_runs(const RunSpan& s, const Body& body)
                 st[u] = d & 0xffffu;
                 len[u] = (d >> 16) - st[u];
                 longer = longer || len[u] > 64u;
-                if (lane < len[u]) v[u] = body.load(base0 + (int64_t)(u * 16 * kPage) + st[u], lane);
+                if (lane < len[u]) v[u] = body.load(base0 + st[u], lane);
+                base0 += apart;
             }
 #pragma unroll
             for (int u = 0; u < kU; ++u)
                 if (lane < len[u]) body.use(v[u]);
             if (!longer) continue;
+            base0 -= kU * apart;
 #pragma unroll 1
-            for (int u = 0; u < kU; ++u) {
+            for (int u = 0; u < kU; ++u, base0 += apart) {
                 const uint32_t d = (uint32_t)__builtin_amdgcn_readlane((int)both, (q + u) & 63);
                 const uint32_t n = (d >> 16) - (d & 0xffffu);
-                const int64_t base = base0 + (int64_t)(u * 16 * kPage) + (d & 0xffffu);
+                const int64_t base = base0 + (d & 0xffffu);
                 for (uint32_t j = 64; j < n; j += 256) {
                     typename Body::Payload w[4];
 #pragma unroll
@@ -698,8 +820,8 @@ __device__ __forceinline__ double row_sum(unsigned long long a, uint32_t e, int 
     return ldexp((double)(long long)a, (int)e - 126 - Q);
 }
 
-// One block per work unit: a bucket of 8192 rows, or a slice of its level's
-// pages.  Two passes over the bucket's runs: the largest exponent of each
+// One block per work unit: a bucket of 8192 rows, or every S-th page's part of
+// it.  Two passes over the bucket's runs: the largest exponent of each
 // row (LDS max over the key words), then the values, as whole
 // numbers of their row's grid, added into 64-bit integers in LDS.  With at
 // most 2^b pairs in the unit, the grid is 2^-Q of the row's largest binade,
@@ -711,8 +833,8 @@ __device__ __forceinline__ double row_sum(unsigned long long a, uint32_t e, int 
 // 1024 threads and 144 KB of LDS (the first pass's maxima lie where the sums
 // go, and are packed to 16 bits a row before the second): one block a CU.
 template <class VT>
-__global__ void __launch_bounds__(1024) k_page_reduce(TableLevels t,
-                                                      const PagePlan* __restrict__ plan,
+__global__ void __launch_bounds__(1024) k_page_reduce(const PagePlan* __restrict__ plan,
+                                                      const PageUnit* __restrict__ units,
                                                       const uint32_t* __restrict__ keys,
                                                       const VT* __restrict__ vals,
                                                       const uint16_t* __restrict__ run_start,
@@ -727,18 +849,13 @@ __global__ void __launch_bounds__(1024) k_page_reduce(TableLevels t,
     // runs share cache lines
     const int bx = (int)blockIdx.x & 7, by = (int)blockIdx.x >> 3;
     const int u = ((by >> 5) * 8 + bx) * 32 + (by & 31);
-    if (u >= plan->unit_base[t.L]) return;
-    int l = t.L - 1;
-    while (l > 0 && u >= plan->unit_base[l - 1]) --l;
-    const int D = level_digits(t, l), S = plan->slices[l];
-    const int v = u - plan->unit_base[l];
-    const int slice = v / D, d = v - slice * D;
-    const int pb = plan->page_base[l], np = plan->page_base[l + 1] - pb;
+    if (u >= plan->n_units) return;
+    const PageUnit w = units[u];
     RunSpan s;
-    s.run_start = run_start + (int64_t)pb * kRunStride + d;
-    s.first = (int64_t)pb * kPage;
-    s.p0 = (int)((int64_t)np * slice / S);
-    s.p1 = (int)((int64_t)np * (slice + 1) / S);
+    s.run_start = run_start + w.page * kRunStride + w.bucket;
+    s.first = w.page * kPage;
+    s.step = w.slices;
+    s.runs = w.runs;
     for (int q = tid; q < 2 * kRows; q += 1024) mx[q] = 0u;
     if (tid == 0) pairs = 0u;
     __syncthreads();
@@ -760,48 +877,89 @@ __global__ void __launch_bounds__(1024) k_page_reduce(TableLevels t,
     if (special) for_runs(s, RunAdd<VT, true>{keys, vals, ex, acc, ck});
     else for_runs(s, RunAdd<VT, false>{keys, vals, ex, acc, ck});
     __syncthreads();
-    const uint32_t rows = t.offset[l + 1] - t.offset[l];
-    double2* dst = partial + ((int64_t)(plan->slot_base[l] + d * S + slice) << kRowBits);
+    double2* dst = partial + ((int64_t)w.slot << kRowBits);
+    float2* row = reinterpret_cast<float2*>(out) + w.row;
 #pragma unroll
     for (int r = 0; r < kRows / 1024; ++r) {
         const int q = tid + 1024 * r;
+        if ((uint32_t)q >= w.rows) continue;
         const uint32_t e = ex[q];
         const double x = row_sum(acc[q], e & 255u, Q), y = row_sum(acc[kRows + q], e >> 8, Q);
-        const uint32_t row = (uint32_t)d * kRows + q;
-        if (S > 1) dst[q] = make_double2(x, y);
-        else if (row < rows)
-            *reinterpret_cast<float2*>(out + 2 * ((int64_t)t.offset[l] + row)) =
-                make_float2((float)x, (float)y);
+        if (w.slices > 1) dst[q] = make_double2(x, y);
+        else row[q] = make_float2((float)x, (float)y);
     }
 }
 
-// Sliced levels: each row is the sum of its slices' partials in order.
-__global__ void __launch_bounds__(256) k_page_combine(TableLevels t,
-                                                      const PagePlan* __restrict__ plan,
-                                                      const double2* __restrict__ partial,
-                                                      float* __restrict__ out) {
-    const uint32_t all = (uint32_t)plan->row_base[t.L];
-    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < all; i += gridDim.x * 256u) {
-        int l = 0;
-        while (i >= (uint32_t)plan->row_base[l + 1]) ++l;
-        const uint32_t q = i - (uint32_t)plan->row_base[l];
-        const int S = plan->slices[l];
-        const double2* src = partial +
-                             ((int64_t)(plan->slot_base[l] + (int)(q >> kRowBits) * S) << kRowBits) +
-                             (q & (uint32_t)(kRows - 1));
-        double a = 0.0, b = 0.0;
-#pragma unroll 4
-        for (int j = 0; j < S; ++j) {
-            const double2 p = src[(int64_t)j << kRowBits];
-            a += p.x;
-            b += p.y;
+// Buckets of several slices: each row is the sum of its slices' partials, in
+// one order for a number of slices; buckets without pairs: zeros.  A block
+// takes 512 rows; from 8 slices on, 64 rows at a time by four waves, a quarter
+// of the slices each (a single level of 72 rows with 16 M pairs, where hundreds
+// of slices meet: backward 596 -> 383 us).
+__global__ void __launch_bounds__(256) k_page_merge(const PagePlan* __restrict__ plan,
+                                                    const PageUnit* __restrict__ merges,
+                                                    const double2* __restrict__ partial,
+                                                    float* __restrict__ out) {
+    constexpr int kPart = 512;
+    __shared__ double2 sums[4][64];
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int all = plan->n_merges * (kRows / kPart);
+    for (int e = (int)blockIdx.x; e < all; e += (int)gridDim.x) {
+        const PageUnit m = merges[e / (kRows / kPart)];
+        const int slices = m.slices, q0 = e % (kRows / kPart) * kPart;   // row within the bucket
+        const int n = min((int)m.rows - q0, kPart);
+        float2* dst = reinterpret_cast<float2*>(out) + m.row + q0;
+        const double2* src = partial + ((int64_t)m.slot << kRowBits) + q0;
+        if (slices < 8) {
+            for (int q = tid; q < n; q += 256) {
+                double2 p[7];
+#pragma unroll
+                for (int j = 0; j < 7; ++j)
+                    if (j < slices) p[j] = src[((int64_t)j << kRowBits) + q];
+                double2 sum = make_double2(0.0, 0.0);
+#pragma unroll
+                for (int j = 0; j < 7; ++j)
+                    if (j < slices) {
+                        sum.x += p[j].x;
+                        sum.y += p[j].y;
+                    }
+                dst[q] = make_float2((float)sum.x, (float)sum.y);
+            }
+            continue;
         }
-        *reinterpret_cast<float2*>(out + 2 * ((int64_t)t.offset[l] + q)) =
-            make_float2((float)a, (float)b);
+        for (int q = 0; q < n; q += 64) {
+            double2 sum = make_double2(0.0, 0.0);
+            if (q + lane < n)
+                for (int j0 = wave; j0 < slices; j0 += 32) {
+                    double2 p[8];
+#pragma unroll
+                    for (int c = 0; c < 8; ++c)
+                        if (j0 + 4 * c < slices)
+                            p[c] = src[((int64_t)(j0 + 4 * c) << kRowBits) + q + lane];
+#pragma unroll
+                    for (int c = 0; c < 8; ++c)
+                        if (j0 + 4 * c < slices) {
+                            sum.x += p[c].x;
+                            sum.y += p[c].y;
+                        }
+                }
+            sums[wave][lane] = sum;
+            __syncthreads();
+            if (wave == 0 && q + lane < n) {
+#pragma unroll
+                for (int v = 1; v < 4; ++v) {
+                    sum.x += sums[v][lane].x;
+                    sum.y += sums[v][lane].y;
+                }
+                dst[q + lane] = make_float2((float)sum.x, (float)sum.y);
+            }
+            __syncthreads();
+        }
     }
 }
 
-void table_pages_carve(WsCarver& c, int64_t pages, bool half_vals, TablePages* out) {
+void table_pages_carve(WsCarver& c, const am_grid_desc* g, int64_t pages, bool half_vals,
+                       TablePages* out) {
+    const int64_t buckets = table_levels(g).n_buckets;
     TablePages w{};
     w.pages = pages;
     w.half_vals = half_vals;
@@ -809,36 +967,48 @@ void table_pages_carve(WsCarver& c, int64_t pages, bool half_vals, TablePages* o
     w.vals = c.take<char>((size_t)pages * kPage * (half_vals ? 4 : 8));
     w.run_start = c.take<uint16_t>((size_t)pages * kRunStride + 2);
     w.partial = c.take<double2>((size_t)slot_bound(pages * kPage) << kRowBits);
+    // about 16 pages to a block that counts them; none for a few pages, which
+    // the plan counts itself (one launch of 5 us less)
+    const int64_t chunks = ceil_div(pages, 16 * (int64_t)g->n_levels);
+    w.chunks = (int32_t)(pages <= 4 * (int64_t)g->n_levels
+                             ? 0
+                             : (chunks > kMostChunks ? kMostChunks : chunks));
+    w.pairs = c.take<uint32_t>((size_t)w.chunks * buckets);
     w.plan = c.take<PagePlan>(1);
+    w.max_units = buckets + units_of(pages * kPage);   // a bucket's S <= n / U + 1
+    w.units = c.take<PageUnit>((size_t)w.max_units);
+    w.merges = c.take<PageUnit>((size_t)buckets);
     *out = w;
 }
 
-int table_pages_plan(TablePages& w, const am_grid_desc* g, const uint64_t* scan, int64_t units,
-                     int active, int64_t per_level, hipStream_t s) {
-    hipLaunchKernelGGL(k_page_plan, dim3(1), dim3(64), 0, s, table_levels(g), scan, units, active,
-                       per_level, w.pages, w.plan);
-    AM_LAUNCH_CHECK();
-    return AM_OK;
-}
-
 template <class VT>
-static int run_pages(TablePages& w, const am_grid_desc* g, float* dtable, hipStream_t s) {
+static int run_pages(TablePages& w, const am_grid_desc* g, const PageSource& src, float* dtable,
+                     hipStream_t s) {
     const TableLevels t = table_levels(g);
     KernelTimer kt_("seg_reduce", s);
-    // units <= buckets + pairs / unit pairs (both unit sizes of k_page_plan)
-    const int64_t m = w.pages * kPage, least = m / kUnitLeast, most = m / kUnitMost;
-    const int64_t units = table_digits(g) + (least < 1024 ? least : (most > 1024 ? most : 1024)) + 2;
-    const unsigned grid = (unsigned)(ceil_div(units, 256) * 256);   // whole groups of 8 x 32
-    hipLaunchKernelGGL((k_page_reduce<VT>), dim3(grid), dim3(1024), 0, s, t, w.plan, w.keys,
+    if (w.chunks > 0) {
+        hipLaunchKernelGGL(k_bucket_pairs, dim3((unsigned)w.chunks, (unsigned)t.L), dim3(1024), 0, s,
+                           t, src, w.run_start, w.pairs);
+        AM_LAUNCH_CHECK();
+    }
+    hipLaunchKernelGGL(k_page_plan, dim3(1), dim3(1024), 0, s, t, src, w.run_start, w.pairs,
+                       w.chunks, w.plan, w.units, w.merges);
+    AM_LAUNCH_CHECK();
+    const unsigned grid = (unsigned)(ceil_div(w.max_units, 256) * 256);   // whole groups of 8 x 32
+    hipLaunchKernelGGL((k_page_reduce<VT>), dim3(grid), dim3(1024), 0, s, w.plan, w.units, w.keys,
                        reinterpret_cast<const VT*>(w.vals), w.run_start, dtable, w.partial);
     AM_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_page_combine, dim3(2048), dim3(256), 0, s, t, w.plan, w.partial, dtable);
+    hipLaunchKernelGGL(k_page_merge, dim3(2048), dim3(256), 0, s, w.plan, w.merges, w.partial,
+                       dtable);
     AM_LAUNCH_CHECK();
     return AM_OK;
 }
 
-int table_pages_run(TablePages& w, const am_grid_desc* g, float* dtable, hipStream_t s) {
-    return w.half_vals ? run_pages<uint32_t>(w, g, dtable, s) : run_pages<uint2>(w, g, dtable, s);
+int table_pages_run(TablePages& w, const am_grid_desc* g, const uint64_t* scan, int64_t units,
+                    int active, int64_t per_level, float* dtable, hipStream_t s) {
+    const PageSource src{scan, units, active, per_level, w.pages};
+    return w.half_vals ? run_pages<uint32_t>(w, g, src, dtable, s)
+                       : run_pages<uint2>(w, g, src, dtable, s);
 }
 
 template <class VT>
