@@ -1014,7 +1014,9 @@ void pairs_carve(WsCarver& c, const GeoArgs& a, const am_grid_desc* g, int64_t n
 // A step that does not fit leaves less than 4096 pairs' room in its page.
 int64_t pairs_bound(const GeoArgs& a, const PairHead& h, int LJ, int64_t n) {
     if (!h.paged) return ceil_div(n, 16) * (lane_pairs(a) * LJ * 64);
-    return h.units * (lane_pairs(a) * 1024 / (kPage - 4096) + 1);
+    auto pages = [&](int64_t samples) { return lane_pairs(a) * samples / (kPage - 4096) + 1; };
+    const int64_t whole = n / 1024, rest = n % 1024;   // units of 1024 samples, and a smaller one
+    return a.active * (whole * pages(1024) + (rest ? pages(rest) : 0));
 }
 
 // Moves one count (flag "sdf_bwd_count_shift"), so that a test can see the
