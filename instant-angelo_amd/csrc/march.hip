@@ -221,8 +221,106 @@ __device__ __forceinline__ int march_wave(const MarchArgs& a, const float* o, co
     return j;
 }
 
-// Lanes per ray of the background marching (8 measured no faster).
-constexpr int kMarchBgGroup = 4;
+// Lanes per ray of march_group and of the background marching (8 measured no
+// faster).
+constexpr int kMarchGroup = 4;
+
+// The same with kMarchGroup lanes to a ray, for many rays of few steps or of
+// many steps a cell, where a wave to a ray leaves most of its lanes idle or
+// within few cells (use_group): inside, the
+// group's lanes take their steps as above but by the additions themselves;
+// a voxel skip is walked from the first lane outside.
+__device__ int march_group(const MarchArgs& a, const float* o, const float* d, float near,
+                           float far, const uint8_t* __restrict__ grid, float* __restrict__ ts,
+                           float* __restrict__ te, int32_t* __restrict__ ri, int32_t ray) {
+    constexpr int G = kMarchGroup;
+    const int g = lane_id() % G, gbase = lane_id() - g;
+    const float inv[3] = {1.0f / d[0], 1.0f / d[1], 1.0f / d[2]};
+    const float step = a.step;
+    const uint32_t mask = (1u << G) - 1u;
+    float t0 = near;
+    float t1 = t0 + step;
+    float tm = (t0 + t1) * 0.5f;
+    int j = 0;
+    while (true) {
+        // this lane's state: g occupied steps ahead
+        float c0 = t0, c1 = t1, cm = tm;
+        bool alive = true;
+        for (int q = 0; q < g; ++q) {
+            const float prev = cm;
+            c0 = c1;
+            c1 = c0 + step;
+            cm = (c0 + c1) * 0.5f;
+            alive = alive && (cm > prev);
+        }
+        const bool cond = alive && cm < far && !(a.cap > 0 && j + g >= a.cap);
+        float xyz[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) xyz[k] = __fmaf_rn(cm, d[k], o[k]);
+        const bool occ = cond && occupied(a, xyz, grid);
+        const uint32_t bo = (uint32_t)(__ballot(occ) >> gbase) & mask;
+        const uint32_t bc = (uint32_t)(__ballot(cond) >> gbase) & mask;
+        const int m = __builtin_ctz(~bo);   // first lane not an occupied in-range state (G: none)
+        if (g < m && ts) {
+            ts[j + g] = c0;
+            te[j + g] = c1;
+            if (ri) ri[j + g] = ray;
+        }
+        if (m == G) {   // all G were samples: continue from the last lane's successor
+            const float n0 = c1, n1 = n0 + step, nm = (n0 + n1) * 0.5f;
+            const int ok = nm > cm ? 1 : 0;
+            t0 = __shfl(n0, gbase + G - 1, 64);
+            t1 = __shfl(n1, gbase + G - 1, 64);
+            tm = __shfl(nm, gbase + G - 1, 64);
+            const int okg = __shfl(ok, gbase + G - 1, 64);
+            j += G;
+            if (!okg) break;
+            continue;
+        }
+        j += m;
+        if (!((bc >> m) & 1u)) break;   // state m ends the march
+        // state m is in range and unoccupied: the voxel skip from its midpoint
+        const float tmm = __shfl(cm, gbase + m, 64);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) xyz[k] = __fmaf_rn(tmm, d[k], o[k]);
+        const float target = tmm + dist_next_voxel(a, xyz, d, inv);
+        float tt = tmm;
+        bool stuck = false;
+        do {
+            const float nt = tt + step;
+            if (!(nt > tt)) {
+                stuck = true;
+                break;
+            }
+            tt = nt;
+        } while (tt < target);
+        if (stuck) break;
+        tm = tt;
+        t0 = tm - step * 0.5f;
+        t1 = tm + step * 0.5f;
+    }
+    return j;
+}
+
+// Ray and lane of a thread of the marching kernels: four waves or (GROUP) 64
+// groups of lanes a block.
+template <bool GROUP>
+__device__ __forceinline__ int64_t march_ray() {
+    if constexpr (GROUP) return ((int64_t)blockIdx.x * 256 + threadIdx.x) / kMarchGroup;
+    else return (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+}
+template <bool GROUP>
+__device__ __forceinline__ int march(const MarchArgs& a, const float* o, const float* d, float near,
+                                     float far, const uint8_t* __restrict__ grid,
+                                     float* __restrict__ ts, float* __restrict__ te,
+                                     int32_t* __restrict__ ri, int32_t ray) {
+    if constexpr (GROUP) return march_group(a, o, d, near, far, grid, ts, te, ri, ray);
+    else return march_wave(a, o, d, near, far, grid, ts, te, ri, ray);
+}
+template <bool GROUP>
+__device__ __forceinline__ bool march_lead() {
+    return lane_id() % (GROUP ? kMarchGroup : 64) == 0;
+}
 
 // ---- background marching (nerfacc 0.3.3 ray_marching with
 // ContractionType.UN_BOUNDED_SPHERE and a cone angle, as called by
@@ -326,12 +424,12 @@ __global__ void __launch_bounds__(64) k_march_bg_count(MarchBgArgs b,
                                                       const uint8_t* __restrict__ grid,
                                                       int32_t* __restrict__ counts) {
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t i = tid / kMarchBgGroup;
-    const int g = (int)(tid % kMarchBgGroup);
+    const int64_t i = tid / kMarchGroup;
+    const int g = (int)(tid % kMarchGroup);
     if (i >= n) return;
     const float o[3] = {rays[6 * i], rays[6 * i + 1], rays[6 * i + 2]};
     const float d[3] = {rays[6 * i + 3], rays[6 * i + 4], rays[6 * i + 5]};
-    const int j = march_group_bg<kMarchBgGroup>(b, o, d, t_near[i], t_far[i], grid, nullptr, nullptr,
+    const int j = march_group_bg<kMarchGroup>(b, o, d, t_near[i], t_far[i], grid, nullptr, nullptr,
                                               nullptr, (int32_t)i, g, lane_id() - g);
     if (g == 0) counts[i] = j;
 }
@@ -345,8 +443,8 @@ __global__ void __launch_bounds__(64) k_march_bg_fill(MarchBgArgs b, const float
                                                      float* __restrict__ ts,
                                                      float* __restrict__ te) {
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t i = tid / kMarchBgGroup;
-    const int g = (int)(tid % kMarchBgGroup);
+    const int64_t i = tid / kMarchGroup;
+    const int g = (int)(tid % kMarchGroup);
     if (i >= n) return;
     const int32_t base = packed[2 * i];
     const float o[3] = {rays[6 * i], rays[6 * i + 1], rays[6 * i + 2]};
@@ -354,7 +452,7 @@ __global__ void __launch_bounds__(64) k_march_bg_fill(MarchBgArgs b, const float
     MarchBgArgs c = b;
     c.m.cap = packed[2 * i + 1];  // never write past the counted samples
     if (c.m.cap == 0) return;
-    march_group_bg<kMarchBgGroup>(c, o, d, t_near[i], t_far[i], grid, ts + base, te + base,
+    march_group_bg<kMarchGroup>(c, o, d, t_near[i], t_far[i], grid, ts + base, te + base,
                                 ridx + base, (int32_t)i, g, lane_id() - g);
 }
 
@@ -398,19 +496,20 @@ __global__ void k_ray_aabb(const float* __restrict__ rays, int64_t n, float aabb
     aabb_one(o, d, aabb, t_near + i, t_far + i);
 }
 
+template <bool GROUP>
 __global__ void __launch_bounds__(256) k_march_count(MarchArgs a, const float* __restrict__ rays,
                                                    int64_t n, const float* __restrict__ t_near,
                                                    const float* __restrict__ t_far,
                                                    const float* __restrict__ jitter,
                                                    const uint8_t* __restrict__ grid,
                                                    int32_t* __restrict__ counts) {
-    const int64_t i = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int64_t i = march_ray<GROUP>();
     if (i >= n) return;
     const float o[3] = {rays[6 * i], rays[6 * i + 1], rays[6 * i + 2]};
     const float d[3] = {rays[6 * i + 3], rays[6 * i + 4], rays[6 * i + 5]};
-    const int j = march_wave(a, o, d, ray_near(t_near, jitter, i, a.step), t_far[i], grid, nullptr,
+    const int j = march<GROUP>(a, o, d, ray_near(t_near, jitter, i, a.step), t_far[i], grid, nullptr,
                              nullptr, nullptr, (int32_t)i);
-    if (lane_id() == 0) counts[i] = j;
+    if (march_lead<GROUP>()) counts[i] = j;
 }
 
 // packed[i] = (start, count) from counts and their exclusive scan; total.
@@ -424,6 +523,7 @@ __global__ void k_march_pack(const int32_t* __restrict__ counts, const int32_t* 
     if (i == n - 1) total[0] = starts[i] + counts[i];
 }
 
+template <bool GROUP>
 __global__ void __launch_bounds__(256) k_march_fill(MarchArgs a, const float* __restrict__ rays,
                                                   int64_t n, const float* __restrict__ t_near,
                                                   const float* __restrict__ t_far,
@@ -432,7 +532,7 @@ __global__ void __launch_bounds__(256) k_march_fill(MarchArgs a, const float* __
                                                   const int32_t* __restrict__ packed,
                                                   int32_t* __restrict__ ridx,
                                                   float* __restrict__ ts, float* __restrict__ te) {
-    const int64_t i = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int64_t i = march_ray<GROUP>();
     if (i >= n) return;
     const int32_t base = packed[2 * i];
     const float o[3] = {rays[6 * i], rays[6 * i + 1], rays[6 * i + 2]};
@@ -440,13 +540,14 @@ __global__ void __launch_bounds__(256) k_march_fill(MarchArgs a, const float* __
     MarchArgs b = a;
     b.cap = packed[2 * i + 1];  // never write past the counted samples
     if (b.cap == 0) return;
-    march_wave(b, o, d, ray_near(t_near, jitter, i, a.step), t_far[i], grid, ts + base, te + base,
+    march<GROUP>(b, o, d, ray_near(t_near, jitter, i, a.step), t_far[i], grid, ts + base, te + base,
                ridx + base, (int32_t)i);
 }
 
 // Staged marching (a per-ray sample cap is set): the count pass also writes
 // each ray's samples into a cap-strided staging area, and the fill pass
 // copies them to their packed positions instead of marching again.
+template <bool GROUP>
 __global__ void __launch_bounds__(256) k_march_count_staged(MarchArgs a,
                                                           const float* __restrict__ rays, int64_t n,
                                                           const float* __restrict__ t_near,
@@ -456,14 +557,14 @@ __global__ void __launch_bounds__(256) k_march_count_staged(MarchArgs a,
                                                           int32_t* __restrict__ counts,
                                                           float* __restrict__ st0,
                                                           float* __restrict__ st1) {
-    const int64_t i = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int64_t i = march_ray<GROUP>();
     if (i >= n) return;
     const float o[3] = {rays[6 * i], rays[6 * i + 1], rays[6 * i + 2]};
     const float d[3] = {rays[6 * i + 3], rays[6 * i + 4], rays[6 * i + 5]};
     const int64_t base = i * (int64_t)a.cap;   // a.cap > 0: samples j < cap
-    const int j = march_wave(a, o, d, ray_near(t_near, jitter, i, a.step), t_far[i], grid,
+    const int j = march<GROUP>(a, o, d, ray_near(t_near, jitter, i, a.step), t_far[i], grid,
                              st0 + base, st1 + base, nullptr, (int32_t)i);
-    if (lane_id() == 0) counts[i] = j;
+    if (march_lead<GROUP>()) counts[i] = j;
 }
 
 // One wave per ray: its staged samples to the packed outputs, coalesced.
@@ -506,6 +607,31 @@ static MarchArgs march_args(const float* roi6, const uint8_t* grid, int res, flo
     a.res_pow2 = res > 0 && (res & (res - 1)) == 0;
     a.inv_res = a.res_pow2 ? 1.0f / (float)res : 0.0f;
     return a;
+}
+
+// Four lanes to a ray or a wave to a ray, once there are enough rays to fill the
+// chip either way.  A wave's round costs the same however few of its 64 points
+// lie in the box (few steps), or however few cells they cross (cells of many
+// steps, which a group skips at once, 16 rays a wave).  Whole call, 128^3 scene
+// grid, four lanes against a wave, by steps in the box's diagonal:
+//              17         35         49         69         99        1019       3464
+//   1048576  324 / 953  503 / 1141 642 / 1203 843 / 1140 1138 / 1314 4384 / 4168 8611 / 11512 us
+//    131072   96 / 168  127 / 191  144 / 198  174 / 188  221 / 208   770 / 576   1444 / 1512
+//     32768   69 / 82    94 / 91   112 / 91   120 / 93   149 / 98    447 / 212    798 / 455
+// (1019 and 3464 steps: 4.6 and 15.6 a cell.)
+static bool use_group(const MarchArgs& a, int64_t n_rays) {
+    float sq = 0.0f, least = a.roi[3] - a.roi[0];
+    for (int d = 0; d < 3; ++d) {
+        const float range = a.roi[3 + d] - a.roi[d];
+        sq += range * range;
+        least = std::fmin(least, range);
+    }
+    const float steps = std::sqrt(sq) / a.step;
+    if (steps <= 80.0f) return (float)n_rays > 1600.0f * steps;
+    return a.has_grid && least > 8.0f * (float)a.res * a.step && n_rays > 65536;
+}
+static unsigned march_blocks(int64_t n_rays, bool group) {
+    return (unsigned)ceil_div(n_rays, group ? 256 / kMarchGroup : 4);
 }
 
 static size_t scan_tmp_bytes(int64_t n) {
@@ -575,10 +701,11 @@ extern "C" int am_march_count(const float* rays, int64_t n_rays, const float* t_
     char* stmp = c.take<char>(sb + 256);
     if (!c.ok()) return workspace_short(c.used, workspace_bytes);
     const MarchArgs a = march_args(roi6_host, grid, grid_res, step, cap);
-    const unsigned nb = (unsigned)ceil_div(n_rays, 4);
+    const bool group = use_group(a, n_rays);
     {
         KernelTimer kt_("march_count", s);
-        hipLaunchKernelGGL(k_march_count, dim3(nb), dim3(256), 0, s, a, rays, n_rays, t_near, t_far,
+        auto kern = group ? k_march_count<true> : k_march_count<false>;
+        hipLaunchKernelGGL(kern, dim3(march_blocks(n_rays, group)), dim3(256), 0, s, a, rays, n_rays, t_near, t_far,
                            jitter, grid, counts);
     }
     AM_LAUNCH_CHECK();
@@ -606,8 +733,9 @@ extern "C" int am_march_fill(const float* rays, int64_t n_rays, const float* t_n
     const MarchArgs a = march_args(roi6_host, grid, grid_res, step, cap);
     {
         KernelTimer kt_("march_fill", to_stream(stream));
-        hipLaunchKernelGGL(k_march_fill, dim3((unsigned)ceil_div(n_rays, 4)), dim3(256), 0,
-                           to_stream(stream), a, rays, n_rays, t_near, t_far, jitter, grid, packed,
+        const bool group = use_group(a, n_rays);
+        auto kern = group ? k_march_fill<true> : k_march_fill<false>;
+        hipLaunchKernelGGL(kern, dim3(march_blocks(n_rays, group)), dim3(256), 0, to_stream(stream), a, rays, n_rays, t_near, t_far, jitter, grid, packed,
                            ray_indices, t_starts, t_ends);
     }
     AM_LAUNCH_CHECK();
@@ -652,8 +780,9 @@ extern "C" int am_march_count_staged(const float* rays, int64_t n_rays, const fl
     const MarchArgs a = march_args(roi6_host, grid, grid_res, step, cap);
     {
         KernelTimer kt_("march_count", s);
-        hipLaunchKernelGGL(k_march_count_staged,
-                           dim3((unsigned)ceil_div(n_rays, 4)), dim3(256), 0, s, a,
+        const bool group = use_group(a, n_rays);
+        auto kern = group ? k_march_count_staged<true> : k_march_count_staged<false>;
+        hipLaunchKernelGGL(kern, dim3(march_blocks(n_rays, group)), dim3(256), 0, s, a,
                            rays, n_rays, t_near, t_far, jitter, grid, counts, st0, st1);
     }
     AM_LAUNCH_CHECK();
@@ -722,7 +851,7 @@ extern "C" int am_march_bg_count(const float* rays, int64_t n_rays, const float*
     b.cone = cone_angle;
     {
         KernelTimer kt_("march_bg_count", s);
-        hipLaunchKernelGGL(k_march_bg_count, dim3((unsigned)ceil_div(n_rays * kMarchBgGroup, 64)),
+        hipLaunchKernelGGL(k_march_bg_count, dim3((unsigned)ceil_div(n_rays * kMarchGroup, 64)),
                            dim3(64), 0, s,
                            b, rays, n_rays, t_near, t_far, grid, counts);
     }
@@ -754,7 +883,7 @@ extern "C" int am_march_bg_fill(const float* rays, int64_t n_rays, const float* 
     b.cone = cone_angle;
     {
         KernelTimer kt_("march_bg_fill", to_stream(stream));
-        hipLaunchKernelGGL(k_march_bg_fill, dim3((unsigned)ceil_div(n_rays * kMarchBgGroup, 64)),
+        hipLaunchKernelGGL(k_march_bg_fill, dim3((unsigned)ceil_div(n_rays * kMarchGroup, 64)),
                            dim3(64), 0,
                            to_stream(stream), b, rays, n_rays, t_near, t_far, grid, packed,
                            ray_indices, t_starts, t_ends);
