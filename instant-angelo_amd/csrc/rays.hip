@@ -103,9 +103,16 @@ __global__ void k_morton_keys(const float* __restrict__ pts, int64_t n, float r,
 // passes at 65 k samples, by the scattered writes at 1 M.  A merge sort of the
 // same keys (one launch a doubling), with its key, index and inverse kernels:
 // 65 k samples 43 -> 22 us, 262 k 99 -> 25, 940 k 169 -> 45, 4.8 M 230 -> 150.
+// Twice the blocks above kOrderWide samples, where a block a CU no longer
+// covers its loads' latency (60 M samples, 30-bit keys 3298 -> 2979 us, the sort
+// 2947; 20 M 1049 -> 968).
 constexpr int kOrderTile = 1024;     // samples a tile: one a thread
 constexpr int kOrderBlocks = 256;
+constexpr int64_t kOrderWide = 1 << 24;
 constexpr int kDigits = 256;
+static inline int64_t order_blocks(int64_t n) {
+    return n > kOrderWide ? 2 * kOrderBlocks : kOrderBlocks;
+}
 
 struct OrderPass {
     const float* pts;      // first pass: keys from the positions
@@ -141,6 +148,20 @@ __global__ void __launch_bounds__(kOrderTile) k_order_hist(OrderPass a,
     }
     __syncthreads();
     if (tid < kDigits) hist[(int64_t)blockIdx.x * kDigits + tid] = h[tid];
+}
+
+// The wave's lanes with this lane's digit, and how many of them lie before it.
+__device__ __forceinline__ int digit_rank(bool on, uint32_t digit, uint64_t* lanes) {
+    uint64_t same = __ballot(on);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        const bool bit = digit >> b & 1u;
+        const uint64_t set = __ballot(bit);
+        same &= bit ? set : ~set;
+    }
+    *lanes = same;
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
 }
 
 template <bool FIRST, bool LAST>
@@ -190,15 +211,8 @@ __global__ void __launch_bounds__(kOrderTile) k_order_scatter(OrderPass a,
         const bool on = i < a.n;
         const uint2 it = on ? order_item<FIRST>(a, i) : make_uint2(0u, 0u);
         const uint32_t digit = it.x >> a.shift & ((1u << a.width) - 1u);
-        uint64_t same = __ballot(on);   // the wave's lanes with this lane's digit
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            const bool bit = digit >> b & 1u;
-            const uint64_t set = __ballot(bit);
-            same &= bit ? set : ~set;
-        }
-        const int rank = (int)__builtin_amdgcn_mbcnt_hi(
-            (uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+        uint64_t same;
+        const int rank = digit_rank(on, digit, &same);
         if (on && rank == 0) count[wave][digit] = (uint32_t)__popcll(same);
         __syncthreads();
         if (tid < kDigits) {   // counts to places, waves in order
@@ -230,6 +244,93 @@ __global__ void __launch_bounds__(kOrderTile) k_order_scatter(OrderPass a,
     }
 }
 
+// All passes of up to kOrderOne samples in one block and one launch, the samples
+// in LDS between passes: bound by that launch (1000 samples, 15- and 30-bit keys
+// 16 us, two launches a pass 24 and 36, the sort 27; 4096 samples 16 and 26
+// against 25 and 36, the sort 32).
+constexpr int kOneTiles = 4;
+constexpr int kOrderOne = kOneTiles * kOrderTile;
+
+__global__ void __launch_bounds__(kOrderTile) k_order_one(OrderPass a, int passes) {
+    __shared__ uint2 items[kOrderOne];
+    __shared__ uint32_t count[kOrderTile / 64][kDigits];   // a tile's, per wave; its places
+    __shared__ uint32_t place[kDigits];
+    __shared__ uint32_t wave_sum[4];
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = (int)a.n, tiles = (n + kOrderTile - 1) / kOrderTile;
+    uint2 it[kOneTiles];
+#pragma unroll
+    for (int t = 0; t < kOneTiles; ++t) {
+        const int i = t * kOrderTile + tid;
+        it[t] = i < n ? order_item<true>(a, i) : make_uint2(0u, 0u);
+    }
+    for (int p = 0; p < passes; ++p) {
+        const int shift = p * a.width;
+        const uint32_t mask = (1u << a.width) - 1u;
+        if (tid < kDigits) place[tid] = 0u;
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < kOneTiles; ++t)
+            if (t * kOrderTile + tid < n) atomicAdd(&place[it[t].x >> shift & mask], 1u);
+        __syncthreads();
+        uint32_t all = 0, incl = 0;
+        if (tid < kDigits) {
+            incl = all = place[tid];
+#pragma unroll
+            for (int s = 1; s < 64; s <<= 1) {
+                const uint32_t o = __shfl_up(incl, s, 64);
+                if (lane >= s) incl += o;
+            }
+            if (lane == 63) wave_sum[wave] = incl;
+        }
+        __syncthreads();
+        if (tid < kDigits) {
+            uint32_t at = incl - all;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) at += w < wave ? wave_sum[w] : 0u;
+            place[tid] = at;
+        }
+#pragma unroll
+        for (int t = 0; t < kOneTiles; ++t) {
+            if (t >= tiles) break;
+            for (int q = tid; q < (kOrderTile / 64) * kDigits; q += kOrderTile) (&count[0][0])[q] = 0u;
+            __syncthreads();
+            const bool on = t * kOrderTile + tid < n;
+            const uint32_t digit = it[t].x >> shift & mask;
+            uint64_t same;
+            const int rank = digit_rank(on, digit, &same);
+            if (on && rank == 0) count[wave][digit] = (uint32_t)__popcll(same);
+            __syncthreads();
+            if (tid < kDigits) {   // counts to places, waves in order
+                uint32_t at = place[tid];
+#pragma unroll
+                for (int w = 0; w < kOrderTile / 64; ++w) {
+                    const uint32_t c = count[w][tid];
+                    count[w][tid] = at;
+                    at += c;
+                }
+                place[tid] = at;
+            }
+            __syncthreads();
+            if (on) {
+                const uint32_t to = count[wave][digit] + (uint32_t)rank;
+                if (p + 1 < passes) items[to] = it[t];
+                else {
+                    a.perm[to] = (int32_t)it[t].y;
+                    a.inv[it[t].y] = (int32_t)to;
+                }
+            }
+            __syncthreads();
+        }
+        if (p + 1 < passes) {
+#pragma unroll
+            for (int t = 0; t < kOneTiles; ++t)
+                if (t * kOrderTile + tid < n) it[t] = items[t * kOrderTile + tid];
+            __syncthreads();
+        }
+    }
+}
+
 }  // namespace am
 
 using namespace am;
@@ -237,7 +338,7 @@ using namespace am;
 extern "C" size_t am_morton_order_workspace_size(int64_t n, int32_t bits) {
     if (n < 0 || bits < 1 || bits > 10) return 0;
     WsCarver c(nullptr, 0);
-    c.take<uint32_t>(kOrderBlocks * kDigits);
+    c.take<uint32_t>((size_t)order_blocks(n) * kDigits);
     for (int b = 0; b < 2; ++b) c.take<uint2>((size_t)n + 1);
     return c.used + 256;
 }
@@ -252,7 +353,7 @@ extern "C" int am_morton_order(const float* pts, int64_t n, float radius, int32_
     AM_CHECK_ARG(pts && perm && inv && workspace, "NULL buffer");
     hipStream_t s = to_stream(stream);
     WsCarver c(workspace, workspace_bytes);
-    uint32_t* hist = c.take<uint32_t>(kOrderBlocks * kDigits);
+    uint32_t* hist = c.take<uint32_t>((size_t)order_blocks(n) * kDigits);
     uint2* items[2];
     for (int b = 0; b < 2; ++b) items[b] = c.take<uint2>((size_t)n + 1);
     if (!c.ok()) return workspace_short(c.used, workspace_bytes);
@@ -267,8 +368,13 @@ extern "C" int am_morton_order(const float* pts, int64_t n, float radius, int32_
     a.inv = inv;
     a.width = width;
     a.n = n;
-    a.tiles = (int)ceil_div(all_tiles, kOrderBlocks);
+    a.tiles = (int)ceil_div(all_tiles, order_blocks(n));
     const unsigned nb = (unsigned)ceil_div(all_tiles, a.tiles);
+    if (n <= kOrderOne) {
+        hipLaunchKernelGGL(k_order_one, dim3(1), dim3(kOrderTile), 0, s, a, passes);
+        AM_LAUNCH_CHECK();
+        return AM_OK;
+    }
     for (int p = 0; p < passes; ++p) {
         const bool last = p == passes - 1;
         a.shift = p * width;
