@@ -38,7 +38,9 @@ def log(*a):
 
 
 def algorithmic_bytes(kernel, spec, n_samples, n_rays, n_pairs, mixed=False):
-    """Algorithmic HBM bytes of one launch (per-step averages).
+    """Algorithmic HBM bytes of one launch (per-step averages): every
+    evaluation's gathers counted in full.  requested_bytes has what the kernels
+    ask for where they share rows between evaluations.
 
     geo_fwd: per encode evaluation of L levels, F=2 features, b_t B table
       entries (4 fp32, 2 in the mixed form's fp16 rows): 12 B position +
@@ -51,9 +53,10 @@ def algorithmic_bytes(kernel, spec, n_samples, n_rays, n_pairs, mixed=False):
       gradients (27 floats); writes the encode gradients (13 x L*F floats).
     pair_count: position, direction, FD values.  pair_emit: the same + the
       encode gradients + 12 B (8 B mixed) per (row, value) pair written.
-    radix_sort: each pair (4 B row + 8 B value; 4 B value in the mixed form)
-      read and written once.
-    seg_reduce: each pair read once + one 8 B row written per pair (bound).
+    radix_sort (levels past 2^21 rows alone): each pair (4 B row + 8 B value;
+      4 B value in the mixed form) read and written once.
+    seg_reduce (after that sort): each pair read once + one 8 B row written per
+      pair (bound).
     composite: 40 B per sample + 32 B per ray.
     Analytic-gradient mode: 7 evaluations (base with position derivatives +
     6 curvature), 7 derivative slots stored, 3 more encode-gradient slots.
@@ -87,6 +90,26 @@ def algorithmic_bytes(kernel, spec, n_samples, n_rays, n_pairs, mixed=False):
     if kernel in ("composite_fwd", "composite_bwd"):
         return n_samples * 40 + n_rays * 32
     return None
+
+
+def requested_bytes(kernel, spec, n_samples, n_rays, n_pairs, mixed=False, offsets=None,
+                    table_rows=0):
+    """What one launch asks of memory: algorithmic_bytes, but for
+    geo_fwd with central differences: 8 rows a level for each cluster's centre,
+      and for each of the 12 offset evaluations the 4 rows of one more face where
+      the offset leaves the centre's cell.  offsets: its length in cells of each
+      gathered level, the chance to leave the cell; beyond one cell all 8 rows.
+    seg_reduce by pages (no sort): 4 B of each pair for its exponents, then the
+      pair, and 8 B a table row written.
+    """
+    total = algorithmic_bytes(kernel, spec, n_samples, n_rays, n_pairs, mixed)
+    row = 2 * (2 if mixed else 4)
+    if kernel == "geo_fwd" and offsets and evals_per_sample(spec) == 13:
+        rows = 2 * 8 * len(offsets) + 12 * sum(4 * d if d <= 1 else 8 for d in offsets)
+        total += n_samples * row * (rows - 13 * 8 * len(offsets))
+    elif kernel == "seg_reduce" and table_rows:
+        total = n_pairs * (4 + (8 if mixed else 12)) + table_rows * 8
+    return total if total is None else int(total)
 
 
 def evals_per_sample(spec):
@@ -411,14 +434,14 @@ def main():
     ap.add_argument("--rays", type=int, default=None)
     ap.add_argument("--table-atomic", action="store_true",
                     help="SDF table gradient by float atomics (run-to-run summation order "
-                         "varies) instead of the deterministic sort + reduce")
+                         "varies) instead of the deterministic reduction")
     ap.add_argument("--level-sweep", action="store_true",
                     help="only time the fused SDF forward over one step's samples with 1, 2, "
                          "4, 8, 12, 16 active levels (3 launches each; for per-level HBM "
                          "counters under rocprofv3) and print that as the JSON line")
     ap.add_argument("--sync-free", action="store_true",
-                    help="SDF backward without its pair-count host read (pair arrays and "
-                         "sort sized for the worst-case pair count)")
+                    help="SDF backward without its pair-count host read (pair arrays "
+                         "sized for the worst-case pair count)")
     ap.add_argument("--no-pipeline", action="store_true",
                     help="march each step's rays at the start of the step (by default the "
                          "next step's rays are drawn and marched on a second stream while "
@@ -495,10 +518,15 @@ def main():
     # roofline of the dominant kernel, and of every kernel with a byte model
     # (launch averages: one launch per step for each of these kernels)
     roof, per_kernel = None, {}
+    grid = wl.model.geometry.grid_module.grid
+    offset = wl.model.geometry._finite_difference_eps / (2.0 * wl.model.geometry.radius)
+    offsets = [offset * grid.scale[q] for q in range(spec.get("start_level") or spec["levels"])]
     for k, v in kern.items():
         if bg_per_step and k in ("radix_sort", "seg_reduce"):
             continue   # shared with the background encode's backward: no per-step byte model
-        nbytes = algorithmic_bytes(k, spec, fg_per_step, rays, pairs_per_step, wl.mixed)
+        nbytes = requested_bytes(
+            k, spec, fg_per_step, rays, pairs_per_step, wl.mixed, offsets,
+            0 if "radix_sort" in kern else int(grid.n_entries))
         if nbytes is None:
             continue
         # the byte models are per step: divide by the kernel's time per step
@@ -568,7 +596,7 @@ def main():
         "table_pairs_per_step": round(pairs_per_step, 1),
         "sdf_bwd_sync_free": bool(args.sync_free),
         "march_pipelined": bool(wl.pipeline),
-        "table_gradient": "atomic" if args.table_atomic else "deterministic (sort + reduce)",
+        "table_gradient": "atomic" if args.table_atomic else "deterministic",
         "sdf_bwd_host_reads_per_step": host_reads,
         "allocator_in_timed_steps": alloc,
         "roofline": roof,
