@@ -20,10 +20,12 @@ static int64_t bucket_slots(int64_t m) { return 2 * (m / kUnitItems) + 1; }
 // and merge more partial sums.  Reduce and merge with 768 / 960 / 1024 / 1216 /
 // 1440 / 2048 units: 940 k samples, 16 levels 1930 / 1925 / 1911 / 1827 / 1760 /
 // 1776 us; 480 k, 4 levels 576 / 584 / 667 / 586 / 659 / 774; 240 k, 16 levels
-// of 2^19 rows 438 / 469 / - / 420 / 441 / -.  65 k samples, 8 levels, with
-// 16384 / 32768 pairs at least: 133 / 95 us.
+// of 2^19 rows 438 / 469 / - / 420 / 441 / -.  With 16384 / 32768 / 49152 /
+// 65536 pairs at least: 65 k samples, 8 levels 133 / 96 / 74 / 94 us; the
+// background's 29 M pairs - / 244 / 242 / 259; 65 k samples, 16 levels - / 164 /
+// 186 / 187.
 constexpr int64_t kUnitMost = 1 << 19;
-constexpr int64_t kUnitLeast = 32768;
+constexpr int64_t kUnitLeast = 49152;
 constexpr int64_t kUnits = 1216;
 __host__ __device__ inline int64_t unit_pairs(int64_t total) {
     const int64_t u = total / kUnits;
@@ -599,8 +601,12 @@ __device__ __forceinline__ uint64_t block_scan(uint64_t v, uint64_t* wave_sum, u
 // one block's: 940 k samples within 0.002 of a point, 2^21 rows a level, reduce
 // 7.6 -> 3.3 ms, within 0.1: 2.76 -> 2.52; 2 M points of the stand-alone grid
 // within 0.4 % of the box 29.5 -> 5.3 ms.  Spread samples pay 5 to 10 us for
-// the counts (20 k samples: 85 -> 90 us in all).  Buckets without pairs have no
-// unit; the merge writes their zeros.
+// the counts (20 k samples: 87 -> 91 us in all).  Counts and units in one launch
+// were no faster: with the units cut by the last of the counting blocks its
+// fences write the emission's dirty lines back (27 to 54 us), and with a range
+// of units for each level every block pays for finding its unit (20 k samples,
+// reduce 72 -> 77 us) or the XCDs for the ranges' gaps (29 M pairs 231 -> 245).
+// Buckets without pairs have no unit; the merge writes their zeros.
 __global__ void __launch_bounds__(1024) k_page_plan(TableLevels t, PageSource src,
                                                     const uint16_t* __restrict__ run_start,
                                                     const uint32_t* __restrict__ pairs, int chunks,

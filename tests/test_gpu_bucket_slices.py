@@ -10,8 +10,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("L,log2T,base,scale,active,n,width", [
     (2, 21, 128, 4.0, 2, 500, 0.004),      # a page a level; 500 buckets without pairs
-    (2, 21, 128, 4.0, 2, 6000, 0.004),     # a bucket just past a unit and a half, or not
-    (2, 21, 128, 4.0, 2, 12000, 0.004),    # a few slices
+    (2, 21, 128, 4.0, 2, 9300, 0.004),     # a bucket just past a unit and a half (73,728 pairs)
+    (2, 21, 128, 4.0, 2, 25000, 0.004),    # a few slices
     (2, 21, 128, 4.0, 2, 60000, 0.004),    # many slices, merged by four waves
     (1, 6, 4, 2.0, 1, 70001, 1.0),         # one bucket of 64 rows
     (5, 17, 16, 2.0, 4, 30011, 0.1),       # a last bucket cut by its level's end, an empty level
