@@ -53,7 +53,7 @@ int am_version(void);
 int am_timer_enable(int32_t on);
 int am_timer_read(const char* name, double* total_ms, int64_t* count);
 /* Work units recorded under `name` since am_timer_enable (e.g.
- * "table_pairs": the (row, value) pairs the table-gradient sorts received). */
+ * "table_pairs": the (row, value) pairs the table-gradient reductions received). */
 int am_timer_units(const char* name, int64_t* units);
 
 /* Implementation variant switches, for measurement and tests (no
@@ -109,8 +109,10 @@ int am_grid_init(am_grid_desc* g, int32_t n_levels, int32_t n_features,
 int am_hashgrid_fwd(const am_grid_desc* g, const float* x, int64_t n, const float* table,
                     int32_t active_levels, float* out, void* stream);
 
-/* Deterministic backward: dtable[n_entries,F] (fully overwritten) by
- * sort-by-row + segmented reduce; dx[n,3] (nullable) = dL/dx.
+/* Deterministic backward: dtable[n_entries,F] (fully overwritten) by exact
+ * sums of each row's pairs (other feature counts, levels past 2^21 rows or not
+ * one after another: sort by row and segmented reduce); dx[n,3] (nullable) =
+ * dL/dx.
  * Replaces tcnn's encoding backward (atomic scatter) behind the same call. */
 size_t am_hashgrid_bwd_workspace_size(const am_grid_desc* g, int64_t n, int32_t active_levels);
 int am_hashgrid_bwd(const am_grid_desc* g, const float* x, int64_t n, const float* table,

@@ -123,8 +123,7 @@ def sh_encode(dirs01, degree):
 # memory); "auto": store while the store fits store_limit_bytes.
 # sync_free: the backward sizes its pair arrays for the worst-case pair
 # count (library flag "sdf_bwd_sync_free") in a workspace held at that
-# bound, so it makes no host read of the count (its sort then covers the
-# bound; same gradients).
+# bound, so it makes no host read of the count (same gradients).
 SDF_BACKWARD = {"mode": "auto", "store_limit_bytes": 24 << 30, "sync_free": False}
 
 # The SDF backward's workspace is sized by its actual table-gradient pairs

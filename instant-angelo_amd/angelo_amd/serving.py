@@ -18,9 +18,8 @@ the count) over
 sample positions, fused SDF field (base + FD normal), fused radiance and
 compositing, with padded samples outside every ray's range.  The captured
 regions hold only kernel launches on buffers that live as long as the
-graph: the fused field runs in the caller's order there (the spatial
-order's library sort clears its state with memset nodes, which must not be
-captured), the forward keeps no backward buffers (no grad mode), and the
+graph: the fused field runs in the caller's order there (no ordering pass in
+a replayed step), the forward keeps no backward buffers (no grad mode), and the
 table / weights are those of the warm-up run before capture.  Models with
 the learned background render eagerly.
 Per-ray and per-point results do not depend on what else is in the batch
@@ -190,7 +189,7 @@ class FieldServer:
         """Post-march render of the batch (captured per sample bucket)."""
         m = self.model
         pts, mid, dists = fn.sample_points(rays, ridx, t0, t1)
-        # the caller's order: the spatial order's sort may not run in a graph
+        # the caller's order: no ordering pass in a replayed step
         sdf, _, normal, feature, _ = m.geometry.fused(pts, with_grad=True, with_laplace=False,
                                                       order=False if self.use_graphs else None)
         rgb = m.texture.fused(feature, normal, rays, ridx)
@@ -262,8 +261,8 @@ class FieldServer:
 
     # ---- SDF batch --------------------------------------------------------
     def _sdf_stage(self):
-        # lattice points are in lattice order already (coherent gathers), and
-        # the spatial order's sort may not run in a graph
+        # lattice points are in lattice order already (coherent gathers): no
+        # ordering pass in a replayed step
         return self.model.geometry.fused(self.s_pts, with_grad=False, order=False)[0]
 
     def _sdf_batch(self, n):

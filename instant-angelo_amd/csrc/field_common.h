@@ -10,8 +10,8 @@ static inline int field_blocks(int64_t n) {
     return persistent_blocks((n + 15) / 16, 4, kFieldBlocksMax);
 }
 
-// Grids of the SDF forward and of the pair passes (count, emit); their
-// tiles' results do not depend on the grid.  Each is a whole number of
+// Grids of the SDF forward and of the sorted and atomic forms' pair passes
+// (count, emit); their tiles' results do not depend on the grid.  Each is a whole number of
 // rounds of the blocks the device holds at once on 256 CUs (the register
 // counts of the fp32 16-level kernels): the forward two rounds of 768 in the
 // difference form (three waves a SIMD; 1024 blocks: 3.2 ms where 1536 take 2.9),

@@ -1301,7 +1301,7 @@ static int geo_fwd_launch(const GeoArgs& a, const float* pts, const float* randn
 }
 
 // The backward's workspace before the pair arrays: the pair count is only
-// known after the count pass, so the sort buffers are carved afterwards
+// known after the count pass, so the pair arrays are carved afterwards
 // from the rest (sized for the worst case by the size query).
 struct GeoBwdWs {
     float* fdv;

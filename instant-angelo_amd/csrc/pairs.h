@@ -22,8 +22,6 @@ struct PairHead {
     size_t scan_bytes;
 };
 
-// `sorted`: the arrays' form whatever the grid (the atomic form's counts are
-// not needed at all).
 void pairs_carve(WsCarver& c, const GeoArgs& a, const am_grid_desc* g, int64_t n, PairHead* h);
 // Count pass and scan; h.status[0] = capacity the emission needs (pages, or
 // pairs), h.status[2] = pairs.

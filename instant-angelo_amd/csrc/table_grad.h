@@ -13,10 +13,10 @@
 //
 // Sorted form (other feature counts, larger levels, other layouts): stable
 // radix sort of the pairs by row, then a fixed-order segmented reduce.
-// Two-feature tables sort only the key bits above `begin_bit`: the pairs of each bucket of
-// 2^begin_bit rows are then contiguous and in emission order, and one wave
-// per bucket finishes the job with an in-wave stable split sort and a
-// segmented scan into per-row accumulators in LDS.
+// Two-feature tables sort only the key bits above `begin_bit`: the pairs of
+// each bucket of 2^begin_bit rows are then contiguous and in emission order,
+// and one wave per bucket finishes the job with an in-wave stable split sort
+// and a segmented scan into per-row accumulators in LDS.
 //
 // There the emitters write pairs into keys[0] / vals[0].  Keys equal to the
 // sentinel mark empty slots; they sort last and are skipped.
